@@ -124,10 +124,10 @@ int check_launch_ws(const char* fn, int64_t need, const void* workspace, int64_t
 }
 
 // LLaMA block decode workspace, each region 256-byte aligned:
-//   n [B*D] | qkv [3*B*D] | ctx [B*D] | h [B*D] | hid [B*H] | tmp [B*max(D,H)]
+//   n [B*D] | qkv [3*B*D] | ctx [B*D] | h [B*D] | hid [B*H]
 //   | attention partials | GEMM split-K partials (the GEMM path only)
 struct DecodeWs {
-    int64_t n, qkv, ctx, h, hid, tmp, part, split, total;
+    int64_t n, qkv, ctx, h, hid, part, split, total;
 };
 // The block's GEMV forms (RMSNorm folded in, q/k/v side by side, residual
 // epilogues) serve the batches on which every projection runs the GEMV.
@@ -146,6 +146,34 @@ SkinnyPlan decode_skinny_plan(int64_t B, int64_t K, int64_t N, int nw, int64_t G
     return p;
 }
 
+// Past the GEMV batches the block's projections run the super-block form of
+// the skinny kernel where the forward's plan gives it for the total width (q,
+// k and v side by side; gate and up in one launch): 17..32 rows.  Measured for
+// 32 sequences of 2000 tokens, D = 2048, H = 5632: one block 219 us with it and
+// the GEMMs' epilogues below, 275 with seven GEMMs (and their split-K sums)
+// and separate adds and silu.
+SkinnyPlan decode_rows_plan(int64_t B, int64_t K, int64_t N, int nw, int64_t G, int cus) {
+    const I4Geom g(K, N, G);
+    SkinnyPlan p = skinny_plan(B, K, I4Geom(K, nw * N, G), cus);
+    if (p.C == 0 || p.form != 1 || p.MB != 2 || g.spc % (2 * p.C) != 0) return SkinnyPlan{};
+    return p;
+}
+
+// y = x W + bias + res for a projection of such a batch, on the kernel the
+// plain forward takes for the shape.
+hipError_t decode_project(const float* x, int64_t B, int64_t K, int64_t N, const sgq_int4_linear& w, const I4Geom& g,
+                          const float* res, float* y, void* split, int cus, hipStream_t s) {
+    const SkinnyPlan p = decode_rows_plan(B, K, N, 1, g.G, cus);
+    if (p.C > 0) {
+        SkinnyExtra ex;
+        ex.res = res;
+        return launch_skinny_i4(x, B, K, N, 1, &w.packed, &w.devscales, &w.bias, g, p, y, split, s, &ex);
+    }
+    if (linear_uses_gemv(B, K, N))
+        return launch_gemv_i4_multi(x, B, K, N, 1, &w.packed, &w.devscales, &w.bias, g, y, N, res, nullptr, 0.0f, s);
+    return launch_gemm_i4(x, B, K, N, 1, &w.packed, &w.devscales, &w.bias, g, {nullptr, res}, y, split, s);
+}
+
 DecodeWs decode_ws(int64_t B, int64_t D, int64_t H, int64_t max_len) {
     DecodeWs w;
     int64_t o = 0;
@@ -159,14 +187,16 @@ DecodeWs decode_ws(int64_t B, int64_t D, int64_t H, int64_t max_len) {
     w.ctx = take(B * D);
     w.h = take(B * D);
     w.hid = take(B * H);
-    w.tmp = take(B * (D > H ? D : H));
     w.part = take(attn_workspace_floats(B, D, max_len));
     int64_t split = 0;
     if (!decode_uses_gemv(B, D, H)) {
-        const int64_t a = gemm_workspace_bytes(B, D, D), b = gemm_workspace_bytes(B, D, H),
-                      c = gemm_workspace_bytes(B, H, D);
-        split = a > b ? a : b;
-        split = split > c ? split : c;
+        // The GEMM's or the skinny kernel's partials of any projection, on any
+        // device and for any group size.
+        for (int64_t need : {gemm_workspace_bytes(B, D, 3 * D), gemm_workspace_bytes(B, D, D),
+                             gemm_workspace_bytes(B, D, H), gemm_workspace_bytes(B, H, D),
+                             skinny_ws_bound(B, D, 3 * D, 1), skinny_ws_bound(B, D, D, 1), skinny_ws_bound(B, D, H, 2),
+                             skinny_ws_bound(B, H, D, 1)})
+            if (need > split) split = need;
     }
     w.split = o;
     o += align_up(split > 0 ? split : 1);
@@ -285,7 +315,7 @@ int linear_int4(const char* fn, const float* x, int64_t M, int64_t K, int64_t N,
         const int lw = check_launch_ws(fn, gemm_launch_ws_bytes(4, M, K, N, (int)g.spc, cus), workspace,
                                        workspace_bytes);
         if (lw != SGQ_OK) return lw;
-        SGQ_HIP(launch_gemm_i4(x, M, K, N, packed, devscales, g, bias, y, workspace, s), "gemm_i4");
+        SGQ_HIP(launch_gemm_i4(x, M, K, N, 1, &packed, &devscales, &bias, g, {}, y, workspace, s), "gemm_i4");
     }
     return ok();
 }
@@ -720,9 +750,8 @@ int sgq_swiglu_int4(const float* x, int64_t M, int64_t K, int64_t N, const void*
                                    workspace, workspace_bytes);
     if (lw != SGQ_OK) return lw;
     void* split = (char*)workspace + align_up(M * N * 4);
-    SGQ_HIP(launch_gemm_i4(x, M, K, N, packed_gate, devscales_gate, g, bias_gate, h, split, s), "gemm_i4");
-    SGQ_HIP(launch_gemm_i4(x, M, K, N, packed_up, devscales_up, g, bias_up, u, split, s), "gemm_i4");
-    SGQ_HIP(launch_silu_mul(h, u, M * N, s), "silu_mul");
+    SGQ_HIP(launch_gemm_i4(x, M, K, N, 1, &packed_gate, &devscales_gate, &bias_gate, g, {}, h, split, s), "gemm_i4");
+    SGQ_HIP(launch_gemm_i4(x, M, K, N, 1, &packed_up, &devscales_up, &bias_up, g, {h}, h, split, s), "gemm_i4");
     return ok();
 }
 
@@ -790,14 +819,13 @@ int sgq_llama_block_decode_int4(const sgq_llama_block_int4* blk, const float* x,
     float* ctx = (float*)(base + w.ctx);
     float* h = (float*)(base + w.h);
     float* hid = (float*)(base + w.hid);
-    float* tmp = (float*)(base + w.tmp);
     float* part = (float*)(base + w.part);
     void* split = base + w.split;
 
     // attn->forward(norm1->forward(x)), then the residual: h = x + o(ctx).
     // The GEMV path applies each RMSNorm inside the projection that reads it.
     const bool gemv = decode_uses_gemv(B, D, H);
-    const int cus = gemv ? device_cus(s) : 0;
+    const int cus = device_cus(s);
     if (gemv) {
         const void* pk[3] = {blk->q.packed, blk->k.packed, blk->v.packed};
         const float* ds[3] = {blk->q.devscales, blk->k.devscales, blk->v.devscales};
@@ -823,18 +851,27 @@ int sgq_llama_block_decode_int4(const sgq_llama_block_int4* blk, const float* x,
                 "gemv_o");
     } else {
         SGQ_HIP(launch_rms_norm(x, B, D, blk->norm1, blk->eps, n, s), "rms_norm");
-        float* qb = qkv;
-        float* kb = qkv + B * D;
-        float* vb = qkv + 2 * B * D;
-        SGQ_HIP(launch_gemm_i4(n, B, D, D, blk->q.packed, blk->q.devscales, gdd, blk->q.bias, qb, split, s), "gemm_q");
-        SGQ_HIP(launch_gemm_i4(n, B, D, D, blk->k.packed, blk->k.devscales, gdd, blk->k.bias, kb, split, s), "gemm_k");
-        SGQ_HIP(launch_gemm_i4(n, B, D, D, blk->v.packed, blk->v.devscales, gdd, blk->v.bias, vb, split, s), "gemm_v");
-        SGQ_HIP(launch_attention_decode(qb, kb, vb, D, B, D, k_cache, v_cache, max_tokens, pos, max_len,
+        const SkinnyPlan sq = decode_rows_plan(B, D, D, 3, G, cus);
+        int64_t ldq = 3 * D;  // q, k and v side by side, or one after the other
+        float *qb = qkv, *kb = qkv + D, *vb = qkv + 2 * D;
+        const void* pk[3] = {blk->q.packed, blk->k.packed, blk->v.packed};
+        const float* ds[3] = {blk->q.devscales, blk->k.devscales, blk->v.devscales};
+        const float* bs[3] = {blk->q.bias, blk->k.bias, blk->v.bias};
+        if (sq.C > 0) {
+            SkinnyExtra ex;
+            ex.nw = 3;
+            ex.ldy = 3 * D;
+            SGQ_HIP(launch_skinny_i4(n, B, D, D, 1, pk, ds, bs, gdd, sq, qkv, split, s, &ex), "skinny_qkv");
+        } else {
+            ldq = D;
+            kb = qkv + B * D;
+            vb = qkv + 2 * B * D;
+            SGQ_HIP(launch_gemm_i4(n, B, D, D, 3, pk, ds, bs, gdd, {}, qkv, split, s), "gemm_qkv");
+        }
+        SGQ_HIP(launch_attention_decode(qb, kb, vb, ldq, B, D, k_cache, v_cache, max_tokens, pos, max_len,
                                         blk->attn_scale, part, ctx, s),
                 "attention");
-        SGQ_HIP(launch_gemm_i4(ctx, B, D, D, blk->o.packed, blk->o.devscales, gdd, blk->o.bias, tmp, split, s),
-                "gemm_o");
-        SGQ_HIP(launch_add(x, tmp, h, B * D, s), "add");
+        SGQ_HIP(decode_project(ctx, B, D, D, blk->o, gdd, x, h, split, cus, s), "project_o");
     }
     // h + mlp->forward(norm2->forward(h))
     if (gemv) {
@@ -858,15 +895,21 @@ int sgq_llama_block_decode_int4(const sgq_llama_block_int4* blk, const float* x,
                 "gemv_down");
     } else {
         SGQ_HIP(launch_rms_norm(h, B, D, blk->norm2, blk->eps, n, s), "rms_norm");
-        SGQ_HIP(launch_gemm_i4(n, B, D, H, blk->gate.packed, blk->gate.devscales, gdh, blk->gate.bias, hid, split, s),
-                "gemm_gate");
-        SGQ_HIP(launch_gemm_i4(n, B, D, H, blk->up.packed, blk->up.devscales, gdh, blk->up.bias, tmp, split, s),
-                "gemm_up");
-        SGQ_HIP(launch_silu_mul(hid, tmp, B * H, s), "silu_mul");
-        SGQ_HIP(launch_gemm_i4(hid, B, H, D, blk->down.packed, blk->down.devscales, ghd, blk->down.bias, tmp, split,
-                               s),
-                "gemm_down");
-        SGQ_HIP(launch_add(h, tmp, out, B * D, s), "add");
+        const SkinnyPlan sg = decode_rows_plan(B, D, H, 1, G, cus);
+        if (sg.C > 0) {
+            const void* pk[2] = {blk->gate.packed, blk->up.packed};
+            const float* ds[2] = {blk->gate.devscales, blk->up.devscales};
+            const float* bs[2] = {blk->gate.bias, blk->up.bias};
+            SGQ_HIP(launch_skinny_i4(n, B, D, H, 2, pk, ds, bs, gdh, sg, hid, split, s), "skinny_gate_up");
+        } else {
+            SGQ_HIP(launch_gemm_i4(n, B, D, H, 1, &blk->gate.packed, &blk->gate.devscales, &blk->gate.bias, gdh, {}, hid,
+                                   split, s),
+                    "gemm_gate");
+            SGQ_HIP(launch_gemm_i4(n, B, D, H, 1, &blk->up.packed, &blk->up.devscales, &blk->up.bias, gdh, {hid}, hid,
+                                   split, s),
+                    "gemm_up");
+        }
+        SGQ_HIP(decode_project(hid, B, H, D, blk->down, ghd, h, out, split, cus, s), "project_down");
     }
     return ok();
 }

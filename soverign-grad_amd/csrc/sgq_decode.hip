@@ -1,6 +1,6 @@
 // sgq_decode.hip -- the non-projection kernels of one LLaMA block decode step:
-// RMSNorm, attention of one new token per sequence over its key/value cache,
-// and residual adds.  The projections are the quantized GEMV/GEMM kernels of
+// RMSNorm and attention of one new token per sequence over its key/value
+// cache.  The projections (and the residual adds, in their epilogues) are the quantized GEMV/GEMM kernels of
 // sgq_linear.hip.
 //
 // Reference: LLaMABlock::forward (include/sovereigngrad/models.hpp:217-222)
@@ -55,14 +55,6 @@ __global__ __launch_bounds__(kBlock) void k_rms_norm(const float* __restrict__ x
     ss = block_sum(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float)D + eps);
     for (int64_t d = threadIdx.x; d < D; d += kBlock) orow[d] = (xr[d] * inv) * g[d];
-}
-
-// y[i] = a[i] + b[i]: the block's residual connections (equal-shape add,
-// src/ops.cpp:142-148).
-__global__ __launch_bounds__(kBlock) void k_add(const float* __restrict__ a, const float* __restrict__ b,
-                                                float* __restrict__ y, int64_t n) {
-    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-        y[i] = a[i] + b[i];
 }
 
 // out[i, :] = w[(int)idx[i], :], or zeros for an id outside [0, V)
@@ -380,14 +372,6 @@ hipError_t launch_embedding(const float* idx, int64_t n, const float* w, int64_t
                             hipStream_t s) {
     if (n <= 0 || E <= 0) return hipSuccess;
     k_embedding<<<(unsigned)n, kBlock, 0, s>>>(idx, w, V, E, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_add(const float* a, const float* b, float* y, int64_t n, hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    int64_t blocks = ceil_div(n, kBlock);
-    if (blocks > 4096) blocks = 4096;
-    k_add<<<(unsigned)blocks, kBlock, 0, s>>>(a, b, y, n);
     return hipGetLastError();
 }
 

@@ -1,0 +1,194 @@
+// sgq_device.h -- device helpers shared by the forward kernels of libsgq.so
+// (buffer loads, code conversion, the three-term bf16 split).  Device-only;
+// include from .hip files.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "sgq_internal.h"
+
+namespace sgq {
+namespace {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// Byte B of w read as a signed int8 and converted to fp32: the compiler emits
+// one v_cvt_f32_i32 with an SDWA sign-extended byte select.  For INT4, a byte
+// holding a code in its high nibble and zero below reads as 16*q exactly.
+// Plain C++ rather than inline asm: the hazard recognizer does not track
+// registers written inside inline asm, so an instruction that reads such a
+// register too soon after it is written (an MFMA operand, for one) would get
+// no wait states.
+template <int B>
+__device__ __forceinline__ float cvt_sbyte(uint32_t w) {
+    return (float)(signed char)(w >> (8 * B));
+}
+
+__device__ __forceinline__ float i8_byte(uint32_t w, int b) {
+    return b == 0 ? cvt_sbyte<0>(w) : (b == 1 ? cvt_sbyte<1>(w) : (b == 2 ? cvt_sbyte<2>(w) : cvt_sbyte<3>(w)));
+}
+
+__device__ __forceinline__ float f4get(const float4& v, int i) {
+    return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
+}
+
+// Raw buffer resource over [p, p + bytes): loads through it take a 32-bit
+// lane offset plus a wave-uniform SGPR offset (no per-load 64-bit address
+// math), and every dword past `bytes` reads as 0 -- which is how rows past K
+// and row quads past the strip end contribute nothing.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+}
+
+constexpr int kOobOff = 0x40000000;  // a lane offset past every buffer the forward kernels read
+
+__device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// Loads of weight codes that a launch reads once (the GEMV with one row
+// group, the INT4 skinny kernels: their workgroups partition the columns and
+// K ranges) carry the non-temporal cache policy (`nt`): the stream does not
+// displace x and the scales, which every workgroup of a scale column reads
+// again.  Kernels whose workgroups read a code again (row groups, GEMM row
+// tiles) keep the default policy.  Measured on MI355X (INT4
+// g128, M = 1, graphs of 100 calls): 4096->4096 4.42 -> 4.03 us, 4096->11008
+// 7.33 -> 6.85, 11008->4096 8.15 -> 7.26, 8192->8192 9.75 -> 8.27.
+constexpr int kStreamPolicy = 2;  // buffer-instruction cache policy bit nt (gfx940+)
+__device__ __forceinline__ uint4 buf_load16_stream(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kStreamPolicy);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint32_t buf_load4_stream(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, kStreamPolicy);
+}
+
+// Four floats at byte offset voff + soff (zero past the end).  ALIGN4: the
+// buffer holds a multiple of four floats, so a quad is entirely in or out and
+// one 128-bit load serves; otherwise four 32-bit loads.
+template <bool ALIGN4>
+__device__ __forceinline__ float4 buf_load4f(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    if (ALIGN4) {
+        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+        return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+    } else {
+        return make_float4(__uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 0, soff, 0)),
+                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 4, soff, 0)),
+                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 8, soff, 0)),
+                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 12, soff, 0)));
+    }
+}
+
+// silu(v) = v / (1 + exp(-v)), as simd::vec_silu (simd.hpp:103-108); the
+// device expf differs from libm's by at most a few ulp, the division is
+// correctly rounded.
+__device__ __forceinline__ float silu_f32(float v) { return v / (1.0f + expf(-v)); }
+
+// GemmEpilogue of one product (its bias added).
+__device__ __forceinline__ float gemm_epilogue(const GemmEpilogue& e, float v, int64_t o) {
+    if (e.gate) v = silu_f32(e.gate[o]) * v;
+    if (e.res) v = v + e.res[o];
+    return v;
+}
+
+// Workgroups are dispatched round-robin over the device's X = 2^xlog XCDs
+// (workgroup b runs on XCD b % X; a full MI355X has 8, its partitions 4, 2 or
+// 1, read per device as device_xcds), and each XCD has its own L2.  Strips
+// that share a scale column (and, for the MFMA GEMM, tiles that share
+// operands) should run on the same XCD, so the first X*(n/X) workgroup ids are
+// permuted to give XCD x the contiguous range [x*(n/X), (x+1)*(n/X)); the
+// remaining ids map to themselves.  A bijection on [0, n) for any xlog (0: the
+// identity), so the XCD count only affects speed.
+__device__ __forceinline__ int xcd_swizzle(int b, int n, int xlog) {
+    const int per = n >> xlog;
+    const int sw = (b & ((1 << xlog) - 1)) * per + (b >> xlog);
+    return b >= (per << xlog) ? b : sw;  // a select, not a branch, ahead of the first loads
+}
+
+// Workgroup barrier ordering LDS accesses only: waits for this wave's LDS
+// operations, not for its global loads.  __syncthreads() is a release fence
+// as well, and gfx950 counts loads and stores on one counter (vmcnt), so it
+// waits for every load in flight -- prefetched data included.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+// Upper halves (bf16 bits) of two floats in one dword, lo in bits 0-15.
+__device__ __forceinline__ uint32_t pack_hi16(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+__device__ __forceinline__ float trunc_bf16(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
+
+// Eight nibble codes (k order, nibble 0 first) as the bf16 values 16q of a B
+// operand: high nibbles masked in place and low nibbles shifted up read as
+// signed bytes 16q, converted exactly.
+__device__ __forceinline__ bf16x8 nibbles_bf16x16(uint32_t t) {
+    const uint32_t hi = t & 0xF0F0F0F0u, lo = (t << 4) & 0xF0F0F0F0u;
+    const uint4 b = make_uint4(pack_hi16(cvt_sbyte<0>(lo), cvt_sbyte<0>(hi)), pack_hi16(cvt_sbyte<1>(lo), cvt_sbyte<1>(hi)),
+                               pack_hi16(cvt_sbyte<2>(lo), cvt_sbyte<2>(hi)), pack_hi16(cvt_sbyte<3>(lo), cvt_sbyte<3>(hi)));
+    return __builtin_bit_cast(bf16x8, b);
+}
+
+// Splits eight floats into the bf16 planes h, m, l (four dwords each).
+__device__ __forceinline__ void split3(const float* v, uint4& h, uint4& m, uint4& l) {
+    // No fma: fused with the multiply that made v (x * s), a - trunc(a)
+    // would take the unrounded product, and h + m + l would miss v by up to
+    // an ulp.
+#pragma clang fp contract(off)
+    uint32_t ph[4], pm[4], pl[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = v[2 * i], b = v[2 * i + 1];
+        ph[i] = pack_hi16(a, b);
+        const float ra = a - trunc_bf16(a), rb = b - trunc_bf16(b);
+        pm[i] = pack_hi16(ra, rb);
+        pl[i] = pack_hi16(ra - trunc_bf16(ra), rb - trunc_bf16(rb));
+    }
+    h = make_uint4(ph[0], ph[1], ph[2], ph[3]);
+    m = make_uint4(pm[0], pm[1], pm[2], pm[3]);
+    l = make_uint4(pl[0], pl[1], pl[2], pl[3]);
+}
+
+// split3 of four floats (two dwords per plane).
+__device__ __forceinline__ void split3_4(const float* v, uint2& h, uint2& m, uint2& l) {
+#pragma clang fp contract(off)
+    uint32_t ph[2], pm[2], pl[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const float a = v[2 * i], b = v[2 * i + 1];
+        ph[i] = pack_hi16(a, b);
+        const float ra = a - trunc_bf16(a), rb = b - trunc_bf16(b);
+        pm[i] = pack_hi16(ra, rb);
+        pl[i] = pack_hi16(ra - trunc_bf16(ra), rb - trunc_bf16(rb));
+    }
+    h = make_uint2(ph[0], ph[1]);
+    m = make_uint2(pm[0], pm[1]);
+    l = make_uint2(pl[0], pl[1]);
+}
+
+// One output of the forward as the reference forms it: sum over k in
+// [k0, k1) of x[k] * (q[k][n] * s), in k order (the non-finite fallback).
+template <int BITS>
+__device__ float output_exact(const float* xrow, const uint4* W, const float* S, int mode, int Kpad, int RQ, int n,
+                              int k0, int k1) {
+    float acc = 0.0f;
+    for (int k = k0; k < k1; ++k) {
+        float q, s;
+        if constexpr (BITS == 8) {
+            q = (float)reinterpret_cast<const signed char*>(W)[((int64_t)(n >> 2) * RQ + (k >> 2)) * 16 + (n & 3) * 4 +
+                                                                (k & 3)];
+            s = mode ? S[0] : S[k];
+        } else {
+            const uint32_t d = reinterpret_cast<const uint32_t*>(W + (int64_t)(n >> 3) * RQ)[k];
+            q = (float)(((int)(d << (28 - 4 * (n & 7)))) >> 28);
+            s = S[(int64_t)((n >> 3) / mode) * Kpad + k];
+        }
+        acc = fmaf(xrow[k], q * s, acc);
+    }
+    return acc;
+}
+
+}  // namespace
+}  // namespace sgq

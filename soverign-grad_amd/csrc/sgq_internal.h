@@ -317,13 +317,17 @@ hipError_t launch_skinny_i8(const float* x, int64_t M, int64_t K, int64_t N, con
 // INT4 weights of one shape on one input: ng == 1 writes y = x * W + bias,
 // ng == 2 the gated MLP h = silu(x * Wg + bg) * (x * Wu + bu).  With split K,
 // ws holds skinny_ws_bytes(p, M, N, ng) bytes (16-byte aligned).
-// The whole-K form (p.form == 0, p.S == 1) can also run nw (1..3, ng == 1)
-// weights of one shape side by side, weight w writing columns w * N .. w * N
-// + N - 1 of rows of ldy floats, and fold an RMSNorm of x (gamma, eps) into
-// the projections, as launch_gemv_i4_multi does.
+// Both forms can also run nw (1..3, ng == 1) weights of one shape side by
+// side, weight w writing columns w * N .. w * N + N - 1 of rows of ldy floats
+// (ws: nw times the bytes).  The whole-K form (p.form == 0, p.S == 1) folds an
+// RMSNorm of x (gamma, eps) into the projections, as launch_gemv_i4_multi
+// does, and takes several weights only with it; the super-block form
+// (p.form == 1) adds res (same indexing as y) to the output, and takes several
+// weights of 17 or more rows of 16-byte aligned x.
 struct SkinnyExtra {
     int nw = 1;
     int64_t ldy = 0;  // 0: N
+    const float* res = nullptr;
     const float* gamma = nullptr;
     float eps = 0.0f;
 };
@@ -343,6 +347,15 @@ hipError_t launch_gemv_i4_multi(const float* x, int64_t M, int64_t K, int64_t N,
 // bytes, 0 when K is not split) and a second kernel adds them in fixed order.
 struct GemmPlan {
     int KS, sps;  // splits of K, 32-row stages per split
+};
+constexpr int kMaxSplits = 16;
+// What an INT4 GEMM does to each product v = x W + bias at element o before
+// it stores y[o]: v = silu(gate[o]) * v; v += res[o], each where its pointer is
+// set.  gate and res may be y itself (each element is read before it is
+// written, by the thread that writes it).
+struct GemmEpilogue {
+    const float* gate = nullptr;
+    const float* res = nullptr;
 };
 struct GemmTile {
     int64_t bm, bn, per_cu;  // tile rows and columns, workgroups resident per CU
@@ -372,18 +385,41 @@ int64_t gemm_launch_ws_bytes(int bits, int64_t M, int64_t K, int64_t N, int mode
 // GEMV, 1 the three-term bf16 GEMM, 2 the fp32 GEMM, 3 the flat INT4 kernel,
 // 4 the skinny MFMA kernel; ks the K splits (1: none).
 void linear_plan(int bits, int64_t M, int64_t K, int64_t N, int64_t group_size, int64_t cus, int* path, int* ks);
+int xcd_rect_rows(int64_t tm, int64_t tn, int64_t xb, int64_t wb, int64_t xcds);
 hipError_t launch_gemm_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* scales,
                           bool per_tensor, const float* bias, float* y, void* ws, hipStream_t s);
-hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, const void* packed,
-                          const float* devscales, const I4Geom& g, const float* bias, float* y, void* ws,
-                          hipStream_t s);
+// nw (1..3) weights of one shape on one input: weight w writes y + w * M * N.
+// ws: gemm_workspace_bytes(M, K, nw * N) bytes.
+hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
+                          const float* const* devscales, const float* const* bias, const I4Geom& g,
+                          const GemmEpilogue& ep, float* y, void* ws, hipStream_t s);
+// The INT4 GEMM of independent wavefront tiles (sgq_gemm.hip), for scale
+// columns of a multiple of four strips; p.KS > 1 writes partial tiles to ws.
+struct GemmWaveShape {
+    int rb;  // row blocks of 16 per wavefront tile: 2 or 4
+    int sk;  // K ranges within a workgroup: 1, 2 or 4
+    // Rows and columns of a workgroup's four wavefronts: 2 x 2 tiles of 128
+    // columns, 1 x 2 with two K ranges, one tile with four.
+    int64_t rows() const { return (sk == 1 ? 2 : 1) * 16 * rb; }
+    int64_t cols() const { return (sk == 4 ? 1 : 2) * 128; }
+};
+inline bool gemm_wave_takes(int spc) { return spc % 4 == 0; }
+GemmWaveShape gemm_wave_shape(int64_t M, int64_t N, int spc, int KS, int64_t cus);
+hipError_t launch_gemm_wave(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
+                            const float* const* devscales, const float* const* bias, const I4Geom& g, const GemmPlan& p,
+                            const GemmWaveShape& w, const GemmEpilogue& ep, float* y, void* ws, hipStream_t s);
+// y of nw weights: the sum of the KS partial results in part ([nw][KS][M][N]),
+// in split order, with bias and epilogue.
+hipError_t launch_splitk_reduce(const float* part, int KS, int64_t M, int64_t N, int nw, const float* const* bias,
+                                const GemmEpilogue& ep, float* y, hipStream_t s);
 hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N, const void* packed,
                                  const float* scales, int64_t G, const float* bias, float* y, hipStream_t s);
 
 // Gated MLP: h = silu(x*Wg + bg) * (x*Wu + bu).  The GEMV form (M <= kGemvMaxM)
 // runs both weights in one launch (as does the skinny kernel, launch_skinny_i4
-// with ng == 2); larger batches run two projections and launch_silu_mul
-// (h = silu(h) * u, elementwise over n floats).
+// with ng == 2); GEMM batches run two projections, the second with the first
+// as its epilogue's gate; the INT8 skinny kernel and the flat INT4 layout two
+// projections and launch_silu_mul (h = silu(h) * u, elementwise over n floats).
 hipError_t launch_swiglu_gemv_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed_g,
                                  const float* scales_g, const float* bias_g, const void* packed_u,
                                  const float* scales_u, const float* bias_u, bool per_tensor, float* h,
@@ -397,7 +433,6 @@ hipError_t launch_silu_mul(float* h, const float* u, int64_t n, hipStream_t s);
 // ---- LLaMA block decode step (sgq_decode.hip) ---------------------------
 hipError_t launch_rms_norm(const float* x, int64_t rows, int64_t D, const float* g, float eps, float* out,
                            hipStream_t s);
-hipError_t launch_add(const float* a, const float* b, float* y, int64_t n, hipStream_t s);
 hipError_t launch_embedding(const float* idx, int64_t n, const float* w, int64_t V, int64_t E, float* out,
                             hipStream_t s);
 // Attention of one new token per sequence over its cache: keys split into

@@ -23,6 +23,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "sgq_device.h"
 #include "sgq_internal.h"
 #include "sgq_lanes.h"
 
@@ -37,25 +38,6 @@ constexpr int kThreads = 256;
 #define SGQ_GEMV_MIX_MAXMT 2
 #endif
 constexpr int kGemvMixMaxRows = SGQ_GEMV_MIX_MAXMT;
-
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-// Byte B of w read as a signed int8 and converted to fp32: the compiler emits
-// one v_cvt_f32_i32 with an SDWA sign-extended byte select.  For INT4, a byte
-// holding a code in its high nibble and zero below reads as 16*q exactly.
-// Plain C++ rather than inline asm: the hazard recognizer does not track
-// registers written inside inline asm, so an instruction that reads such a
-// register too soon after it is written (an MFMA operand, for one) would get
-// no wait states.
-template <int B>
-__device__ __forceinline__ float cvt_sbyte(uint32_t w) {
-    return (float)(signed char)(w >> (8 * B));
-}
-
-__device__ __forceinline__ float i8_byte(uint32_t w, int b) {
-    return b == 0 ? cvt_sbyte<0>(w) : (b == 1 ? cvt_sbyte<1>(w) : (b == 2 ? cvt_sbyte<2>(w) : cvt_sbyte<3>(w)));
-}
 
 // INT4 decode of the GEMV.  A two's-complement nibble q in [-8, 7] XOR 8 is
 // its offset-binary form u = q + 8 in [0, 15].  Masked into the low bits of a
@@ -91,83 +73,6 @@ __device__ float i4_column_exact(const uint4* W, const float* SC, int j, int e, 
     }
     return acc;
 }
-
-__device__ __forceinline__ float f4get(const float4& v, int i) {
-    return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
-}
-
-// Raw buffer resource over [p, p + bytes): loads through it take a 32-bit
-// lane offset plus a wave-uniform SGPR offset (no per-load 64-bit address
-// math), and every dword past `bytes` reads as 0 -- which is how rows past K
-// and row quads past the strip end contribute nothing.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-}
-
-constexpr int kOobOff = 0x40000000;  // a lane offset past every buffer the forward kernels read
-
-__device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-
-// Loads of weight codes that a launch reads once (the GEMV with one row
-// group, the INT4 skinny kernels: their workgroups partition the columns and
-// K ranges) carry the non-temporal cache policy (`nt`): the stream does not
-// displace x and the scales, which every workgroup of a scale column reads
-// again.  Kernels whose workgroups read a code again (row groups, GEMM row
-// tiles) keep the default policy.  Measured on MI355X (INT4
-// g128, M = 1, graphs of 100 calls): 4096->4096 4.42 -> 4.03 us, 4096->11008
-// 7.33 -> 6.85, 11008->4096 8.15 -> 7.26, 8192->8192 9.75 -> 8.27.
-constexpr int kStreamPolicy = 2;  // buffer-instruction cache policy bit nt (gfx940+)
-__device__ __forceinline__ uint4 buf_load16_stream(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kStreamPolicy);
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint32_t buf_load4_stream(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, kStreamPolicy);
-}
-
-// Four floats at byte offset voff + soff (zero past the end).  ALIGN4: the
-// buffer holds a multiple of four floats, so a quad is entirely in or out and
-// one 128-bit load serves; otherwise four 32-bit loads.
-template <bool ALIGN4>
-__device__ __forceinline__ float4 buf_load4f(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    if (ALIGN4) {
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-        return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-    } else {
-        return make_float4(__uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 0, soff, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 4, soff, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 8, soff, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 12, soff, 0)));
-    }
-}
-
-// silu(v) = v / (1 + exp(-v)), as simd::vec_silu (simd.hpp:103-108); the
-// device expf differs from libm's by at most a few ulp, the division is
-// correctly rounded.
-__device__ __forceinline__ float silu_f32(float v) { return v / (1.0f + expf(-v)); }
-
-// Workgroups are dispatched round-robin over the device's X = 2^xlog XCDs
-// (workgroup b runs on XCD b % X; a full MI355X has 8, its partitions 4, 2 or
-// 1, read per device as device_xcds), and each XCD has its own L2.  Strips
-// that share a scale column (and, for the MFMA GEMM, tiles that share
-// operands) should run on the same XCD, so the first X*(n/X) workgroup ids are
-// permuted to give XCD x the contiguous range [x*(n/X), (x+1)*(n/X)); the
-// remaining ids map to themselves.  A bijection on [0, n) for any xlog (0: the
-// identity), so the XCD count only affects speed.
-__device__ __forceinline__ int xcd_swizzle(int b, int n, int xlog) {
-    const int per = n >> xlog;
-    const int sw = (b & ((1 << xlog) - 1)) * per + (b >> xlog);
-    return b >= (per << xlog) ? b : sw;  // a select, not a branch, ahead of the first loads
-}
-
-// Workgroup barrier ordering LDS accesses only: waits for this wave's LDS
-// operations, not for its global loads.  __syncthreads() is a release fence
-// as well, and gfx950 counts loads and stores on one counter (vmcnt), so it
-// waits for every load in flight -- prefetched data included.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Arguments of one GEMV launch (passed by value in the kernel arguments).
 struct GemvArgs {
@@ -519,25 +424,20 @@ constexpr int kBM = 128, kBN = 128, kBK = SGQ_GEMM_BK, kLdsStride = kBK + 4;
 constexpr int kStoreBlock = SGQ_GEMM_STORE_BLOCK;  // 16-k block of a stage before which the next stage is stored
 static_assert(kBK % 16 == 0 && kBK <= 64, "stage depth is a multiple of 16");
 
-template <int BITS, bool KALIGN4>
+template <bool KALIGN4>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm(const float* __restrict__ x, int M, int K, int N,
                                                    const uint4* __restrict__ W, const float* __restrict__ S,
                                                    int mode, int Kpad, int RQ, int NS, int KS, int sps,
-                                                   const float* __restrict__ bias, float* __restrict__ y,
+                                                   const float* __restrict__ bias, const GemmEpilogue ep, float* y,
                                                    float* __restrict__ part) {
-    // mode: INT8 -> per_tensor flag; INT4 -> strips per scale column (spc).
+    // mode: strips per scale column (spc).
     // Workgroup b computes split b % KS (stages [kt0, kt1) of sps each) of
     // tile b / KS; with KS > 1 it writes part[split][M][N] instead of y.
-    constexpr int SW = (BITS == 4) ? 8 : 4;
+    constexpr int SW = 8;                       // columns per strip
     constexpr int KQ = kBK / 4;                 // row quads per stage
-    constexpr int kStrips = kBN / SW;           // strips per tile: 16 (INT4) or 32 (INT8)
-    // INT4: B dequantized to fp32 [n][k].  INT8: B as the raw 16-byte chunks
-    // (strip, row quad), each dword four consecutive k of one column -- what
-    // an MFMA lane consumes -- with the strip stride padded to KQ*4 + 8 dwords
-    // so the 32 lanes of a half-wave read 32 different banks.
+    constexpr int kStrips = kBN / SW;           // strips per tile
     __shared__ __attribute__((aligned(16))) float As[2][kBM][kLdsStride];
-    __shared__ __attribute__((aligned(16))) float Bs[BITS == 4 ? 2 : 1][BITS == 4 ? kBN : 1][kLdsStride];
-    __shared__ __attribute__((aligned(16))) uint4 Bq[BITS == 8 ? 2 : 1][BITS == 8 ? kStrips : 1][KQ + 2];
+    __shared__ __attribute__((aligned(16))) float Bs[2][kBN][kLdsStride];  // B dequantized, [n][k]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int ntn = (N + kBN - 1) / kBN;
@@ -546,11 +446,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int m0 = tm * kBM, n0 = tn * kBN;
     const int KT = (Kpad + kBK - 1) / kBK;  // the last stage may reach past Kpad: masked below
     const int kt0 = split * sps, kt1 = (kt0 + sps) < KT ? (kt0 + sps) : KT;
-    // Scales: INT8 per-channel scales[k] (zero past K), per-tensor scales[0];
-    // INT4 devscales[sc][Kpad].
-    const __amdgpu_buffer_rsrc_t rS =
-        make_rsrc(S, BITS == 8 ? (mode ? 4u : (uint32_t)K * 4u) : (uint32_t)(((NS + mode - 1) / mode) * Kpad) * 4u);
-    const float s_all = (BITS == 8 && mode) ? S[0] : 0.0f;
+    // Scales: devscales[sc][Kpad].
+    const __amdgpu_buffer_rsrc_t rS = make_rsrc(S, (uint32_t)(((NS + mode - 1) / mode) * Kpad) * 4u);
 
     constexpr int kBChunks = kStrips * KQ;      // chunks of B per stage
     constexpr int kAVec = kBM * kBK / 4 / kThreads;  // float4 of A per thread per stage
@@ -564,7 +461,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     struct Regs {
         float4 a[kAVec];
         uint4 b[kBPer];
-        float4 s;  // INT8 per-channel: scales of this thread's four A columns k
     };
     // Buffer resources over this tile's rows of x and strips of W: rows past
     // M and strips past NS read as zero; k past K and row quads past RQ (which
@@ -599,34 +495,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int vo = ((t / KQ) * RQ + t % KQ) * 16;
             rg.b[i] = buf_load16(rW, (t < kBChunks && rq < RQ) ? vo : kOobOff, soffB);
         }
-        // Every A float4 of this thread sits at column quad tid % KQ of the stage.
-        if constexpr (BITS == 8)
-            if (!mode) rg.s = buf_load4f<KALIGN4>(rS, (tid % KQ) * 16, kt * kBK * 4);  // zero past K
     };
     auto store = [&](const Regs& rg, int buf, int kt) {
-        // INT8: the scale of row k of W goes into column k of A, (x * s) * q
-        // (the reference forms x * (q * s): the same products up to one
-        // rounding); columns past K are exactly zero, also for a non-finite
-        // per-tensor scale.
-        float4 sa = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-        if constexpr (BITS == 8) {
-            if (mode) {
-                const int k = kt * kBK + (tid % KQ) * 4;
-                sa = make_float4(k < K ? s_all : 0.0f, k + 1 < K ? s_all : 0.0f, k + 2 < K ? s_all : 0.0f,
-                                 k + 3 < K ? s_all : 0.0f);
-            } else {
-                sa = rg.s;
-            }
-        }
 #pragma unroll
         for (int i = 0; i < kAVec; ++i) {
             const int idx = tid + kThreads * i;
             const int row = idx / KQ, kq = idx % KQ;
-            if constexpr (BITS == 8)
-                *(float4*)&As[buf][row][kq * 4] =
-                    make_float4(rg.a[i].x * sa.x, rg.a[i].y * sa.y, rg.a[i].z * sa.z, rg.a[i].w * sa.w);
-            else
-                *(float4*)&As[buf][row][kq * 4] = rg.a[i];
+            *(float4*)&As[buf][row][kq * 4] = rg.a[i];
         }
 #pragma unroll
         for (int i = 0; i < kBPer; ++i) {
@@ -635,33 +510,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int jl = t / KQ, kl = (t % KQ) * 4;
             const int k = kt * kBK + kl;
             const uint32_t dw[4] = {rg.b[i].x, rg.b[i].y, rg.b[i].z, rg.b[i].w};
-            if constexpr (BITS == 8) {
-                (void)dw;
-                (void)k;
-                Bq[buf][jl][kl / 4] = rg.b[i];
-            } else {
-                const int bj = n0 / SW + jl;
-                const int jc = bj < NS ? bj : NS - 1;
-                // devscales rows stop at Kpad (codes there are zero); the
-                // 1/16 turns the 16*q read of a high nibble back into q (exact)
-                const float4 s4 = buf_load4f<true>(rS, k < Kpad ? ((jc / mode) * Kpad + kl) * 4 : kOobOff,
-                                                   kt * kBK * 4);
-                const float sc[4] = {s4.x * 0.0625f, s4.y * 0.0625f, s4.z * 0.0625f, s4.w * 0.0625f};
-                uint32_t lo[4], hi[4];
+            const int bj = n0 / SW + jl;
+            const int jc = bj < NS ? bj : NS - 1;
+            // devscales rows stop at Kpad (codes there are zero); the
+            // 1/16 turns the 16*q read of a high nibble back into q (exact)
+            const float4 s4 = buf_load4f<true>(rS, k < Kpad ? ((jc / mode) * Kpad + kl) * 4 : kOobOff,
+                                               kt * kBK * 4);
+            const float sc[4] = {s4.x * 0.0625f, s4.y * 0.0625f, s4.z * 0.0625f, s4.w * 0.0625f};
+            uint32_t lo[4], hi[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    hi[r] = dw[r] & 0xF0F0F0F0u;         // byte c: column 2c+1 of row r, as 16*q
-                    lo[r] = (dw[r] << 4) & 0xF0F0F0F0u;  // byte c: column 2c
-                }
+            for (int r = 0; r < 4; ++r) {
+                hi[r] = dw[r] & 0xF0F0F0F0u;         // byte c: column 2c+1 of row r, as 16*q
+                lo[r] = (dw[r] << 4) & 0xF0F0F0F0u;  // byte c: column 2c
+            }
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    *(float4*)&Bs[buf][jl * 8 + 2 * c][kl] =
-                        make_float4(i8_byte(lo[0], c) * sc[0], i8_byte(lo[1], c) * sc[1], i8_byte(lo[2], c) * sc[2],
-                                    i8_byte(lo[3], c) * sc[3]);
-                    *(float4*)&Bs[buf][jl * 8 + 2 * c + 1][kl] =
-                        make_float4(i8_byte(hi[0], c) * sc[0], i8_byte(hi[1], c) * sc[1], i8_byte(hi[2], c) * sc[2],
-                                    i8_byte(hi[3], c) * sc[3]);
-                }
+            for (int c = 0; c < 4; ++c) {
+                *(float4*)&Bs[buf][jl * 8 + 2 * c][kl] =
+                    make_float4(i8_byte(lo[0], c) * sc[0], i8_byte(lo[1], c) * sc[1], i8_byte(lo[2], c) * sc[2],
+                                i8_byte(lo[3], c) * sc[3]);
+                *(float4*)&Bs[buf][jl * 8 + 2 * c + 1][kl] =
+                    make_float4(i8_byte(hi[0], c) * sc[0], i8_byte(hi[1], c) * sc[1], i8_byte(hi[2], c) * sc[2],
+                                i8_byte(hi[3], c) * sc[3]);
             }
         }
     };
@@ -688,18 +557,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             float4 a[4], b[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) a[i] = *(const float4*)&As[buf][wm * 64 + i * 16 + lr][lk];
-            if constexpr (BITS == 8) {
-                // one dword: column n, rows lk .. lk+3, converted here
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int nl = wn * 64 + j * 16 + lr;
-                    const uint32_t bd = ((const uint32_t*)&Bq[buf][nl >> 2][lk >> 2])[nl & 3];
-                    b[j] = make_float4(cvt_sbyte<0>(bd), cvt_sbyte<1>(bd), cvt_sbyte<2>(bd), cvt_sbyte<3>(bd));
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) b[j] = *(const float4*)&Bs[buf][wn * 64 + j * 16 + lr][lk];
-            }
+            for (int j = 0; j < 4; ++j) b[j] = *(const float4*)&Bs[buf][wn * 64 + j * 16 + lr][lk];
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
@@ -729,15 +588,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int j = 0; j < 4; ++j) {
             const int n = n0 + wn * 64 + j * 16 + lr;
             if (n >= N) continue;
-            const float bv = (bias && KS == 1) ? bias[n] : 0.0f;
-            float* out = KS == 1 ? y : part + (int64_t)split * M * N;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + wm * 64 + i * 16 + (lane >> 4) * 4 + r;
-                if (m < M) {
-                    const float v = acc[i][j][r];
-                    out[(int64_t)m * N + n] = (bias && KS == 1) ? v + bv : v;
-                }
+                if (m >= M) continue;
+                const int64_t o = (int64_t)m * N + n;
+                if (KS == 1)
+                    y[o] = gemm_epilogue(ep, bias ? acc[i][j][r] + bias[n] : acc[i][j][r], o);
+                else
+                    part[(int64_t)split * M * N + o] = acc[i][j][r];
             }
         }
 }
@@ -769,85 +628,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 // planes) or one column (B): one MFMA operand.  Per-tensor INT8 puts x itself
 // into A and multiplies by the scale in the epilogue.
 // ---------------------------------------------------------------------------
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int kB3BK = 32;           // k per stage: one 16x16x32 MFMA step
 constexpr int kB3KG = kB3BK / 8;    // 8-k groups per stage
 constexpr int kB3RQ = kB3BK / 4;    // row quads per stage
-
-// Upper halves (bf16 bits) of two floats in one dword, lo in bits 0-15.
-__device__ __forceinline__ uint32_t pack_hi16(float lo, float hi) {
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-__device__ __forceinline__ float trunc_bf16(float v) { return __uint_as_float(__float_as_uint(v) & 0xFFFF0000u); }
-
-// Eight nibble codes (k order, nibble 0 first) as the bf16 values 16q of a B
-// operand: high nibbles masked in place and low nibbles shifted up read as
-// signed bytes 16q, converted exactly.
-__device__ __forceinline__ bf16x8 nibbles_bf16x16(uint32_t t) {
-    const uint32_t hi = t & 0xF0F0F0F0u, lo = (t << 4) & 0xF0F0F0F0u;
-    const uint4 b = make_uint4(pack_hi16(cvt_sbyte<0>(lo), cvt_sbyte<0>(hi)), pack_hi16(cvt_sbyte<1>(lo), cvt_sbyte<1>(hi)),
-                               pack_hi16(cvt_sbyte<2>(lo), cvt_sbyte<2>(hi)), pack_hi16(cvt_sbyte<3>(lo), cvt_sbyte<3>(hi)));
-    return __builtin_bit_cast(bf16x8, b);
-}
-
-// Splits eight floats into the bf16 planes h, m, l (four dwords each).
-__device__ __forceinline__ void split3(const float* v, uint4& h, uint4& m, uint4& l) {
-    // No fma: fused with the multiply that made v (x * s), a - trunc(a)
-    // would take the unrounded product, and h + m + l would miss v by up to
-    // an ulp.
-#pragma clang fp contract(off)
-    uint32_t ph[4], pm[4], pl[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float a = v[2 * i], b = v[2 * i + 1];
-        ph[i] = pack_hi16(a, b);
-        const float ra = a - trunc_bf16(a), rb = b - trunc_bf16(b);
-        pm[i] = pack_hi16(ra, rb);
-        pl[i] = pack_hi16(ra - trunc_bf16(ra), rb - trunc_bf16(rb));
-    }
-    h = make_uint4(ph[0], ph[1], ph[2], ph[3]);
-    m = make_uint4(pm[0], pm[1], pm[2], pm[3]);
-    l = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-}
-
-// split3 of four floats (two dwords per plane).
-__device__ __forceinline__ void split3_4(const float* v, uint2& h, uint2& m, uint2& l) {
-#pragma clang fp contract(off)
-    uint32_t ph[2], pm[2], pl[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const float a = v[2 * i], b = v[2 * i + 1];
-        ph[i] = pack_hi16(a, b);
-        const float ra = a - trunc_bf16(a), rb = b - trunc_bf16(b);
-        pm[i] = pack_hi16(ra, rb);
-        pl[i] = pack_hi16(ra - trunc_bf16(ra), rb - trunc_bf16(rb));
-    }
-    h = make_uint2(ph[0], ph[1]);
-    m = make_uint2(pm[0], pm[1]);
-    l = make_uint2(pl[0], pl[1]);
-}
-
-// One output of the forward as the reference forms it: sum over k in
-// [k0, k1) of x[k] * (q[k][n] * s), in k order (the non-finite fallback).
-template <int BITS>
-__device__ float output_exact(const float* xrow, const uint4* W, const float* S, int mode, int Kpad, int RQ, int n,
-                              int k0, int k1) {
-    float acc = 0.0f;
-    for (int k = k0; k < k1; ++k) {
-        float q, s;
-        if constexpr (BITS == 8) {
-            q = (float)reinterpret_cast<const signed char*>(W)[((int64_t)(n >> 2) * RQ + (k >> 2)) * 16 + (n & 3) * 4 +
-                                                                (k & 3)];
-            s = mode ? S[0] : S[k];
-        } else {
-            const uint32_t d = reinterpret_cast<const uint32_t*>(W + (int64_t)(n >> 3) * RQ)[k];
-            q = (float)(((int)(d << (28 - 4 * (n & 7)))) >> 28);
-            s = S[(int64_t)((n >> 3) / mode) * Kpad + k];
-        }
-        acc = fmaf(xrow[k], q * s, acc);
-    }
-    return acc;
-}
 
 // Tile shape: WM x WN wavefronts, each RB x CB blocks of 16x16 outputs, so
 // the tile is BM = 16 * RB * WM rows by BN = 16 * CB * WN columns.  A wider
@@ -861,10 +644,9 @@ struct G3Shape {
     static constexpr int BM = 16 * RB * WM, BN = 16 * CB * WN;
     static constexpr int WPE = RB * CB >= 16 ? 2 : 1;  // minimum waves per SIMD the register budget keeps
 };
-using G3Wide = G3Shape<2, 4, 4, 4>;  // 128 x 256, 8 wavefronts: INT8
-using G3Tile = G3Shape<2, 4, 2, 4>;  // 128 x 128, 4 wavefronts: INT4
+using G3Wide = G3Shape<2, 4, 4, 4>;  // 128 x 256, 8 wavefronts
 // Skinny batches (17..64 rows) waste most of a 128-row tile's MFMA work and
-// split work: they take 32- or 64-row tiles (either code width, 128 columns).
+// split work: they take 32- or 64-row tiles of 128 columns.
 using G3Rows32 = G3Shape<1, 2, 2, 4>;  // 32 x 128, 2 wavefronts
 using G3Rows64 = G3Shape<2, 2, 2, 4>;  // 64 x 128, 4 wavefronts
 
@@ -876,36 +658,32 @@ struct Gemm3Args {
     int M, K, N;
     const uint4* W;
     const float* S;
-    int mode, Kpad, RQ, NS, KS, sps;
+    int Kpad, RQ, NS, KS, sps;
     const float* bias;
     float* y;
     float* part;
     int xr, xlog;
-    int ko;  // INT4: byte offset / 256 of the k-octet copy
 };
 
-template <int BITS, bool KALIGN4, bool PT, class SH>
+template <bool KALIGN4, bool PT, class SH>
 __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE))) void k_gemm3(const Gemm3Args ga) {
     const float* __restrict__ x = ga.x;
     const int M = ga.M, K = ga.K, N = ga.N;
     const uint4* __restrict__ W = ga.W;
     const float* __restrict__ S = ga.S;
-    const int mode = ga.mode, Kpad = ga.Kpad, RQ = ga.RQ, NS = ga.NS, KS = ga.KS, sps = ga.sps;
+    const int Kpad = ga.Kpad, RQ = ga.RQ, NS = ga.NS, KS = ga.KS, sps = ga.sps;
     const float* __restrict__ bias = ga.bias;
     float* __restrict__ y = ga.y;
     float* __restrict__ part = ga.part;
     const int xr = ga.xr, xlog = ga.xlog;
-    // mode: INT8 -> per-tensor flag (also the template flag PT, so that no
-    // stage holds a branch); INT4 -> strips per scale column (a multiple of
-    // 16: one scale column per 128-column tile).  Workgroup b computes split
-    // b % KS (stages [kt0, kt1) of sps each) of tile b / KS.  xr > 0 (no K
-    // split): each XCD takes a rectangle of xr tile rows (see below).
-    constexpr int SW = (BITS == 4) ? 8 : 4;
+    // Workgroup b computes split b % KS (stages [kt0, kt1) of sps each) of
+    // tile b / KS.  xr > 0 (no K split): each XCD takes a rectangle of xr tile
+    // rows (see below).
+    constexpr int SW = 4;  // columns per strip
     constexpr int NT = SH::NT, BM = SH::BM, BN = SH::BN, RB = SH::RB, CB = SH::CB;
     constexpr int EA = BM * kB3KG / NT;  // A entries (row, k group) per thread
     constexpr int EB = BN * kB3KG / NT;  // B entries (column, k group) per thread
     static_assert(BM * kB3KG % NT == 0 && EA >= 1 && BN * kB3KG % NT == 0 && EB >= 1, "entries spread evenly");
-    static_assert(BITS == 8 || BN == 128, "an INT4 tile spans one scale column");
     __shared__ uint4 As[2][3][kB3KG][BM];
     __shared__ uint4 Bs[2][kB3KG][BN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -942,34 +720,19 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
     constexpr int kStep = NT / 4;  // rows or columns between a thread's entries
     const int mrows = (M - m0) < BM ? (M - m0) : BM;
     const __amdgpu_buffer_rsrc_t rX = make_rsrc(x + (int64_t)m0 * K, (uint32_t)mrows * (uint32_t)K * 4u);
-    // Scale of column k of A (zero past K): per-channel scales[k], INT4 the
-    // tile's scale column devscales[sc][k].  Per-tensor: x itself goes into A
-    // (zero past K) and the epilogue multiplies by scales[0].
-    __amdgpu_buffer_rsrc_t rS;
-    if constexpr (BITS == 8)
-        rS = make_rsrc(S, PT ? 4u : (uint32_t)K * 4u);
-    else
-        rS = make_rsrc(S + (int64_t)((n0 / SW) / mode) * Kpad, (uint32_t)K * 4u);
-    // B side: an entry holds the eight k of its k group for one column.
-    // INT8: the column's dword of the two strip chunks (row quads 2 * kg and
-    // 2 * kg + 1) that hold them; strips past NS read as zero.  INT4: one
-    // dword of the k-octet copy, block (column / 16, stage) dword 16 kg +
-    // column % 16, which holds exactly those eight codes; column blocks past
-    // the weight's read as zero.
-    const int KB = (Kpad + kB3BK - 1) / kB3BK;
-    __amdgpu_buffer_rsrc_t rW;
-    if constexpr (BITS == 8) {
-        const int nstr = (NS - n0 / SW) < (BN / SW) ? (NS - n0 / SW) : (BN / SW);
-        rW = make_rsrc(W + (int64_t)(n0 / SW) * RQ, (uint32_t)nstr * (uint32_t)RQ * 16u);
-    } else {
-        const int ncb = ((NS + 1) / 2 - n0 / 16) < (BN / 16) ? ((NS + 1) / 2 - n0 / 16) : (BN / 16);
-        rW = make_rsrc(W + ((int64_t)ga.ko + (int64_t)(n0 / 16) * KB) * 16, (uint32_t)ncb * (uint32_t)KB * 256u);
-    }
+    // Scale of column k of A (zero past K): per-channel scales[k].  Per-tensor:
+    // x itself goes into A (zero past K) and the epilogue multiplies by scales[0].
+    const __amdgpu_buffer_rsrc_t rS = make_rsrc(S, PT ? 4u : (uint32_t)K * 4u);
+    // B side: an entry holds the eight k of its k group for one column, the
+    // column's dword of the two strip chunks (row quads 2 * kg and 2 * kg + 1)
+    // that hold them; strips past NS read as zero.
+    const int nstr = (NS - n0 / SW) < (BN / SW) ? (NS - n0 / SW) : (BN / SW);
+    const __amdgpu_buffer_rsrc_t rW = make_rsrc(W + (int64_t)(n0 / SW) * RQ, (uint32_t)nstr * (uint32_t)RQ * 16u);
 
     struct Regs {
         float4 a[EA][2];  // [entry][quad]
         float4 s[2];      // scales of the thread's eight k
-        uint2 b[EB];      // [entry]: INT8 {lo, hi} dwords, INT4 the k-octet dword in .x
+        uint2 b[EB];      // [entry]: {lo, hi} dwords
     };
     auto load = [&](Regs& rg, int kt) {
         const int kb = kt * kB3BK + akg * 8;
@@ -994,25 +757,15 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
 #pragma unroll
             for (int q = 0; q < 2; ++q) rg.s[q] = buf_load4f<KALIGN4>(rS, (akg * 8 + 4 * q) * 4, soff);
         }
-        if constexpr (BITS == 8) {
-            // RQ is a multiple of 4, so both row quads of the pair are in or out together.
-            const bool in = kt * kB3RQ + 2 * akg < RQ;
-            const int bsoff = kt * kB3RQ * 16;
+        // RQ is a multiple of 4, so both row quads of the pair are in or out together.
+        const bool in = kt * kB3RQ + 2 * akg < RQ;
+        const int bsoff = kt * kB3RQ * 16;
 #pragma unroll
-            for (int c = 0; c < EB; ++c) {
-                const int n = ar + kStep * c;
-                const int vd = ((n / SW) * RQ + 2 * akg) * 16 + (n & 3) * 4;
-                rg.b[c].x = __builtin_amdgcn_raw_buffer_load_b32(rW, in ? vd : kOobOff, bsoff, 0);
-                rg.b[c].y = __builtin_amdgcn_raw_buffer_load_b32(rW, in ? vd + 16 : kOobOff, bsoff, 0);
-            }
-        } else {
-            const bool in = kt < KB;
-#pragma unroll
-            for (int c = 0; c < EB; ++c) {
-                const int n = ar + kStep * c;
-                const int vd = (n >> 4) * KB * 256 + (16 * akg + (n & 15)) * 4;
-                rg.b[c].x = __builtin_amdgcn_raw_buffer_load_b32(rW, in ? vd : kOobOff, kt * 256, 0);
-            }
+        for (int c = 0; c < EB; ++c) {
+            const int n = ar + kStep * c;
+            const int vd = ((n / SW) * RQ + 2 * akg) * 16 + (n & 3) * 4;
+            rg.b[c].x = __builtin_amdgcn_raw_buffer_load_b32(rW, in ? vd : kOobOff, bsoff, 0);
+            rg.b[c].y = __builtin_amdgcn_raw_buffer_load_b32(rW, in ? vd + 16 : kOobOff, bsoff, 0);
         }
     };
     auto store = [&](const Regs& rg, int buf) {
@@ -1027,18 +780,13 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
         }
 #pragma unroll
         for (int c = 0; c < EB; ++c) {
-            if constexpr (BITS == 8) {
-                // bytes of the column's dword in each chunk: k = 0..3, then 4..7
-                const uint32_t lo = rg.b[c].x, hi = rg.b[c].y;
-                float f[8];
-                f[0] = cvt_sbyte<0>(lo), f[1] = cvt_sbyte<1>(lo), f[2] = cvt_sbyte<2>(lo), f[3] = cvt_sbyte<3>(lo);
-                f[4] = cvt_sbyte<0>(hi), f[5] = cvt_sbyte<1>(hi), f[6] = cvt_sbyte<2>(hi), f[7] = cvt_sbyte<3>(hi);
-                Bs[buf][akg][ar + kStep * c] = make_uint4(pack_hi16(f[0], f[1]), pack_hi16(f[2], f[3]),
-                                                           pack_hi16(f[4], f[5]), pack_hi16(f[6], f[7]));
-            } else {
-                // the eight codes as 16q (the epilogue divides by 16)
-                Bs[buf][akg][ar + kStep * c] = __builtin_bit_cast(uint4, nibbles_bf16x16(rg.b[c].x));
-            }
+            // bytes of the column's dword in each chunk: k = 0..3, then 4..7
+            const uint32_t lo = rg.b[c].x, hi = rg.b[c].y;
+            float f[8];
+            f[0] = cvt_sbyte<0>(lo), f[1] = cvt_sbyte<1>(lo), f[2] = cvt_sbyte<2>(lo), f[3] = cvt_sbyte<3>(lo);
+            f[4] = cvt_sbyte<0>(hi), f[5] = cvt_sbyte<1>(hi), f[6] = cvt_sbyte<2>(hi), f[7] = cvt_sbyte<3>(hi);
+            Bs[buf][akg][ar + kStep * c] = make_uint4(pack_hi16(f[0], f[1]), pack_hi16(f[2], f[3]),
+                                                       pack_hi16(f[4], f[5]), pack_hi16(f[6], f[7]));
         }
     };
 
@@ -1052,11 +800,10 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
     // Raised wave priority while a wavefront issues its MFMAs lets the two
     // wavefronts of a SIMD drift out of phase: one in its MFMAs, the other
     // loading and splitting.  Measured per form (two runs, builds
-    // interleaved): INT4 with the priority over all MFMAs of a stage, 4-5%
-    // faster; INT8 per-tensor over the first half (up to the store),
-    // 1.4-1.8%; INT8 per-channel, whose store does more VALU work, 1-5% slower
-    // with either, so without.  2: whole stage, 1: first half, 0: none.
-    constexpr int kPrio = BITS == 4 ? 2 : (PT ? 1 : 0);
+    // interleaved): per tensor, over the first half of a stage (up to the
+    // store), 1.4-1.8% faster; per channel, whose store does more VALU work,
+    // 1-5% slower with it, so without.
+    constexpr bool kPrio = PT;
     auto stage = [&](int kt, const Regs& next, Regs& fill) {
         const int buf = kt & 1;
         load(fill, kt + 2);  // past the last stage these read zeros
@@ -1067,10 +814,10 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
         for (int p = 0; p < 3; ++p)
 #pragma unroll
             for (int i = 0; i < RB; ++i) af[p][i] = As[buf][p][lkg][wm * 16 * RB + i * 16 + lr];
-        if constexpr (kPrio > 0) __builtin_amdgcn_s_setprio(1);
+        if constexpr (kPrio) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
-            if (kPrio == 1 && i == RB / 2) __builtin_amdgcn_s_setprio(0);
+            if (kPrio && i == RB / 2) __builtin_amdgcn_s_setprio(0);
             if (i == RB / 2 && kt + 1 < kt1) store(next, buf ^ 1);
 #pragma unroll
             for (int j = 0; j < CB; ++j)
@@ -1080,7 +827,6 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
                                                                         __builtin_bit_cast(bf16x8, bq[j]), acc[i][j],
                                                                         0, 0, 0);
         }
-        if constexpr (kPrio == 2) __builtin_amdgcn_s_setprio(0);
         lds_barrier();
     };
 
@@ -1114,9 +860,8 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + wm * 16 * RB + i * 16 + lkg * 4 + r;
                 if (m < M) {
-                    // INT4 codes entered as 16q: an exact division by 16.
-                    float v = BITS == 4 ? acc[i][j][r] * 0.0625f : (PT ? acc[i][j][r] * s_all : acc[i][j][r]);
-                    if (!isfinite(v)) v = output_exact<BITS>(x + (int64_t)m * K, W, S, mode, Kpad, RQ, n, klo, khi);
+                    float v = PT ? acc[i][j][r] * s_all : acc[i][j][r];
+                    if (!isfinite(v)) v = output_exact<8>(x + (int64_t)m * K, W, S, PT ? 1 : 0, Kpad, RQ, n, klo, khi);
                     out[(int64_t)m * N + n] = (bias && KS == 1) ? v + bv : v;
                 }
             }
@@ -1166,11 +911,12 @@ struct SkinnyArgs {
     int nblk;     // grid size
     int slog;     // log2 of the number of K ranges
     int sbs;      // super-blocks (128 rows) per K range
-    // Whole-K form only: weight w of nw side by side writes columns
-    // w * N .. w * N + N - 1 of y; NORM: the RMSNorm weight and epsilon.
+    // Weight w of nw side by side writes columns w * N .. w * N + N - 1 of y.
     int ldy;
-    int wgpw;     // workgroups per weight
-    FastDiv wgd;  // division by wgpw
+    int wgpw;          // workgroups (column groups) per weight
+    FastDiv wgd;       // division by wgpw
+    const float* res;  // super-block form: added to the output (same indexing), or null
+    // Whole-K form only (NORM): the RMSNorm weight and epsilon.
     const float* gamma;
     float eps;
     int xlog;     // log2 of the device's XCD count
@@ -1449,9 +1195,13 @@ struct SkinnyRegs {
 // first quad of each k block of row n (quad t is k block t) and lane n + 8 the
 // second; a row_ror:8 exchange completes each A operand (the same bf16
 // planes).
-template <int NW, int C, int NG, bool XA, int MB, bool SPLIT, bool HALF>
+//
+// MULTI (NG == 1): a.wgpw column groups per weight over nw weights of one
+// shape side by side, as k_skinny3.
+template <int NW, int C, int NG, bool XA, int MB, bool SPLIT, bool HALF, bool MULTI>
 __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, const SkinnyArgs a) {
     static_assert(!HALF || MB == 1, "the half-row form has one row block");
+    static_assert(!MULTI || NG == 1, "weights side by side are plain projections");
     constexpr int XT = HALF ? 4 : 8;  // x quads per lane, row block and super-block
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, n = lane & 15;
@@ -1461,7 +1211,17 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
     // column group are neighbours, so they share an XCD's L2 for the scales).
     const int v = xcd_swizzle(blockIdx.x, nblk, pk & 255);
     const int split = SPLIT ? (v & ((1 << slog) - 1)) : 0;
-    const int cgrp = SPLIT ? (v >> slog) : v;
+    const int vg = SPLIT ? (v >> slog) : v;
+    const int wt = MULTI ? a.wgd.div(vg) : 0;  // weight of the side-by-side set
+    const int cgrp = MULTI ? vg - wt * a.wgpw : vg;
+    const uint4* Wq[NG];
+    const float* SCq[NG];
+#pragma unroll
+    for (int q = 0; q < NG; ++q) {
+        const int wi = NG == 1 ? wt : q;
+        Wq[q] = (MULTI || q > 0) ? a.W[wi] : hW0;
+        SCq[q] = (MULTI || q > 0) ? a.SC[wi] : hS0;
+    }
     const int blk0 = cgrp * C;  // first column block
     const int sc = fastdiv_of(wpcm, (pk >> 8) & 255).div(cgrp);
     const int nsb = (Kpad + kSkinnySB - 1) / kSkinnySB;
@@ -1479,7 +1239,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
     float4 sreg[NG][SCI];
 #pragma unroll
     for (int q = 0; q < NG; ++q) {
-        const __amdgpu_buffer_rsrc_t rS = make_rsrc((q == 0 ? hS0 : a.SC[q]) + (int64_t)sc * Kpad, (uint32_t)Kpad * 4u);
+        const __amdgpu_buffer_rsrc_t rS = make_rsrc(SCq[q] + (int64_t)sc * Kpad, (uint32_t)Kpad * 4u);
 #pragma unroll
         for (int it = 0; it < SCI; ++it) {
             const int r4 = threadIdx.x + it * NW * 64;
@@ -1490,7 +1250,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
     __amdgpu_buffer_rsrc_t rW[NG];
 #pragma unroll
     for (int q = 0; q < NG; ++q)
-        rW[q] = make_rsrc((q == 0 ? hW0 : a.W[q]) + ((int64_t)ko + (int64_t)blk0 * nkb) * 16,
+        rW[q] = make_rsrc(Wq[q] + ((int64_t)ko + (int64_t)blk0 * nkb) * 16,
                           (uint32_t)C * (uint32_t)nkb * 256u);
     const __amdgpu_buffer_rsrc_t rX = make_rsrc(hx, (uint32_t)hM * (uint32_t)K * 4u);
     int wv[C];
@@ -1655,9 +1415,10 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
                     // h + m + l turns an infinite x * s into inf - inf: recompute
                     // a non-finite total as the reference's k-order sum.
                     if (!isfinite(s))
-                        s = i4_column_exact<false>(a.W[q], a.SC[q], strip, el, a.spc, a.Kpad, a.RQ,
+                        s = i4_column_exact<false>(Wq[q], SCq[q], strip, el, a.spc, a.Kpad, a.RQ,
                                                    a.x + (int64_t)m * K, nullptr, klo, khi);
-                    if (!SPLIT && a.bias[q]) s = s + a.bias[q][col];
+                    const float* bq = a.bias[NG == 1 ? wt : q];
+                    if (!SPLIT && bq) s = s + bq[col];
                 }
                 o[q][b][i] = s;
             }
@@ -1670,14 +1431,16 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
             const int c = t >> 8, m = ((t >> 4) & 15) + 16 * b, sl = t & 15;
             const int col = 16 * (blk0 + c) + sl;
             if (t < 256 * C && m < a.M && col < a.N) {
-                const int64_t at = (int64_t)m * a.N + col;
                 if constexpr (SPLIT) {
-                    const int64_t MN = (int64_t)a.M * a.N;
+                    const int64_t MN = (int64_t)a.M * a.N, at = (int64_t)m * a.N + col;
 #pragma unroll
-                    for (int q = 0; q < NG; ++q) a.part[((int64_t)q << a.slog | split) * MN + at] = o[q][b][i];
+                    for (int q = 0; q < NG; ++q)
+                        a.part[((int64_t)(NG == 1 ? wt : q) << a.slog | split) * MN + at] = o[q][b][i];
                 } else {
+                    const int64_t at = (int64_t)m * a.ldy + (int64_t)wt * a.N + col;
                     float r0 = o[0][b][i];
                     if constexpr (NG == 2) r0 = silu_f32(o[0][b][i]) * o[1][b][i];
+                    if (a.res) r0 = r0 + a.res[at];
                     a.y[at] = r0;
                 }
             }
@@ -1876,32 +1639,44 @@ __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ h
 }
 
 // The skinny kernel's K ranges added in range order, plus the bias; NG == 2:
-// h = silu(gate + bias) * (up + bias2).  part is [NG][S][M*N].
+// h = silu(gate + bias) * (up + bias2).  part is [NG][S][M*N].  NG == 1 sums
+// blockIdx.y of nw weights side by side (rows of ldy floats) and adds res
+// where it is set (same indexing as y, which it may be).
+// The leading scalar arguments are preloaded into SGPRs.
+struct SkinnyReduceArgs {
+    const float* bias[3];
+    const float* res;
+    int ldy;
+};
 template <int NG>
-__global__ __launch_bounds__(kThreads) void k_skinny_reduce(const float* __restrict__ part, int S, int64_t MN, int N,
-                                                            const float* __restrict__ bias,
-                                                            const float* __restrict__ bias2, float* __restrict__ y) {
-    for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < MN; o += (int64_t)gridDim.x * blockDim.x) {
-        float r[NG];
+__global__ __launch_bounds__(kThreads) void k_skinny_reduce(const float* __restrict__ part, float* y, int MN, int S, int N,
+                                                            const SkinnyReduceArgs a) {
+    const int wt = NG == 1 ? (int)blockIdx.y : 0;
+    const int o = blockIdx.x * kThreads + threadIdx.x;  // M <= 32 rows: 32-bit indices
+    if (o >= MN) return;
+    float r[NG];
+    int m = 0, n = o;
 #pragma unroll
-        for (int q = 0; q < NG; ++q) {
-            float t[kSkinnyMaxSplits];
+    for (int q = 0; q < NG; ++q) {
+        const float* pq = part + (int64_t)(NG == 1 ? wt : q) * S * MN + o;
+        float t[kSkinnyMaxSplits];
 #pragma unroll
-            for (int sp = 0; sp < kSkinnyMaxSplits; ++sp)  // all loads first
-                t[sp] = sp < S ? part[((int64_t)q * S + sp) * MN + o] : 0.0f;
-            float v = 0.0f;
+        for (int sp = 0; sp < kSkinnyMaxSplits; ++sp)  // all loads first
+            t[sp] = sp < S ? pq[(int64_t)sp * MN] : 0.0f;
+        float v = 0.0f;
 #pragma unroll
-            for (int sp = 0; sp < kSkinnyMaxSplits; ++sp)
-                if (sp < S) v += t[sp];
-            const float* bq = q == 0 ? bias : bias2;
-            if (bq) v = v + bq[o % N];
-            r[q] = v;
-        }
-        if constexpr (NG == 2)
-            y[o] = silu_f32(r[0]) * r[1];
-        else
-            y[o] = r[0];
+        for (int sp = 0; sp < kSkinnyMaxSplits; ++sp)
+            if (sp < S) v += t[sp];
+        const float* bq = a.bias[NG == 1 ? wt : q];
+        if (q == 0 && (bq || a.bias[1] || a.ldy != N)) m = (unsigned)o / (unsigned)N, n = o - m * N;
+        if (bq) v = v + bq[n];
+        r[q] = v;
     }
+    const int64_t at = (int64_t)m * a.ldy + (int64_t)wt * N + n;
+    float v = r[0];
+    if constexpr (NG == 2) v = silu_f32(r[0]) * r[1];
+    if (a.res) v = v + a.res[at];
+    y[at] = v;
 }
 
 // h[i] = silu(h[i]) * u[i]: the gated MLP's elementwise tail after two
@@ -1909,23 +1684,6 @@ __global__ __launch_bounds__(kThreads) void k_skinny_reduce(const float* __restr
 __global__ __launch_bounds__(kThreads) void k_silu_mul(float* __restrict__ h, const float* __restrict__ u, int64_t n) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         h[i] = silu_f32(h[i]) * u[i];
-}
-
-// y[m][n] = sum over splits s = 0..KS-1, in that order, of part[s][m][n] (+ bias[n]).
-constexpr int kMaxSplits = 16;
-__global__ __launch_bounds__(kThreads) void k_splitk_reduce(const float* __restrict__ part, int KS, int64_t MN, int N,
-                                                            const float* __restrict__ bias, float* __restrict__ y) {
-    for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < MN; o += (int64_t)gridDim.x * blockDim.x) {
-        float t[kMaxSplits];
-#pragma unroll
-        for (int sp = 0; sp < kMaxSplits; ++sp) t[sp] = sp < KS ? part[sp * MN + o] : 0.0f;  // all loads first
-        float r = 0.0f;
-#pragma unroll
-        for (int sp = 0; sp < kMaxSplits; ++sp)
-            if (sp < KS) r += t[sp];
-        if (bias) r = r + bias[o % N];
-        y[o] = r;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2144,13 +1902,13 @@ template <int C, int NG, int MB, bool XA>
 hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const void* const* packed,
                          const float* const* devscales, const float* const* bias, const I4Geom& g, int form, int S,
                          float* y, float* part, const SkinnyExtra& ex, hipStream_t s) {
-    if (form == 0 && S != 1) return hipErrorInvalidValue;
-    // Side-by-side weights, a row stride and the folded RMSNorm: whole-K form only.
-    const bool plain = ex.nw == 1 && ex.ldy == N && !ex.gamma;
-    if ((!plain && form != 0) || ex.nw < 1 || ex.nw > 3 || (NG == 2 && ex.nw != 1)) return hipErrorInvalidValue;
-    // Side-by-side weights come with the norm (the LLaMA block's q, k and v):
-    // the plain kernels take their one weight from the preloaded arguments.
-    if (ex.nw != 1 && !ex.gamma) return hipErrorInvalidValue;
+    if (form == 0 && (S != 1 || ex.res)) return hipErrorInvalidValue;
+    // The folded RMSNorm: whole-K form only, where side-by-side weights come
+    // with it (the plain kernels take their one weight from the preloaded
+    // arguments); the super-block form runs them side by side without it.
+    if ((ex.gamma && form != 0) || ex.nw < 1 || ex.nw > 3 || (NG == 2 && ex.nw != 1)) return hipErrorInvalidValue;
+    if (form == 0 && ex.nw != 1 && !ex.gamma) return hipErrorInvalidValue;
+    if (form == 0 && ex.ldy != N && !ex.gamma) return hipErrorInvalidValue;
     if (g.Kpad != 4 * g.RQ) return hipErrorInvalidValue;  // SkinnyHot carries RQ only
     SkinnyArgs a{};
     a.x = x;
@@ -2166,6 +1924,7 @@ hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const 
     a.ldy = (int)ex.ldy;
     a.wgpw = (int)(g.NS / (2 * C));
     a.wgd = FastDiv((uint32_t)a.wgpw);
+    a.res = ex.res;
     a.gamma = ex.gamma;
     a.eps = ex.eps;
     a.spc = (int)g.spc;
@@ -2207,23 +1966,42 @@ hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const 
         return hipErrorInvalidValue;
     }
     const bool half = MB == 1 && M <= 8;
+    a.nblk *= ex.nw;
     const SkinnyHot h = skinny_hot(a);
-    if (S > 1 && half)
-        k_skinny_sb<kSkinnyWaves, C, NG, XA, MB, true, MB == 1><<<a.nblk, kSkinnyWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a);
-    else if (S > 1)
-        k_skinny_sb<kSkinnyWaves, C, NG, XA, MB, true, false><<<a.nblk, kSkinnyWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a);
-    else if (half)
-        k_skinny_sb<kSkinnyWaves, C, NG, XA, MB, false, MB == 1><<<a.nblk, kSkinnyWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a);
-    else
-        k_skinny_sb<kSkinnyWaves, C, NG, XA, MB, false, false><<<a.nblk, kSkinnyWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a);
+#define SGQ_SKINNY_SB(SPLIT_, HALF_, MULTI_)                                                            \
+    k_skinny_sb<kSkinnyWaves, C, NG, XA, MB, SPLIT_, HALF_, MULTI_>                                     \
+        <<<a.nblk, kSkinnyWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a)
+    if (ex.nw > 1) {
+        // Several weights: the LLaMA block's q, k and v of 17..32 sequences
+        // (their normed input is the library's own, 16-byte aligned).
+        if constexpr (NG == 1 && MB == 2 && XA) {
+            if (S > 1)
+                SGQ_SKINNY_SB(true, false, true);
+            else
+                SGQ_SKINNY_SB(false, false, true);
+        } else {
+            return hipErrorInvalidValue;
+        }
+    } else if (S > 1 && half) {
+        SGQ_SKINNY_SB(true, MB == 1, false);
+    } else if (S > 1) {
+        SGQ_SKINNY_SB(true, false, false);
+    } else if (half) {
+        SGQ_SKINNY_SB(false, MB == 1, false);
+    } else {
+        SGQ_SKINNY_SB(false, false, false);
+    }
+#undef SGQ_SKINNY_SB
     if (S > 1) {
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        const int64_t MN = M * N;
-        int64_t blocks = ceil_div(MN, kThreads);
-        if (blocks > 4096) blocks = 4096;
-        k_skinny_reduce<NG><<<(unsigned)blocks, kThreads, 0, s>>>(part, S, MN, (int)N, bias[0],
-                                                                  NG == 2 ? bias[1] : nullptr, y);
+        if (M * N >= (int64_t)1 << 31) return hipErrorInvalidValue;
+        SkinnyReduceArgs ra{};
+        for (int q = 0; q < nq; ++q) ra.bias[q] = bias[q];
+        ra.res = ex.res;
+        ra.ldy = (int)ex.ldy;
+        k_skinny_reduce<NG><<<dim3((unsigned)ceil_div(M * N, kThreads), (unsigned)ex.nw), kThreads, 0, s>>>(
+            part, y, (int)(M * N), S, (int)N, ra);
     }
     return hipGetLastError();
 }
@@ -2503,15 +2281,12 @@ int64_t gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     return ks > 1 ? ks * M * N * 4 : 0;
 }
 
-// Which GEMM kernel a shape takes and its tile: the three-term bf16 kernel
-// folds the scale into A, so a tile's columns must share their scale (always
-// for INT8's 256-column tiles; for INT4 when a scale column spans a multiple
-// of 16 strips, i.e. a group that is a multiple of 128).
-static bool gemm_three_term(int bits, int mode) { return bits == 8 || mode % 16 == 0; }
+// The tile an INT4 GEMM plans its K splits by: 128 x 128 for groups that are
+// not a multiple of 128, whatever the batch.
+static GemmTile gemm_i4_tile(int64_t M, int mode) { return mode % 16 == 0 ? gemm_tile(4, M) : GemmTile{kBM, kBN, 2}; }
 
 int64_t gemm_launch_ws_bytes(int bits, int64_t M, int64_t K, int64_t N, int mode, int64_t cus) {
-    const bool three = gemm_three_term(bits, mode);
-    const GemmPlan p = gemm_plan(M, K, N, three ? gemm_tile(bits, M) : GemmTile{kBM, kBN, 2}, cus);
+    const GemmPlan p = gemm_plan(M, K, N, bits == 8 ? gemm_tile(8, M) : gemm_i4_tile(M, mode), cus);
     return p.KS > 1 ? (int64_t)p.KS * M * N * 4 : 0;
 }
 
@@ -2537,9 +2312,8 @@ void linear_plan(int bits, int64_t M, int64_t K, int64_t N, int64_t group_size, 
         return;
     }
     const int mode = bits == 4 ? (int)I4Geom(K, N, group_size).spc : 0;
-    const bool three = gemm_three_term(bits, mode);
-    *path = three ? 1 : 2;
-    *ks = gemm_plan(M, K, N, three ? gemm_tile(bits, M) : GemmTile{kBM, kBN, 2}, cus).KS;
+    *path = mode % 16 == 0 ? 1 : 2;
+    *ks = gemm_plan(M, K, N, bits == 8 ? gemm_tile(8, M) : gemm_i4_tile(M, mode), cus).KS;
 }
 
 // Tile rows per XCD rectangle for a grid of tm x tn tiles without a K split
@@ -2548,7 +2322,7 @@ void linear_plan(int bits, int64_t M, int64_t K, int64_t N, int64_t group_size, 
 // blocks of x (xb bytes each) and per / a column blocks of codes (wb bytes
 // each); 0 when the grid does not tile into xcds such rectangles (the plain
 // XCD order then).
-int xcd_rect_rows_impl(int64_t tm, int64_t tn, int64_t xb, int64_t wb, int64_t xcds) {
+int xcd_rect_rows(int64_t tm, int64_t tn, int64_t xb, int64_t wb, int64_t xcds) {
     const int64_t T = tm * tn;
     if (xcds < 1 || T % xcds != 0) return 0;
     const int64_t per = T / xcds;
@@ -2563,83 +2337,91 @@ int xcd_rect_rows_impl(int64_t tm, int64_t tn, int64_t xb, int64_t wb, int64_t x
 }
 
 int gemm_rect_rows(int bits, int64_t M, int64_t K, int64_t N, int mode, int64_t cus, int64_t xcds) {
-    const bool three = gemm_three_term(bits, mode);
-    const GemmTile t = three ? gemm_tile(bits, M) : GemmTile{kBM, kBN, 2};
-    if (!three || gemm_plan(M, K, N, t, cus).KS != 1) return 0;
-    return xcd_rect_rows_impl(ceil_div(M, t.bm), ceil_div(N, t.bn), t.bm * K * 4, t.bn * K * bits / 8, xcds);
+    const GemmTile t = bits == 8 ? gemm_tile(8, M) : gemm_i4_tile(M, mode);
+    if (gemm_plan(M, K, N, t, cus).KS != 1) return 0;
+    int64_t bm = t.bm, bn = t.bn;
+    if (bits == 4) {
+        if (!gemm_wave_takes(mode)) return 0;  // the fp32 kernel keeps the plain order
+        const GemmWaveShape w = gemm_wave_shape(M, N, mode, 1, cus);
+        bm = w.rows(), bn = w.cols();
+    }
+    return xcd_rect_rows(ceil_div(M, bm), ceil_div(N, bn), bm * K * 4, bn * K * bits / 8, xcds);
 }
 
 namespace {
 
-template <int BITS>
-hipError_t gemm_launch(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* sc, int mode,
-                       int64_t Kpad, int64_t RQ, int64_t NS, const float* bias, float* y, void* ws, hipStream_t s) {
-    // INT4 groups that are not a multiple of 128 take the fp32-MFMA kernel.
-    const bool three = gemm_three_term(BITS, mode);
-    const GemmTile t = three ? gemm_tile(BITS, M) : GemmTile{kBM, kBN, 2};
-    const GemmPlan p = gemm_plan(M, K, N, t, device_cus(s));
-    float* part = p.KS > 1 ? (float*)ws : nullptr;
-    const dim3 grid((unsigned)(ceil_div(M, t.bm) * ceil_div(N, t.bn) * p.KS));
-    const int xcds = device_xcds(s);
-    const int xr = p.KS == 1 ? xcd_rect_rows_impl(ceil_div(M, t.bm), ceil_div(N, t.bn), t.bm * K * 4,
-                                                  t.bn * K * BITS / 8, xcds)
-                             : 0;
-    const int xlog = xcd_log2(xcds);
-    const bool k4 = x_aligned4(x, K);
-    const bool pt = BITS == 8 && mode;
-    // INT4: the k-octet copy follows the strips at their bytes rounded up to
-    // 256 (I4Geom::koct_off).
-    const int ko = BITS == 4 ? (int)ceil_div(NS * RQ * 16, 256) : 0;
-    using Big = typename std::conditional<BITS == 8, G3Wide, G3Tile>::type;
-#define SGQ_GEMM3(SH, A4, PT_)                                                                                 \
-    k_gemm3<BITS, A4, (PT_) && BITS == 8, SH><<<grid, SH::NT, 0, s>>>(Gemm3Args{                                \
-        x, (int)M, (int)K, (int)N, (const uint4*)packed, sc, mode, (int)Kpad, (int)RQ, (int)NS, p.KS, p.sps, bias, \
-        y, part, xr, xlog, ko})
-#define SGQ_GEMM3_SHAPE(SH)               \
-    if (k4 && pt)                         \
-        SGQ_GEMM3(SH, true, true);        \
-    else if (k4)                          \
-        SGQ_GEMM3(SH, true, false);       \
-    else if (pt)                          \
-        SGQ_GEMM3(SH, false, true);       \
-    else                                  \
-        SGQ_GEMM3(SH, false, false);
-    if (three && t.bm == 32) {
-        SGQ_GEMM3_SHAPE(G3Rows32)
-    } else if (three && t.bm == 64) {
-        SGQ_GEMM3_SHAPE(G3Rows64)
-    } else if (three) {
-        SGQ_GEMM3_SHAPE(Big)
-    } else if (k4)
-        k_gemm<BITS, true><<<grid, kThreads, 0, s>>>(x, (int)M, (int)K, (int)N, (const uint4*)packed, sc, mode,
-                                                     (int)Kpad, (int)RQ, (int)NS, p.KS, p.sps, bias, y, part);
+// The three-term INT8 GEMM (k_gemm3) on the tile gemm_tile gives the batch.
+template <class SH>
+void gemm3_launch(const Gemm3Args& a, unsigned grid, bool k4, bool pt, hipStream_t s) {
+    if (k4 && pt)
+        k_gemm3<true, true, SH><<<grid, SH::NT, 0, s>>>(a);
+    else if (k4)
+        k_gemm3<true, false, SH><<<grid, SH::NT, 0, s>>>(a);
+    else if (pt)
+        k_gemm3<false, true, SH><<<grid, SH::NT, 0, s>>>(a);
     else
-        k_gemm<BITS, false><<<grid, kThreads, 0, s>>>(x, (int)M, (int)K, (int)N, (const uint4*)packed, sc, mode,
-                                                      (int)Kpad, (int)RQ, (int)NS, p.KS, p.sps, bias, y, part);
-#undef SGQ_GEMM3_SHAPE
-#undef SGQ_GEMM3
-    if (p.KS > 1) {
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        const int64_t MN = M * N;
-        int64_t blocks = ceil_div(MN, kThreads);
-        if (blocks > 4096) blocks = 4096;
-        k_splitk_reduce<<<(unsigned)blocks, kThreads, 0, s>>>(part, p.KS, MN, (int)N, bias, y);
-    }
-    return hipGetLastError();
+        k_gemm3<false, false, SH><<<grid, SH::NT, 0, s>>>(a);
 }
 }  // namespace
 
 hipError_t launch_gemm_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* scales,
                           bool per_tensor, const float* bias, float* y, void* ws, hipStream_t s) {
-    I8Geom g(K, N);
-    return gemm_launch<8>(x, M, K, N, packed, scales, per_tensor ? 1 : 0, g.Kpad, g.RQ, g.NS, bias, y, ws, s);
+    const I8Geom g(K, N);
+    const GemmTile t = gemm_tile(8, M);
+    const GemmPlan p = gemm_plan(M, K, N, t, device_cus(s));
+    const int64_t tm = ceil_div(M, t.bm), tn = ceil_div(N, t.bn);
+    const int xcds = device_xcds(s);
+    Gemm3Args a{};
+    a.x = x;
+    a.M = (int)M, a.K = (int)K, a.N = (int)N;
+    a.W = (const uint4*)packed;
+    a.S = scales;
+    a.Kpad = (int)g.Kpad, a.RQ = (int)g.RQ, a.NS = (int)g.NS;
+    a.KS = p.KS, a.sps = p.sps;
+    a.bias = bias;
+    a.y = y;
+    a.part = p.KS > 1 ? (float*)ws : nullptr;
+    a.xr = p.KS == 1 ? xcd_rect_rows(tm, tn, t.bm * K * 4, t.bn * K, xcds) : 0;
+    a.xlog = xcd_log2(xcds);
+    const unsigned grid = (unsigned)(tm * tn * p.KS);
+    const bool k4 = x_aligned4(x, K);
+    if (t.bm == 32)
+        gemm3_launch<G3Rows32>(a, grid, k4, per_tensor, s);
+    else if (t.bm == 64)
+        gemm3_launch<G3Rows64>(a, grid, k4, per_tensor, s);
+    else
+        gemm3_launch<G3Wide>(a, grid, k4, per_tensor, s);
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess || p.KS == 1 ? e : launch_splitk_reduce(a.part, p.KS, M, N, 1, &bias, {}, y, s);
 }
 
-hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, const void* packed,
-                          const float* devscales, const I4Geom& g, const float* bias, float* y, void* ws,
-                          hipStream_t s) {
-    return gemm_launch<4>(x, M, K, N, packed, devscales, (int)g.spc, g.Kpad, g.RQ, g.NS, bias, y, ws, s);
+hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
+                          const float* const* devscales, const float* const* bias, const I4Geom& g,
+                          const GemmEpilogue& ep, float* y, void* ws, hipStream_t s) {
+    const int64_t cus = device_cus(s);
+    // Several weights side by side plan their splits as one of the total width.
+    const GemmPlan p = gemm_plan(M, K, nw * N, gemm_i4_tile(M, (int)g.spc), cus);
+    hipError_t e = hipSuccess;
+    if (gemm_wave_takes((int)g.spc)) {
+        e = launch_gemm_wave(x, M, K, N, nw, packed, devscales, bias, g, p,
+                             gemm_wave_shape(M, nw * N, (int)g.spc, p.KS, cus), ep, y, ws, s);
+    } else {
+        const unsigned grid = (unsigned)(ceil_div(M, kBM) * ceil_div(N, kBN) * p.KS);
+        for (int w = 0; w < nw && e == hipSuccess; ++w) {
+            float* part = p.KS > 1 ? (float*)ws + (int64_t)w * p.KS * M * N : nullptr;
+            float* yw = y + (int64_t)w * M * N;
+            if (x_aligned4(x, K))
+                k_gemm<true><<<grid, kThreads, 0, s>>>(x, (int)M, (int)K, (int)N, (const uint4*)packed[w], devscales[w],
+                                                       (int)g.spc, (int)g.Kpad, (int)g.RQ, (int)g.NS, p.KS, p.sps,
+                                                       bias[w], ep, yw, part);
+            else
+                k_gemm<false><<<grid, kThreads, 0, s>>>(x, (int)M, (int)K, (int)N, (const uint4*)packed[w],
+                                                        devscales[w], (int)g.spc, (int)g.Kpad, (int)g.RQ, (int)g.NS,
+                                                        p.KS, p.sps, bias[w], ep, yw, part);
+            e = hipGetLastError();
+        }
+    }
+    return e != hipSuccess || p.KS == 1 ? e : launch_splitk_reduce((const float*)ws, p.KS, M, N, nw, bias, ep, y, s);
 }
 
 hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N, const void* packed,

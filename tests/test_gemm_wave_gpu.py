@@ -1,0 +1,82 @@
+"""The INT4 GEMM of independent wavefront tiles (scale columns of a multiple of
+four strips) at the edges of its tiles: rows around 32 and 64, column blocks
+past the weight, scale groups of 32 to 128 columns, K shorter than its K ranges,
+with a partial stage, odd (rows of x at any 4-byte address), with and without a
+K split over workgroups.
+
+The oracle is x . dequantize(W) in 64 bits.  Each output is bounded on its own:
+an accumulator takes three MFMA additions per 32 k, each of which may round or
+truncate (2^-23 of at most sum |x w|), the K ranges, splits, product and
+epilogue add a few more roundings.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(y, x, w, b, K, splits=16 + 4):
+    x, w = x.double(), w.double()
+    ref, mag = x @ w, x.abs() @ w.abs()
+    if b is not None:
+        ref, mag = ref + b.double(), mag + b.double().abs()
+    bound = (3 * -(-K // 32) + splits + 4) * 2.0**-23 * mag
+    bad = ((y.double() - ref).abs() > bound).sum()
+    assert int(bad) == 0, (int(bad), float(((y.double() - ref).abs() / bound).max()))
+
+
+def _inputs(sgq, dev, M, K, N, G, seed, offset=0):
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(seed)
+    w = torch.randn(K, N, generator=gen, device=dev) * 0.02
+    flat = torch.randn(M * K + offset, generator=gen, device=dev)
+    b = torch.randn(1, N, generator=gen, device=dev)
+    return flat[offset:].reshape(M, K), sgq.quantize_int4(w, G, keep_qdata=False), b
+
+
+@pytest.mark.parametrize("G,N", [(32, 32), (32, 160), (64, 64), (64, 320), (96, 288), (128, 128), (128, 384)])
+@pytest.mark.parametrize("M,K", [(129, 16), (160, 33), (191, 64), (193, 95), (256, 1000), (130, 2049)])
+def test_tile_edges(sgq, dev, M, K, G, N):
+    for offset in (0, 1):  # x at a 16-byte and at a 4-byte address
+        x, qw, b = _inputs(sgq, dev, M, K, N, G, M + K + N, offset)
+        _check(sgq.quantized_matmul_int4(x, qw, b), x, sgq.dequantize_int4(qw), b, K)
+        _check(sgq.quantized_matmul_int4(x, qw), x, sgq.dequantize_int4(qw), None, K)
+
+
+@pytest.mark.parametrize("M,K,N,G", [(2048, 160, 4096, 128), (2049, 97, 4224, 128), (40, 4096, 4096, 32),
+                                     (1025, 512, 5632, 64), (33, 8200, 1152, 128)])
+def test_large_grids(sgq, dev, M, K, N, G):
+    """Four row blocks per wavefront, grids without a K split, small batches over long K."""
+    x, qw, b = _inputs(sgq, dev, M, K, N, G, 5)
+    _check(sgq.quantized_matmul_int4(x, qw, b), x, sgq.dequantize_int4(qw), b, K)
+
+
+@pytest.mark.parametrize("G", [32, 64, 128])
+def test_non_finite_inputs(sgq, dev, G):
+    """Infinities and NaNs land where x . (q * s) puts them."""
+    M, K, N = 140, 300, 256
+    x, qw, _ = _inputs(sgq, dev, M, K, N, G, 7)
+    x[3, 17], x[70, 290], x[139, 0] = float("inf"), float("nan"), -float("inf")
+    y, ref = sgq.quantized_matmul_int4(x, qw).double(), x.double() @ sgq.dequantize_int4(qw).double()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    assert torch.equal(torch.isinf(y), torch.isinf(ref))
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.sign(y[~fin & ~torch.isnan(ref)]), torch.sign(ref[~fin & ~torch.isnan(ref)]))
+
+
+@pytest.mark.parametrize("bits,G", [(4, 128), (4, 32), (4, 24), (8, 0), (8, 1)])
+@pytest.mark.parametrize("M,K,N", [(130, 256, 384), (300, 2048, 768)])
+def test_gated_epilogue(sgq, dev, M, K, N, bits, G):
+    """The gated MLP of GEMM batches: the up projection's epilogue multiplies
+    by silu of the gate projection, the same values as the two forwards and an
+    elementwise product (expf and the division are a few ulp from torch's)."""
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(9)
+    w = [torch.randn(K, N, generator=gen, device=dev) * 0.02 for _ in range(2)]
+    b = [torch.randn(1, N, generator=gen, device=dev) for _ in range(2)]
+    x = torch.randn(M, K, generator=gen, device=dev)
+    q = [sgq.quantize_int8(v, G) if bits == 8 else sgq.quantize_int4(v, G) for v in w]
+    gate, up = (sgq.quantized_matmul(x, q[i], b[i]).double() for i in range(2))
+    h = sgq.quantized_swiglu(x, q[0], q[1], b[0], b[1])
+    ref = gate / (1 + torch.exp(-gate)) * up
+    assert float(((h.double() - ref).abs() / ref.abs().clamp_min(1e-30)).max()) < 16 * 2.0**-24
