@@ -1686,29 +1686,6 @@ __global__ __launch_bounds__(kThreads) void k_silu_mul(float* __restrict__ h, co
         h[i] = silu_f32(h[i]) * u[i];
 }
 
-// ---------------------------------------------------------------------------
-// Generic INT4 forward over the flat layout (shapes the strip layout cannot
-// hold).  One thread per output; per-element scale index, the reference's own
-// product code*scale, FMA accumulation in k order.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void k_linear_i4_flat(const float* __restrict__ x, int64_t M, int64_t K,
-                                                             int64_t N, const unsigned char* __restrict__ P,
-                                                             const float* __restrict__ S, int64_t G,
-                                                             const float* __restrict__ bias, float* __restrict__ y) {
-    for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < M * N;
-         o += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t m = o / N, n = o - m * N;
-        float acc = 0.0f;
-        for (int64_t k = 0; k < K; ++k) {
-            const int64_t i = k * N + n;
-            const uint32_t byte = P[i >> 1];
-            const float q = (float)(((int)(byte << (28 - 4 * (int)(i & 1)))) >> 28);
-            acc = fmaf(x[m * K + k], q * S[i / G], acc);
-        }
-        y[o] = bias ? acc + bias[n] : acc;
-    }
-}
-
 bool x_aligned4(const float* x, int64_t K) { return K % 4 == 0 && (((uintptr_t)x) & 15) == 0; }
 
 #define SGQ_GEMV_HOT_ARGS(h, ag) h.x, h.W0, h.S0, h.K, h.RQ, h.NS, h.M, h.nblk, h.pk, h.spcm, ag
@@ -2422,16 +2399,6 @@ hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, int n
         }
     }
     return e != hipSuccess || p.KS == 1 ? e : launch_splitk_reduce((const float*)ws, p.KS, M, N, nw, bias, ep, y, s);
-}
-
-hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N, const void* packed,
-                                 const float* scales, int64_t G, const float* bias, float* y, hipStream_t s) {
-    int64_t blocks = ceil_div(M * N, kThreads);
-    if (blocks > 65536) blocks = 65536;
-    if (blocks < 1) blocks = 1;
-    k_linear_i4_flat<<<(unsigned)blocks, kThreads, 0, s>>>(x, M, K, N, (const unsigned char*)packed, scales, G,
-                                                            bias, y);
-    return hipGetLastError();
 }
 
 }  // namespace sgq
