@@ -454,10 +454,15 @@ int sgq_quantize_int4(const float* x, int64_t rows, int64_t cols, int64_t group_
     if (!workspace || workspace_bytes < w.total)
         return fail(SGQ_ERR_WORKSPACE, "sgq_quantize_int4: workspace needs %lld bytes", (long long)w.total);
     float* inv = (float*)((char*)workspace + w.inv_off);
+    if (total > 0 && packed && pack_i4_finds_scales(g)) {  // one pass over x
+        SGQ_HIP(launch_pack_i4_tiled(x, false, rows, cols, g.G, nullptr, packed, scales, devscales, qdata_f32, nullptr, s),
+                "pack_i4_tiled");
+        return ok();
+    }
     if (ngroups > 0) SGQ_HIP(launch_group_scales(x, total, g.G, ngroups, 7.0f, scales, inv, s), "group_scales");
     if (total > 0) {
         if (packed && g.tiled) {
-            SGQ_HIP(launch_pack_i4_tiled(x, false, rows, cols, g.G, inv, packed, qdata_f32, nullptr, s),
+            SGQ_HIP(launch_pack_i4_tiled(x, false, rows, cols, g.G, inv, packed, nullptr, nullptr, qdata_f32, nullptr, s),
                     "pack_i4_tiled");
             SGQ_HIP(launch_devscales_i4(scales, g, devscales, s), "devscales_i4");
         } else if (packed || qdata_f32) {
@@ -499,7 +504,7 @@ int sgq_pack_int4(const float* qdata_f32, const float* scales, int64_t K, int64_
     int* flag = (int*)((char*)workspace + w.bad_off);
     SGQ_HIP(launch_fill_zero(flag, sizeof(int), s), "fill_zero");
     if (g.tiled) {
-        SGQ_HIP(launch_pack_i4_tiled(qdata_f32, true, K, N, g.G, nullptr, packed, nullptr, flag, s), "pack_i4_tiled");
+        SGQ_HIP(launch_pack_i4_tiled(qdata_f32, true, K, N, g.G, nullptr, packed, nullptr, nullptr, nullptr, flag, s), "pack_i4_tiled");
         SGQ_HIP(launch_devscales_i4(scales, g, devscales, s), "devscales_i4");
     } else {
         SGQ_HIP(launch_pack_i4_flat(qdata_f32, true, K * N, g.G, nullptr, packed, nullptr, flag, s), "pack_i4_flat");

@@ -283,12 +283,15 @@ int64_t absmax_partial_count(int64_t total);
 hipError_t launch_absmax_partial(const float* x, int64_t total, float* partial, int64_t nparts, hipStream_t s);
 
 // Pack kernels.  from_codes == false: src is x and codes are computed with inv;
-// from_codes == true: src holds fp32 codes, validated into *bad.  packed and
-// qdata may each be null (that output is skipped).
+// from_codes == true: src holds fp32 codes, validated into *bad.  packed (INT8,
+// INT4 flat) and qdata may be null (that output is skipped).  INT4 tiled with
+// inv == nullptr (where pack_i4_finds_scales says so) finds the scales in the
+// same pass and writes them to scales and devscales.
 hipError_t launch_pack_i8_tiled(const float* src, bool from_codes, int64_t K, int64_t N, const float* inv,
                                 bool per_tensor, void* packed, float* qdata, int* bad, hipStream_t s);
-hipError_t launch_pack_i4_tiled(const float* src, bool from_codes, int64_t K, int64_t N, int64_t G,
-                                const float* inv, void* packed, float* qdata, int* bad, hipStream_t s);
+bool pack_i4_finds_scales(const I4Geom& g);
+hipError_t launch_pack_i4_tiled(const float* src, bool from_codes, int64_t K, int64_t N, int64_t G, const float* inv,
+                                void* packed, float* scales, float* devscales, float* qdata, int* bad, hipStream_t s);
 hipError_t launch_pack_i4_flat(const float* src, bool from_codes, int64_t total, int64_t G, const float* inv,
                                void* packed, float* qdata, int* bad, hipStream_t s);
 hipError_t launch_devscales_i4(const float* scales, const I4Geom& g, float* devscales, hipStream_t s);

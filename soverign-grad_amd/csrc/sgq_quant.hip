@@ -18,6 +18,9 @@ namespace {
 
 constexpr int kBlock = 256;
 
+// Four floats at any 4-byte address.
+typedef float float4_u __attribute__((ext_vector_type(4), aligned(4)));
+
 __device__ __forceinline__ float ref_code(float x, float inv, float lo, float hi) {
     float v = roundf(x * inv);
     float m = (v < hi) ? v : hi;  // std::min(hi, v)
@@ -49,18 +52,34 @@ __global__ void k_fill_bias(float* __restrict__ y, int64_t M, int64_t N, const f
     for (; i < M * N; i += stride) y[i] = bias ? bias[i % N] : 0.0f;
 }
 
-// One wavefront per group of G consecutive elements.
+// L lanes per group of G consecutive elements, V elements per load: a wavefront
+// with 128-bit loads for long groups (rows of INT8 per channel), a wavefront
+// for middle ones, eight lanes for groups of up to 128, where most of a
+// wavefront would have nothing to load.
+template <int L, int V>
 __global__ void k_group_scales(const float* __restrict__ x, int64_t total, int64_t G, int64_t ngroups, float qmax,
                                float* __restrict__ scales, float* __restrict__ inv) {
-    const int lane = threadIdx.x & 63;
-    const int64_t wave = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-    const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-    for (int64_t g = wave; g < ngroups; g += nwaves) {
+    const int lane = threadIdx.x % L;
+    const int64_t first = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / L;
+    const int64_t step = ((int64_t)gridDim.x * blockDim.x) / L;
+    for (int64_t g = first; g < ngroups; g += step) {
         const int64_t b = g * G;
         const int64_t e = (b + G < total) ? b + G : total;
         float m = 1e-8f;
-        for (int64_t i = b + lane; i < e; i += 64) m = ref_max(m, fabsf(x[i]));
-        m = wave_max(m);
+        int64_t i = b;
+        if constexpr (V == 4) {
+            const int64_t n4 = (e - b) / 4;
+#pragma unroll 4
+            for (int64_t t = lane; t < n4; t += L) {
+                const float4_u v = *(const float4_u*)(x + b + 4 * t);
+                m = ref_max(ref_max(ref_max(ref_max(m, fabsf(v.x)), fabsf(v.y)), fabsf(v.z)), fabsf(v.w));
+            }
+            i += 4 * n4;
+        }
+#pragma unroll 4
+        for (i += lane; i < e; i += L) m = ref_max(m, fabsf(x[i]));
+#pragma unroll
+        for (int off = L / 2; off > 0; off >>= 1) m = ref_max(m, __shfl_xor(m, off));
         if (lane == 0) {
             scales[g] = m / qmax;
             if (inv) inv[g] = qmax / m;
@@ -83,120 +102,190 @@ __global__ void k_absmax_partial(const float* __restrict__ x, int64_t total, flo
     }
 }
 
-// INT8 strip-major pack: one thread per 16-byte chunk (4 columns x 4 rows).
-__global__ void k_pack_i8_tiled(const float* __restrict__ src, int from_codes, int64_t K, int64_t N, int64_t RQ,
-                                int64_t NS, int64_t nchunks, const float* __restrict__ inv, int per_tensor,
-                                uint4* __restrict__ packed, float* __restrict__ qdata, int* __restrict__ bad) {
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nchunks;
-         c += (int64_t)gridDim.x * blockDim.x) {
-    // Consecutive threads take consecutive strips of the same rows, so the
-    // reads of x (or qdata) are coalesced; each thread writes chunk j*RQ + rq.
-    const int64_t rq = c / NS, j = c - rq * NS;
-    const int64_t k0 = rq * 4;
-    const int64_t n0 = j * 4;
-    uint32_t dw[4];
+// Where a pack kernel's codes come from: x and the groups' scales found in the
+// kernel, x and the inverse scales in inv, or fp32 codes (validated into *bad).
+enum PackFrom { kFromX, kFromXInv, kFromCodes };
+
+// The pack kernels take a tile of 32 rows by 128 columns per workgroup: x and
+// the fp32 codes move in rows (512 contiguous bytes), the packed codes go
+// through LDS so that a strip's rows leave as one 128-byte run (a thread per
+// 16-byte chunk wrote chunks RQ * 16 bytes apart).  HBM bounds them.  Measured
+// on MI355X, a quantize with fp32 codes, before -> now (us): INT4 4096 x 11008
+// g128 373 -> 83 (385 MB, 4.6 TB/s, what a large copy reaches), 4096 x 4096
+// g32 186 -> 32, g24 (scales found first) 208 -> 137; INT8 4096 x 4096 per
+// tensor 141 -> 67, 4096 x 4097 per channel 141 -> 66.
+constexpr int kPackRows = 32, kPackCols = 128;
+
+// INT8 strip-major: chunk (strip, row quad) is 4 columns x 4 rows, dword d
+// column d, byte r row r.
+template <PackFrom FROM>
+__global__ __launch_bounds__(kBlock) void k_pack_i8_tiled(const float* __restrict__ src, int64_t K, int64_t N, int64_t RQ,
+                                                          int64_t NS, int ncol, const float* __restrict__ inv,
+                                                          int per_tensor, uint4* __restrict__ packed,
+                                                          float* __restrict__ qdata, int* __restrict__ bad) {
+    __shared__ __attribute__((aligned(16))) unsigned char col[kPackCols][kPackRows + 4];
+    const int64_t kb = blockIdx.x / ncol, cb = blockIdx.x - kb * ncol;
+    const int64_t k0 = kb * kPackRows, n0 = cb * kPackCols;
+    const int cq = threadIdx.x & 31, r0 = threadIdx.x >> 5;
+    const int64_t n = n0 + 4 * cq;
+    float v[4][4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        const int64_t k = k0 + r0 + 8 * h;
+        const float* p = src + k * N + n;
+        if (k < K && n + 4 <= N) {
+            const float4_u q = *(const float4_u*)p;
+            v[h][0] = q.x, v[h][1] = q.y, v[h][2] = q.z, v[h][3] = q.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[h][e] = k < K && n + e < N ? p[e] : 0.0f;
+        }
+    }
     int badflag = 0;
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        const int64_t n = n0 + d;
-        uint32_t word = 0;
+    for (int h = 0; h < 4; ++h) {
+        const int r = r0 + 8 * h;
+        const int64_t k = k0 + r;
+        const float iv = FROM == kFromXInv && k < K ? (per_tensor ? inv[0] : inv[k]) : 0.0f;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int64_t k = k0 + r;
-            int code = 0;
-            if (k < K && n < N) {
-                float v;
-                if (from_codes) {
-                    v = src[k * N + n];
-                    if (!valid_code(v, -128.0f, 127.0f)) {
-                        badflag = 1;
-                        v = 0.0f;
-                    }
+        for (int e = 0; e < 4; ++e) {
+            float c = 0.0f;
+            if (k < K && n + e < N) {
+                c = v[h][e];
+                if constexpr (FROM == kFromCodes) {
+                    if (!valid_code(c, -128.0f, 127.0f)) badflag = 1, c = 0.0f;
                 } else {
-                    v = ref_code(src[k * N + n], per_tensor ? inv[0] : inv[k], -127.0f, 127.0f);
-                    if (qdata) qdata[k * N + n] = v;
+                    c = ref_code(c, iv, -127.0f, 127.0f);
                 }
-                code = (int)v;
             }
-            word |= ((uint32_t)code & 0xFFu) << (8 * r);
+            v[h][e] = c;
+            col[4 * cq + e][r] = (unsigned char)(int)c;
         }
-        dw[d] = word;
+        if (FROM == kFromXInv && qdata && k < K) {
+            float* q = qdata + k * N + n;
+            if (n + 4 <= N) {
+                *(float4_u*)q = float4_u{v[h][0], v[h][1], v[h][2], v[h][3]};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) q[e] = v[h][e];
+            }
+        }
     }
-    if (packed) packed[j * RQ + rq] = make_uint4(dw[0], dw[1], dw[2], dw[3]);
     if (badflag) atomicOr(bad, 1);
+    if (!packed) return;
+    __syncthreads();
+    // Chunk t % 8 of strip t / 8.
+    const int64_t j = n0 / 4 + (threadIdx.x >> 3), rq = k0 / 4 + (threadIdx.x & 7);
+    if (j < NS && rq < RQ) {
+        uint32_t dw[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+            dw[d] = *(const uint32_t*)&col[4 * (threadIdx.x >> 3) + d][4 * (threadIdx.x & 7)];
+        packed[j * RQ + rq] = make_uint4(dw[0], dw[1], dw[2], dw[3]);
     }
 }
 
-// INT4 strip-major pack: one thread per 16-byte chunk (4 rows x 8 columns).
-__global__ void k_pack_i4_tiled(const float* __restrict__ src, int from_codes, int64_t K, int64_t N, int64_t G,
-                                int64_t RQ, int64_t NS, int64_t nchunks, const float* __restrict__ inv,
-                                uint4* __restrict__ packed, float* __restrict__ qdata, int* __restrict__ bad) {
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nchunks;
-         c += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t rq = c / NS, j = c - rq * NS;
-    const int64_t k0 = rq * 4;
-    const int64_t n0 = j * 8;
-    uint32_t dw[4];
+// INT4 strip-major: the strips, the k-octet copy and (kFromX) the scales in
+// both layouts from one read of x.  A thread takes eight columns of two rows,
+// one strip dword each; a strip's 32 rows are consecutive dwords, and the
+// k-octet dwords are gathered from the tile in LDS: block (cb, kb), dword t is
+// column 16 cb + (t & 15), rows 32 kb + 8 (t >> 4) .. + 7 in nibbles 0..7.
+// kFromX needs whole groups in the tile's rows (G divides 128 and N): the
+// group's maximum is taken over its G / 8 lanes.
+template <PackFrom FROM>
+__global__ __launch_bounds__(kBlock) void k_pack_i4_tiled(const float* __restrict__ src, int64_t K, int64_t N, int64_t G,
+                                                          int64_t Kpad, int64_t RQ, int64_t NS, int ncol,
+                                                          const float* __restrict__ inv, uint32_t* __restrict__ strips,
+                                                          uint32_t* __restrict__ koct, int ngap,
+                                                          float* __restrict__ scales, float* __restrict__ devscales,
+                                                          float* __restrict__ qdata, int* __restrict__ bad) {
+    constexpr int kOct = kPackCols / 8;
+    __shared__ uint32_t word[kOct][kPackRows + 1];
+    __shared__ float tsc[FROM == kFromX ? kOct : 1][kPackRows + 1];
+    const int64_t kb = blockIdx.x / ncol, cb = blockIdx.x - kb * ncol;
+    const int64_t k0 = kb * kPackRows, j0 = cb * kOct;
+    const int oc = threadIdx.x & (kOct - 1), r0 = threadIdx.x / kOct;
+    const int64_t j = j0 + oc;
+    float v[2][8];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int64_t k = k0 + r0 + 16 * h;
+        const bool in = k < K && j < NS;
+        const float* p = src + k * N + 8 * j;
+        const float4_u a = in ? *(const float4_u*)p : float4_u{0.f, 0.f, 0.f, 0.f};
+        const float4_u c = in ? *(const float4_u*)(p + 4) : float4_u{0.f, 0.f, 0.f, 0.f};
+        v[h][0] = a.x, v[h][1] = a.y, v[h][2] = a.z, v[h][3] = a.w;
+        v[h][4] = c.x, v[h][5] = c.y, v[h][6] = c.z, v[h][7] = c.w;
+    }
     int badflag = 0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
+    for (int h = 0; h < 2; ++h) {
+        const int r = r0 + 16 * h;
         const int64_t k = k0 + r;
-        uint32_t word = 0;
-        if (k < K) {
-            // The strip layout requires N % 8 == 0 and G % 8 == 0, so the 8
-            // columns of this row of the strip lie in one group.
-            const int64_t i0 = k * N + n0;
-            const float iv = from_codes ? 0.0f : inv[i0 / G];
+        const bool in = k < K && j < NS;
+        const int64_t i0 = k * N + 8 * j;
+        float iv = 0.0f;
+        if constexpr (FROM == kFromX) {
+            float m = 1e-8f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) m = ref_max(m, fabsf(v[h][e]));
+            for (int o = 1; o < (int)(G >> 3); o <<= 1) m = ref_max(m, __shfl_xor(m, o));
+            iv = 7.0f / m;
+            const float sc = m / 7.0f;
+            if (in && (oc & (int)((G >> 3) - 1)) == 0) scales[i0 / G] = sc;
+            tsc[oc][r] = k < K ? sc : 0.0f;
+        } else if constexpr (FROM == kFromXInv) {
+            if (in) iv = inv[i0 / G];  // N and G are multiples of 8: one group per octet
+        }
+        uint32_t w = 0;
+        if (in) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int64_t i = i0 + e;
-                float v;
-                if (from_codes) {
-                    v = src[i];
-                    if (!valid_code(v, -8.0f, 7.0f)) {
-                        badflag = 1;
-                        v = 0.0f;
-                    }
+                float c = v[h][e];
+                if constexpr (FROM == kFromCodes) {
+                    if (!valid_code(c, -8.0f, 7.0f)) badflag = 1, c = 0.0f;
                 } else {
-                    v = ref_code(src[i], iv, -8.0f, 7.0f);
-                    if (qdata) qdata[i] = v;
+                    c = ref_code(c, iv, -8.0f, 7.0f);
                 }
-                word |= ((uint32_t)(int)v & 0xFu) << (4 * e);
+                v[h][e] = c;
+                w |= ((uint32_t)(int)c & 0xFu) << (4 * e);
+            }
+            if (FROM != kFromCodes && qdata) {
+                *(float4_u*)(qdata + i0) = float4_u{v[h][0], v[h][1], v[h][2], v[h][3]};
+                *(float4_u*)(qdata + i0 + 4) = float4_u{v[h][4], v[h][5], v[h][6], v[h][7]};
             }
         }
-        dw[r] = word;
+        word[oc][r] = w;
     }
-    if (packed) packed[j * RQ + rq] = make_uint4(dw[0], dw[1], dw[2], dw[3]);
     if (badflag) atomicOr(bad, 1);
-    }
-}
-
-// The k-octet copy of an INT4 strip-major weight, built from its strips: one
-// thread per dword t of block (cb, kb), column 16 cb + (t & 15), rows
-// 32 kb + 8 (t >> 4) .. + 7 in nibbles 0..7.  Strip dword (j, row k) is dword
-// 4 * (j * RQ + k / 4) + k % 4, column n of it nibble n % 8.  The first ngap
-// threads also zero the ngap dwords between the strips and the copy, so that
-// the whole buffer is a function of the codes.
-__global__ void k_koct_i4(const uint32_t* __restrict__ strips, int64_t N, int64_t Kpad, int64_t RQ, int64_t KB,
-                          int64_t ndw, uint32_t* __restrict__ koct, uint32_t* __restrict__ gap, int ngap) {
-    const int64_t t0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t0 < ngap) gap[t0] = 0u;
-    for (int64_t d = t0; d < ndw; d += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t blk = d >> 6, t = d & 63;
-        const int64_t cb = blk / KB, kb = blk - cb * KB;
-        const int64_t n = 16 * cb + (t & 15), j = n >> 3;
-        const int e = (int)(n & 7);
-        const int64_t k0 = 32 * kb + 8 * (t >> 4);
-        uint32_t word = 0;
-        if (n < N) {
+    __syncthreads();
+    const int64_t KB = (Kpad + 31) / 32, NB = (NS + 1) / 2;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int64_t k = k0 + i;
-                if (k < Kpad) word |= ((strips[4 * (j * RQ + (k >> 2)) + (k & 3)] >> (4 * e)) & 0xFu) << (4 * i);
-            }
+    for (int h = 0; h < 2; ++h) {
+        const int t = threadIdx.x + h * kBlock;
+        // Strip t / 32, row t % 32.
+        const int64_t js = j0 + (t >> 5), k = k0 + (t & 31);
+        if (js < NS && k < Kpad) strips[4 * js * RQ + k] = word[t >> 5][t & 31];
+        // k-octet dword t % 64 of column block t / 64.
+        const int c = t & 15, g = (t >> 4) & 3;
+        const int64_t blk = j0 / 2 + (t >> 6);
+        if (blk < NB) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                w |= ((word[2 * (t >> 6) + (c >> 3)][8 * g + i] >> (4 * (c & 7))) & 0xFu) << (4 * i);
+            koct[(blk * KB + kb) * 64 + (t & 63)] = w;
         }
-        koct[d] = word;
+        if constexpr (FROM == kFromX) {
+            // Scale column of the tile's strip t / 32 where that strip is its first.
+            const int64_t sc = js * 8 / G;
+            if (js < NS && k < Kpad && (js * 8) % G == 0) devscales[sc * Kpad + k] = tsc[t >> 5][t & 31];
+        }
     }
+    // The dwords between the strips and the copy, so that the whole buffer is a
+    // function of the codes.
+    if (blockIdx.x == 0 && (int)threadIdx.x < ngap) koct[(int64_t)threadIdx.x - ngap] = 0u;
 }
 
 // INT4 flat pack: one thread per byte (elements 2b, 2b+1 of the flattened tensor).
@@ -334,9 +423,12 @@ hipError_t launch_fill_bias(float* y, int64_t M, int64_t N, const float* bias, h
 hipError_t launch_group_scales(const float* x, int64_t total, int64_t G, int64_t ngroups, float qmax, float* scales,
                                float* inv, hipStream_t s) {
     if (ngroups <= 0) return hipSuccess;
-    const int64_t waves_per_block = kBlock / 64;
-    k_group_scales<<<grid_for(ngroups * 64, 1 << 16), kBlock, 0, s>>>(x, total, G, ngroups, qmax, scales, inv);
-    (void)waves_per_block;
+    if (G >= 1024)
+        k_group_scales<64, 4><<<grid_for(ngroups * 64), kBlock, 0, s>>>(x, total, G, ngroups, qmax, scales, inv);
+    else if (G > 128)
+        k_group_scales<64, 1><<<grid_for(ngroups * 64), kBlock, 0, s>>>(x, total, G, ngroups, qmax, scales, inv);
+    else
+        k_group_scales<8, 1><<<grid_for(ngroups * 8), kBlock, 0, s>>>(x, total, G, ngroups, qmax, scales, inv);
     return hipGetLastError();
 }
 
@@ -354,29 +446,42 @@ hipError_t launch_absmax_partial(const float* x, int64_t total, float* partial, 
 
 hipError_t launch_pack_i8_tiled(const float* src, bool from_codes, int64_t K, int64_t N, const float* inv,
                                 bool per_tensor, void* packed, float* qdata, int* bad, hipStream_t s) {
-    I8Geom g(K, N);
-    const int64_t nchunks = g.chunks();
-    if (nchunks <= 0) return hipSuccess;
-    k_pack_i8_tiled<<<grid_for(nchunks), kBlock, 0, s>>>(src, from_codes, K, N, g.RQ, g.NS, nchunks, inv, per_tensor,
-                                                         (uint4*)packed, qdata, bad);
+    const I8Geom g(K, N);
+    if (g.chunks() <= 0) return hipSuccess;
+    const int64_t ncol = ceil_div(N, kPackCols), blocks = ceil_div(g.Kpad, kPackRows) * ncol;
+    if (blocks >= (int64_t)1 << 31) return hipErrorInvalidValue;
+    if (from_codes)
+        k_pack_i8_tiled<kFromCodes><<<(unsigned)blocks, kBlock, 0, s>>>(src, K, N, g.RQ, g.NS, (int)ncol, inv, per_tensor,
+                                                                        (uint4*)packed, qdata, bad);
+    else
+        k_pack_i8_tiled<kFromXInv><<<(unsigned)blocks, kBlock, 0, s>>>(src, K, N, g.RQ, g.NS, (int)ncol, inv, per_tensor,
+                                                                       (uint4*)packed, qdata, bad);
     return hipGetLastError();
 }
 
-hipError_t launch_pack_i4_tiled(const float* src, bool from_codes, int64_t K, int64_t N, int64_t G,
-                                const float* inv, void* packed, float* qdata, int* bad, hipStream_t s) {
-    I4Geom g(K, N, G);
-    const int64_t nchunks = g.chunks();
-    if (nchunks <= 0) return hipSuccess;
-    k_pack_i4_tiled<<<grid_for(nchunks), kBlock, 0, s>>>(src, from_codes, K, N, g.G, g.RQ, g.NS, nchunks, inv,
-                                                         (uint4*)packed, qdata, bad);
-    if (packed) {
-        const int64_t ndw = g.koct_bytes() / 4;
-        const int64_t strip_bytes = g.chunks() * 16;
-        k_koct_i4<<<grid_for(ndw), kBlock, 0, s>>>((const uint32_t*)packed, N, g.Kpad, g.RQ, g.KB(), ndw,
-                                                   (uint32_t*)((char*)packed + g.koct_off()),
-                                                   (uint32_t*)((char*)packed + strip_bytes),
-                                                   (int)((g.koct_off() - strip_bytes) / 4));
-    }
+bool pack_i4_finds_scales(const I4Geom& g) { return g.tiled && g.N % g.G == 0 && kPackCols % g.G == 0; }
+
+hipError_t launch_pack_i4_tiled(const float* src, bool from_codes, int64_t K, int64_t N, int64_t G, const float* inv,
+                                void* packed, float* scales, float* devscales, float* qdata, int* bad, hipStream_t s) {
+    const I4Geom g(K, N, G);
+    if (g.chunks() <= 0) return hipSuccess;
+    const int64_t ncol = ceil_div(g.NS, kPackCols / 8), blocks = g.KB() * ncol;
+    if (blocks >= (int64_t)1 << 31) return hipErrorInvalidValue;
+    const int ngap = (int)((g.koct_off() - g.chunks() * 16) / 4);
+    uint32_t* koct = (uint32_t*)((char*)packed + g.koct_off());
+#define SGQ_PACK_I4(FROM_)                                                                                          \
+    k_pack_i4_tiled<FROM_><<<(unsigned)blocks, kBlock, 0, s>>>(src, K, N, g.G, g.Kpad, g.RQ, g.NS, (int)ncol, inv, \
+                                                               (uint32_t*)packed, koct, ngap, scales, devscales,   \
+                                                               qdata, bad)
+    if (from_codes)
+        SGQ_PACK_I4(kFromCodes);
+    else if (inv)
+        SGQ_PACK_I4(kFromXInv);
+    else if (pack_i4_finds_scales(g))
+        SGQ_PACK_I4(kFromX);
+    else
+        return hipErrorInvalidValue;
+#undef SGQ_PACK_I4
     return hipGetLastError();
 }
 
