@@ -215,7 +215,7 @@ inline SkinnyPlan skinny_plan(int64_t M, int64_t K, const I4Geom& g, int64_t cus
 }
 // INT8 batches on the bf16 matrix cores (k_skinny8): workgroups of MB row
 // blocks of 16 (two above 16 rows) by C column blocks of 16 over all of K, no
-// workspace.  C = 2 where that still gives a workgroup per CU.  The GEMV
+// workspace, C by the rounds the grid takes (below).  The GEMV
 // keeps four rows and little work (its time is a fixed ~3 us plus
 // round_up(M, 8) * K * N at the VALU rate); above 16 rows the GEMM keeps
 // M * K * N > 2^29 (its wider tiles read each x row for more columns).
@@ -241,7 +241,20 @@ inline Skinny8Plan skinny8_plan(int64_t M, int64_t K, int64_t N, int64_t cus) {
     if (round_up(M, 8) * K * N < kSkinny8MinWork) return p;
     if (M > kGemvMaxM && M * K * N > kSkinny8MaxWork) return p;
     p.MB = M > 16 ? 2 : 1;
-    p.C = ceil_div(M, 16 * p.MB) * ceil_div(ceil_div(N, 4), 8) >= cus ? 2 : 1;
+    // One workgroup (16 wavefronts) fills a CU, so a grid runs in rounds of cus
+    // workgroups, each costing the split of x (once per row block and k block,
+    // about 52 instructions) and C column blocks (about 15 each).  Measured (us,
+    // C = 1 / 2 / 4, per channel unless said): 4096 -> 11008 at 16 rows 36.0 / 28.6
+    // / 19.1, at 17 rows over K = 2048 23.4 / 18.4 / 11.9; 2048 -> 5632 at 16 rows
+    // 13.5 / 8.8 / 10.7; 8192 -> 28672 at 8 rows per tensor 88.9 / 73.2 / 58.2;
+    // 4096^2 at 16 rows 12.9 / 14.9 / 18.9; 1024 -> 4096 at 100 rows per tensor
+    // 18.2 / 13.1 / 11.5.
+    int64_t best = 0;
+    for (int c : {1, 2, 4}) {
+        const int64_t wgs = ceil_div(M, 16 * p.MB) * ceil_div(N, 16 * c);
+        const int64_t cost = ceil_div(wgs, cus < 1 ? 1 : cus) * (52 + 15 * c);
+        if (best == 0 || cost < best) best = cost, p.C = c;
+    }
     return p;
 }
 // Workspace of a skinny launch with NG weights: the K ranges' partial sums.

@@ -1461,9 +1461,9 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
 //
 // B operand straight from the strip layout, without a transpose: dword d of
 // an INT8 chunk is column 4j + d over the chunk's four rows, so lane l
-// (g = l >> 4; column n = l & 15 of its block: strip n >> 2, dword n & 3)
-// takes that dword of row quads 2g and 2g + 1 of the k block, rows
-// 8g .. 8g + 7 of its column.  A block past the end reads x (and per-channel
+// (g = l >> 4, n = l & 15) takes C consecutive dwords of row quads 2g and 2g + 1
+// of the k block, rows 8g .. 8g + 7 of columns C n .. C n + C - 1, one for each
+// column block.  A block past the end reads x (and per-channel
 // scales) as zeros; its code dwords are whatever follows and are multiplied
 // by zero.
 struct Skinny8Args {
@@ -1521,9 +1521,9 @@ __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ h
     const __amdgpu_buffer_rsrc_t rW = make_rsrc(hW + (int64_t)s0 * RQ, (uint32_t)nstr * (uint32_t)RQ * 16u);
     const __amdgpu_buffer_rsrc_t rX = make_rsrc(hx + (int64_t)m0 * K, (uint32_t)mrows * (uint32_t)K * 4u);
     const __amdgpu_buffer_rsrc_t rS = make_rsrc(hS, PT ? 4u : (uint32_t)K * 4u);
-    int wv[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) wv[c] = ((4 * c + (n >> 2)) * RQ + 2 * g) * 16 + (n & 3) * 4;
+    // Column n of block c is column C n + c of the workgroup, so the C dwords of
+    // a lane are consecutive in its strip's chunk: one load per row quad.
+    const int wv = ((C * n >> 2) * RQ + 2 * g) * 16 + ((C * n) & 3) * 4;
     const int xr = HALF ? (n & 7) : n, xk = HALF ? 4 * (n >> 3) : 0;
     floatx4 acc[MB][C];
 #pragma unroll
@@ -1538,9 +1538,16 @@ __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ h
         for (int u = 0; u < U; ++u) {
             const int kb = kb0 + u * NW;
 #pragma unroll
-            for (int c = 0; c < C; ++c) {
-                w[u][c][0] = __builtin_amdgcn_raw_buffer_load_b32(rW, wv[c], kb * 128, 0);
-                w[u][c][1] = __builtin_amdgcn_raw_buffer_load_b32(rW, wv[c] + 16, kb * 128, 0);
+            for (int h = 0; h < 2; ++h) {
+                if constexpr (C == 4) {
+                    const uint4 q = buf_load16(rW, wv + 16 * h, kb * 128);
+                    w[u][0][h] = q.x, w[u][1][h] = q.y, w[u][2][h] = q.z, w[u][3][h] = q.w;
+                } else if constexpr (C == 2) {
+                    const auto q = __builtin_amdgcn_raw_buffer_load_b64(rW, wv + 16 * h, kb * 128, 0);
+                    w[u][0][h] = q[0], w[u][1][h] = q[1];
+                } else {
+                    w[u][0][h] = __builtin_amdgcn_raw_buffer_load_b32(rW, wv + 16 * h, kb * 128, 0);
+                }
             }
             const int k0 = kb * 32 + 8 * g + xk;
 #pragma unroll
@@ -1608,27 +1615,29 @@ __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ h
     // Accumulator element r of lane l is output row 4 * (l >> 4) + r of
     // column l & 15 of its block.  The wavefronts' partial tiles are summed
     // in wavefront order through LDS; thread t then owns output t
-    // (t + NW * 64, ...): block bc = t >> 8, row (t >> 4) & 15, column t & 15.
+    // (t + NW * 64, ...): consecutive threads take consecutive columns (a pad
+    // of 16 floats keeps the blocks' reads on different banks).
     constexpr int NBC = MB * C;
     constexpr int OPT = (256 * NBC + NW * 64 - 1) / (NW * 64);
-    __shared__ float red[NW][NBC][4][64];
+    __shared__ float red[NW][NBC][4 * 64 + (C > 1 ? 64 / C : 0)];
 #pragma unroll
     for (int b = 0; b < MB; ++b)
 #pragma unroll
         for (int c = 0; c < C; ++c)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) red[wave][b * C + c][r][lane] = acc[b][c][r];
+            for (int r = 0; r < 4; ++r) red[wave][b * C + c][64 * r + lane] = acc[b][c][r];
     __syncthreads();
     const float s_all = PT ? a.S[0] : 1.0f;
 #pragma unroll
     for (int i = 0; i < OPT; ++i) {
         const int t = threadIdx.x + i * NW * 64;
-        const int bc = t >> 8, mi = (t >> 4) & 15, nl = t & 15;
-        const int m = m0 + 16 * (bc / C) + mi, col = 16 * (cg * C + bc % C) + nl;
+        const int cl = t % (16 * C), mr = t / (16 * C);  // column and row of the workgroup
+        const int mi = mr & 15, nl = cl / C, bc = (mr >> 4) * C + cl % C;
+        const int m = m0 + mr, col = 16 * C * cg + cl;
         if (t < 256 * NBC && m < a.M && col < a.N) {
             float s = 0.0f;
 #pragma unroll
-            for (int w2 = 0; w2 < NW; ++w2) s += red[w2][bc][mi & 3][16 * (mi >> 2) + nl];
+            for (int w2 = 0; w2 < NW; ++w2) s += red[w2][bc][64 * (mi & 3) + 16 * (mi >> 2) + nl];
             if constexpr (PT) s = s * s_all;
             // h + m + l turns an infinite x into inf - inf: recompute a
             // non-finite total as the reference's k-order sum.
@@ -2034,7 +2043,7 @@ hipError_t skinny8_launch(const float* x, int64_t M, int64_t K, int64_t N, const
     a.y = y;
     a.nblk = (int)(ceil_div(M, 16 * MB) * a.ncg);
     a.xlog = xcd_log2(device_xcds(s));
-    constexpr int U = MB == 1 ? 4 : 2;  // register budget of 16 wavefronts per CU
+    constexpr int U = MB == 1 && C < 4 ? 4 : 2;  // register budget of 16 wavefronts per CU
     if (g.Kpad != 4 * g.RQ) return hipErrorInvalidValue;  // Skinny8Hot carries RQ only
     const Skinny8Hot h = skinny8_hot(a);
     if (MB == 1 && M <= 8)
@@ -2059,8 +2068,10 @@ hipError_t launch_skinny_i8(const float* x, int64_t M, int64_t K, int64_t N, con
     }
     SGQ_SKINNY8(1, 1)
     SGQ_SKINNY8(2, 1)
+    SGQ_SKINNY8(4, 1)
     SGQ_SKINNY8(1, 2)
     SGQ_SKINNY8(2, 2)
+    SGQ_SKINNY8(4, 2)
 #undef SGQ_SKINNY8
     return hipErrorInvalidValue;
 }
