@@ -38,6 +38,8 @@ GROUPED = 2  # QuantizationScheme::GroupedAsymmetric
 LAYOUT_INT4_TILED = 0
 LAYOUT_INT4_FLAT = 1
 
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
 # Every entry point of include/sgq.h with its ctypes signature.
 _i64, _int, _vp = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p
 SIGNATURES = {
@@ -84,6 +86,8 @@ _lib_lock = threading.Lock()
 def load_library(path: Optional[os.PathLike] = None) -> ctypes.CDLL:
     """Loads libsgq.so and declares every signature.  Raises if it is missing."""
     global _lib
+    if path is None and _lib is not None:  # set once, complete
+        return _lib
     with _lib_lock:
         if _lib is not None and path is None:
             return _lib
@@ -123,12 +127,15 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # The raw handle, without building a torch.cuda.Stream around it (1.0 us of an eager call).
+    return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
 
 
 def _dev_f32(t: torch.Tensor) -> torch.Tensor:
     if not t.is_cuda:
         raise ValueError("sgq: expected a device tensor")
+    if t.dtype is torch.float32 and t.is_contiguous():
+        return t
     return t.contiguous().to(torch.float32)
 
 
@@ -188,6 +195,8 @@ class QuantizedTensor:
 def _view2d(shape) -> tuple:
     """[rows, cols] view of a weight: rows = shape[0] (src/quantization.cpp:44-45),
     rank-1 tensors are one row."""
+    if len(shape) == 2:
+        return int(shape[0]), int(shape[1])
     if len(shape) >= 2:
         cols = 1
         for d in shape[1:]:
@@ -323,7 +332,7 @@ def dequantize_codes(qx: QuantizedTensor) -> torch.Tensor:
 def _linear_args(x: torch.Tensor, qw: QuantizedTensor, bias: Optional[torch.Tensor]):
     if x.dim() != 2:
         raise ValueError("matmul currently requires 2D tensors!")  # src/ops.cpp:380-382
-    K, N = qw.rows, qw.cols
+    K, N = _view2d(qw.original_shape)
     if x.shape[1] != K:
         raise ValueError("Matrix inner dimensions must match for matmul!")  # src/ops.cpp:387-389
     x = _dev_f32(x)
@@ -341,7 +350,7 @@ def quantized_matmul_int8(x: torch.Tensor, qw: QuantizedTensor, bias: Optional[t
     x, K, N, b = _linear_args(x, qw, bias)
     M = x.shape[0]
     dev = x.device
-    y = out if out is not None else torch.empty((M, N), dtype=torch.float32, device=dev)
+    y = out if out is not None else x.new_empty((M, N))
     ws, nws = _linear_ws.get(lib.sgq_linear_workspace_bytes(8, M, K, N), dev)
     _check(lib.sgq_linear_int8(_ptr(x), M, K, N, _ptr(qw.packed), _ptr(qw.scales), _int8_branch(qw), _ptr(b),
                                _ptr(y), ws, nws, _stream(dev)))
@@ -354,7 +363,7 @@ def quantized_matmul_int4(x: torch.Tensor, qw: QuantizedTensor, bias: Optional[t
     x, K, N, b = _linear_args(x, qw, bias)
     M = x.shape[0]
     dev = x.device
-    y = out if out is not None else torch.empty((M, N), dtype=torch.float32, device=dev)
+    y = out if out is not None else x.new_empty((M, N))
     ws, nws = _linear_ws.get(lib.sgq_linear_workspace_bytes(4, M, K, N), dev)
     _check(lib.sgq_linear_int4(_ptr(x), M, K, N, _ptr(qw.packed), _ptr(qw.scales), _ptr(qw.devscales),
                                qw.group_size, _ptr(b), _ptr(y), ws, nws, _stream(dev)))
