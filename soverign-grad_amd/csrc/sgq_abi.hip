@@ -606,7 +606,7 @@ int sgq_linear_int8(const float* x, int64_t M, int64_t K, int64_t N, const void*
         return fail(SGQ_ERR_UNSUPPORTED, "sgq_linear_int8: K = %lld is too long for this batch", (long long)K);
     const Skinny8Plan sp = skinny8_plan(M, K, N, device_cus(s));
     if (sp.C > 0) {
-        SGQ_HIP(launch_skinny_i8(x, M, K, N, packed, scales, per_tensor, bias, sp, y, s), "skinny_i8");
+        SGQ_HIP(launch_skinny_i8(x, M, K, N, packed, scales, per_tensor, bias, nullptr, sp, y, s), "skinny_i8");
     } else if (linear_uses_gemv(M, K, N)) {
         SGQ_HIP(launch_gemv_i8(x, M, K, N, packed, scales, per_tensor, bias, y, s), "gemv_i8");
     } else {
@@ -615,7 +615,7 @@ int sgq_linear_int8(const float* x, int64_t M, int64_t K, int64_t N, const void*
         const int lw = check_launch_ws("sgq_linear_int8", gemm_launch_ws_bytes(8, M, K, N, 0, device_cus(s)),
                                        workspace, workspace_bytes);
         if (lw != SGQ_OK) return lw;
-        SGQ_HIP(launch_gemm_i8(x, M, K, N, packed, scales, per_tensor, bias, y, workspace, s), "gemm_i8");
+        SGQ_HIP(launch_gemm_i8(x, M, K, N, packed, scales, per_tensor, bias, {}, y, workspace, s), "gemm_i8");
     }
     return ok();
 }
@@ -677,9 +677,9 @@ int sgq_swiglu_int8(const float* x, int64_t M, int64_t K, int64_t N, const void*
     // gated MLP's sums are those of two forward calls.
     const Skinny8Plan sp = skinny8_plan(M, K, N, device_cus(s));
     if (sp.C > 0) {
-        SGQ_HIP(launch_skinny_i8(x, M, K, N, packed_gate, scales_gate, per_tensor, bias_gate, sp, h, s), "skinny_i8");
-        SGQ_HIP(launch_skinny_i8(x, M, K, N, packed_up, scales_up, per_tensor, bias_up, sp, u, s), "skinny_i8");
-        SGQ_HIP(launch_silu_mul(h, u, M * N, s), "silu_mul");
+        SGQ_HIP(launch_skinny_i8(x, M, K, N, packed_gate, scales_gate, per_tensor, bias_gate, nullptr, sp, h, s),
+                "skinny_i8");
+        SGQ_HIP(launch_skinny_i8(x, M, K, N, packed_up, scales_up, per_tensor, bias_up, h, sp, h, s), "skinny_i8");
         return ok();
     }
     if (linear_uses_gemv(M, K, N)) {
@@ -692,9 +692,13 @@ int sgq_swiglu_int8(const float* x, int64_t M, int64_t K, int64_t N, const void*
                                    workspace, workspace_bytes);
     if (lw != SGQ_OK) return lw;
     void* split = (char*)workspace + align_up(M * N * 4);
-    SGQ_HIP(launch_gemm_i8(x, M, K, N, packed_gate, scales_gate, per_tensor, bias_gate, h, split, s), "gemm_i8");
-    SGQ_HIP(launch_gemm_i8(x, M, K, N, packed_up, scales_up, per_tensor, bias_up, u, split, s), "gemm_i8");
-    SGQ_HIP(launch_silu_mul(h, u, M * N, s), "silu_mul");
+    SGQ_HIP(launch_gemm_i8(x, M, K, N, packed_gate, scales_gate, per_tensor, bias_gate, {}, h, split, s), "gemm_i8");
+    if (gemm_i8_epilogue(x, M, K, N, device_cus(s))) {
+        SGQ_HIP(launch_gemm_i8(x, M, K, N, packed_up, scales_up, per_tensor, bias_up, {h}, h, split, s), "gemm_i8");
+    } else {
+        SGQ_HIP(launch_gemm_i8(x, M, K, N, packed_up, scales_up, per_tensor, bias_up, {}, u, split, s), "gemm_i8");
+        SGQ_HIP(launch_silu_mul(h, u, M * N, s), "silu_mul");
+    }
     return ok();
 }
 

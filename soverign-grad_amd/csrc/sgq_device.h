@@ -66,20 +66,13 @@ __device__ __forceinline__ uint32_t buf_load4_stream(__amdgpu_buffer_rsrc_t r, i
     return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, kStreamPolicy);
 }
 
-// Four floats at byte offset voff + soff (zero past the end).  ALIGN4: the
-// buffer holds a multiple of four floats, so a quad is entirely in or out and
-// one 128-bit load serves; otherwise four 32-bit loads.
-template <bool ALIGN4>
+// Four floats at byte offset voff + soff from any 4-byte address (128-bit
+// buffer loads need dword alignment only); each float past the end is zero on
+// its own (the range check of a raw buffer is by dword), so rows of any length
+// and alignment load this way.
 __device__ __forceinline__ float4 buf_load4f(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    if (ALIGN4) {
-        const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-        return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-    } else {
-        return make_float4(__uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 0, soff, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 4, soff, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 8, soff, 0)),
-                           __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff + 12, soff, 0)));
-    }
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+    return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
 }
 
 // silu(v) = v / (1 + exp(-v)), as simd::vec_silu (simd.hpp:103-108); the

@@ -1,6 +1,7 @@
 // sgq_gemm.hip -- the INT4 prefill GEMM of the fused dequantize + matmul
-// forward (src/quantization.cpp:199-206 for batches past the GEMV and skinny
-// kernels) and the sum of split-K partial results.
+// forward (src/quantization.cpp:189-206 for batches past the GEMV and skinny
+// kernels), also INT8's where rows of x are not 16-byte aligned, and the sum of
+// split-K partial results.
 //
 // k_gemm_wave runs the fp32 products on the bf16 matrix cores as three exact
 // bf16 products each, as k_gemm3 does for INT8 (sgq_linear.hip): x * s split
@@ -65,11 +66,12 @@ struct GemmWaveArgs {
 
 // Workgroup b computes split b % KS (stages [kb0, kb1) of sps each) of tile
 // b / KS; its four wavefronts are 4 / sk tiles of sk K ranges each.
-template <int RB, int GPW>
+template <int BITS, int RB, int GPW, bool PT>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_wave(const GemmWaveArgs a) {
     constexpr int CB = kWaveCols / 16;  // column blocks of 16 per wavefront
     constexpr int CPG = CB / GPW;       // of one scale group
     constexpr int BM = 16 * RB;
+    constexpr int BW = BITS == 8 ? 2 : 1;  // code dwords per lane and column block
     __shared__ __attribute__((aligned(16))) float red[4][16][kWaveCols + 4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 15, g = lane >> 4;
@@ -108,47 +110,76 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
         const int mrows = min(BM, M - m0);
         const __amdgpu_buffer_rsrc_t rX = make_rsrc(a.x + (int64_t)m0 * K, (uint32_t)mrows * (uint32_t)K * 4u);
         const int KB = (a.Kpad + 31) >> 5;
-        // Column blocks past the weight's read as zero.
-        const int ncb = min(CB, (a.NS + 1) / 2 - n0 / 16);
-        const __amdgpu_buffer_rsrc_t rW =
-            make_rsrc(W + ((int64_t)a.ko + (int64_t)(n0 / 16) * KB) * 16, (uint32_t)ncb * (uint32_t)KB * 256u);
-        __amdgpu_buffer_rsrc_t rS[GPW];
+        // Column blocks (INT8: strips) past the weight's read as zero.
+        __amdgpu_buffer_rsrc_t rW, rS[GPW];
+        if constexpr (BITS == 8) {
+            const int nstr = min(kWaveCols / 4, a.NS - n0 / 4);
+            rW = make_rsrc(W + (int64_t)(n0 / 4) * a.RQ, (uint32_t)nstr * (uint32_t)a.RQ * 16u);
+            rS[0] = make_rsrc(S, PT ? 4u : (uint32_t)K * 4u);
+        } else {
+            const int ncb = min(CB, (a.NS + 1) / 2 - n0 / 16);
+            rW = make_rsrc(W + ((int64_t)a.ko + (int64_t)(n0 / 16) * KB) * 16, (uint32_t)ncb * (uint32_t)KB * 256u);
 #pragma unroll
-        for (int q = 0; q < GPW; ++q) {
-            const int strip = min(n0 / 8 + q * (2 * CPG), a.NS - 1);
-            rS[q] = make_rsrc(S + (int64_t)(strip / a.spc) * a.Kpad, (uint32_t)a.Kpad * 4u);
+            for (int q = 0; q < GPW; ++q) {
+                const int strip = min(n0 / 8 + q * (2 * CPG), a.NS - 1);
+                rS[q] = make_rsrc(S + (int64_t)(strip / a.spc) * a.Kpad, (uint32_t)a.Kpad * 4u);
+            }
         }
         int xo[RB];
 #pragma unroll
         for (int i = 0; i < RB; ++i) xo[i] = ((i * 16 + lr) * K + 8 * g) * 4;
 
-        uint32_t bw[CB];
+        uint32_t bw[CB][BW];
         float4 xq[RB][2], sv[GPW][2];
         // Past the last stage these read zeros, the next row or column block;
         // what they read is not used.
         auto loadB = [&](int kt) {
+            if constexpr (BITS == 8) {
+                // Column lr of block c is column 64 (c / 4) + 4 lr + c % 4 of the
+                // tile: the four dwords of a chunk of strip lr serve four blocks.
 #pragma unroll
-            for (int c = 0; c < CB; ++c)
-                bw[c] = __builtin_amdgcn_raw_buffer_load_b32(rW, 4 * lane, (c * KB + kt) * 256, 0);
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const uint4 w = buf_load16(rW, (lr * a.RQ + 2 * g + q) * 16, (16 * h * a.RQ + 8 * kt) * 16);
+                        bw[4 * h][q] = w.x, bw[4 * h + 1][q] = w.y, bw[4 * h + 2][q] = w.z, bw[4 * h + 3][q] = w.w;
+                    }
+            } else {
+#pragma unroll
+                for (int c = 0; c < CB; ++c)
+                    bw[c][0] = __builtin_amdgcn_raw_buffer_load_b32(rW, 4 * lane, (c * KB + kt) * 256, 0);
+            }
         };
         auto loadS = [&](float4 (&s)[2], int q, int kt) {
-            s[0] = buf_load4f<true>(rS[q], 32 * g, kt * 128);
-            s[1] = buf_load4f<true>(rS[q], 32 * g + 16, kt * 128);
+            if constexpr (!PT) {
+                s[0] = buf_load4f(rS[q], 32 * g, kt * 128);
+                s[1] = buf_load4f(rS[q], 32 * g + 16, kt * 128);
+            }
         };
         // 128-bit buffer loads need dword alignment only, so rows of any K
         // (and any x) load the same way; full stages stay inside their row.
         auto loadX = [&](int i, int kt) {
-            xq[i][0] = buf_load4f<true>(rX, xo[i], kt * 128);
-            xq[i][1] = buf_load4f<true>(rX, xo[i] + 16, kt * 128);
+            xq[i][0] = buf_load4f(rX, xo[i], kt * 128);
+            xq[i][1] = buf_load4f(rX, xo[i] + 16, kt * 128);
         };
         bf16x8 bq[CB];
-        auto convB = [&](int c) { bq[c] = nibbles_bf16x16(bw[c]); };
+        auto convB = [&](int c) {
+            if constexpr (BITS == 8) {
+                // bytes of the column's dword in each row quad: k = 0..3, then 4..7
+                const uint32_t lo = bw[c][0], hi = bw[c][1];
+                bq[c] = __builtin_bit_cast(
+                    bf16x8, make_uint4(pack_hi16(cvt_sbyte<0>(lo), cvt_sbyte<1>(lo)), pack_hi16(cvt_sbyte<2>(lo), cvt_sbyte<3>(lo)),
+                                       pack_hi16(cvt_sbyte<0>(hi), cvt_sbyte<1>(hi)), pack_hi16(cvt_sbyte<2>(hi), cvt_sbyte<3>(hi))));
+            } else {
+                bq[c] = nibbles_bf16x16(bw[c][0]);
+            }
+        };
         // The planes of row block i scaled by s.
         auto split = [&](uint4 (&ap)[3], int i, const float4 (&s)[2]) {
             float v[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                v[e] = f4get(xq[i][e >> 2], e & 3) * f4get(s[e >> 2], e & 3);
+                v[e] = PT ? f4get(xq[i][e >> 2], e & 3) : f4get(xq[i][e >> 2], e & 3) * f4get(s[e >> 2], e & 3);
             split3(v, ap[0], ap[1], ap[2]);
         };
         auto mfma = [&](const uint4& ap, int i, int c) {
@@ -202,7 +233,7 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
                         for (int p = 0; p < 3; ++p) ap[p] = an[p];
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                if (GPW == 1) sv[0][0] = sn[0], sv[0][1] = sn[1];
+                if (GPW == 1 && !PT) sv[0][0] = sn[0], sv[0][1] = sn[1];
             }
         }
         if (kf < kt1) {
@@ -210,17 +241,25 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
             const int kt = kt1 - 1;
             const int k0 = kt * kStageK + 8 * g;
             loadB(kt);
-#pragma unroll
-            for (int q = 0; q < GPW; ++q) loadS(sv[q], q, kt);
-            auto one = [&](int base, int e) {
-                return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rX, k0 + e < K ? base + 4 * e : kOobOff, 0, 0));
+            auto one = [&](const __amdgpu_buffer_rsrc_t& r, int base, int e) {
+                return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, k0 + e < K ? base + 4 * e : kOobOff, 0, 0));
             };
+            if constexpr (BITS == 8 && !PT) {  // K scales, unpadded
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    sv[0][h] = make_float4(one(rS[0], 4 * k0, 4 * h), one(rS[0], 4 * k0, 4 * h + 1),
+                                           one(rS[0], 4 * k0, 4 * h + 2), one(rS[0], 4 * k0, 4 * h + 3));
+            } else {
+#pragma unroll
+                for (int q = 0; q < GPW; ++q) loadS(sv[q], q, kt);
+            }
 #pragma unroll
             for (int i = 0; i < RB; ++i) {
                 const int base = xo[i] + kt * 128;
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
-                    xq[i][h] = make_float4(one(base, 4 * h), one(base, 4 * h + 1), one(base, 4 * h + 2), one(base, 4 * h + 3));
+                    xq[i][h] = make_float4(one(rX, base, 4 * h), one(rX, base, 4 * h + 1), one(rX, base, 4 * h + 2),
+                                           one(rX, base, 4 * h + 3));
             }
 #pragma unroll
             for (int c = 0; c < CB; ++c) convB(c);
@@ -241,14 +280,24 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
     // Sixteen rows at a time through LDS: the K ranges are added in range
     // order, and a row of a tile is stored by consecutive lanes.
     const int klo = kb0 * kStageK, khi = min(K, kb1 * kStageK);
+    const float s_all = PT ? S[0] : 1.0f;
     const int nt = 4 / sk;  // tiles of the workgroup
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
         if (i > 0) __syncthreads();
+        if constexpr (BITS == 8) {
 #pragma unroll
-        for (int j = 0; j < CB; ++j)
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) red[wave][4 * g + r][16 * j + lr] = acc[i][j][r];
+                for (int r = 0; r < 4; ++r)
+                    *(float4*)&red[wave][4 * g + r][64 * h + 4 * lr] =
+                        make_float4(acc[i][4 * h][r], acc[i][4 * h + 1][r], acc[i][4 * h + 2][r], acc[i][4 * h + 3][r]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < CB; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) red[wave][4 * g + r][16 * j + lr] = acc[i][j][r];
+        }
         __syncthreads();
         // A thread takes four columns at a time.
         for (int t = threadIdx.x; t < nt * 16 * (kWaveCols / 4); t += kWG) {
@@ -261,30 +310,39 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
             const int um = sk == 1 ? tile_w >> 1 : 0, un = sk == 1 ? tile_w & 1 : tile_w;
             const int m = (tm * (sk == 1 ? 2 : 1) + um) * BM + i * 16 + row;
             const int n = (tn * (sk == 4 ? 1 : 2) + un) * kWaveCols + col;
-            if (m >= M || n >= N) continue;  // N is a multiple of 8 (the strip layout): all four or none
-            // The codes entered as 16q.  h + m + l turns an infinite x * s into
-            // inf - inf: recompute a non-finite total as the reference's k-order sum.
-            v.x *= 0.0625f, v.y *= 0.0625f, v.z *= 0.0625f, v.w *= 0.0625f;
+            if (m >= M || n >= N) continue;
+            // INT4 codes entered as 16q; per tensor, x itself in place of x * s.
+            const float f = BITS == 4 ? 0.0625f : s_all;
+            v.x *= f, v.y *= f, v.z *= f, v.w *= f;
+            // h + m + l turns an infinite x * s into inf - inf: recompute a
+            // non-finite total as the reference's k-order sum.
+            const int nc = BITS == 4 ? 4 : min(4, N - n);  // INT4: N is a multiple of 8
             if (!(isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w))) {
 #pragma unroll 1
-                for (int e = 0; e < 4; ++e) {
+                for (int e = 0; e < nc; ++e) {
                     const float w = f4get(v, e);
                     if (isfinite(w)) continue;
-                    const float r = output_exact<4>(a.x + (int64_t)m * K, W, S, a.spc, a.Kpad, a.RQ, n + e, klo, khi);
+                    const float r = output_exact<BITS>(a.x + (int64_t)m * K, W, S, BITS == 8 ? (PT ? 1 : 0) : a.spc, a.Kpad,
+                                                       a.RQ, n + e, klo, khi);
                     v.x = e == 0 ? r : v.x, v.y = e == 1 ? r : v.y, v.z = e == 2 ? r : v.z, v.w = e == 3 ? r : v.w;
                 }
             }
             const int64_t o = (int64_t)m * N + n;
             float* out = KS > 1 ? a.part + (int64_t)(wi * KS + split) * M * N : a.y + (int64_t)wi * M * N;
-            if (KS == 1) {
-                if (bias) v.x += bias[n], v.y += bias[n + 1], v.z += bias[n + 2], v.w += bias[n + 3];
-                v.x = gemm_epilogue(a.ep, v.x, o), v.y = gemm_epilogue(a.ep, v.y, o + 1);
-                v.z = gemm_epilogue(a.ep, v.z, o + 2), v.w = gemm_epilogue(a.ep, v.w, o + 3);
-            }
-            if (a.y16)
+            if (a.y16 && nc == 4) {
+                if (KS == 1) {
+                    if (bias) v.x += bias[n], v.y += bias[n + 1], v.z += bias[n + 2], v.w += bias[n + 3];
+                    v.x = gemm_epilogue(a.ep, v.x, o), v.y = gemm_epilogue(a.ep, v.y, o + 1);
+                    v.z = gemm_epilogue(a.ep, v.z, o + 2), v.w = gemm_epilogue(a.ep, v.w, o + 3);
+                }
                 *(float4*)(out + o) = v;
-            else
-                out[o] = v.x, out[o + 1] = v.y, out[o + 2] = v.z, out[o + 3] = v.w;
+            } else {
+                for (int e = 0; e < nc; ++e) {
+                    float w = f4get(v, e);
+                    if (KS == 1) w = gemm_epilogue(a.ep, bias ? w + bias[n + e] : w, o + e);
+                    out[o + e] = w;
+                }
+            }
         }
     }
 }
@@ -339,44 +397,60 @@ __global__ __launch_bounds__(kWG) void k_splitk_reduce(const float* __restrict__
 // ranges against two without a split: 384 x 4096 -> 11008 116 against 134,
 // 2048 x 4096 -> 11008 457 against 477; with one 40 x 4096 -> 4096 26.4
 // against 23.5, 96 x 11008 -> 4096 45 against 43.
-GemmWaveShape gemm_wave_shape(int64_t M, int64_t N, int spc, int KS, int64_t cus) {
+GemmWaveShape gemm_wave_shape(int64_t M, int64_t N, bool one_scale, int KS, int64_t cus) {
     GemmWaveShape w;
-    w.rb = spc % 16 == 0 && ceil_div(M, 64) * ceil_div(N, kWaveCols) * KS >= 4 * cus ? 4 : 2;
+    w.rb = one_scale && ceil_div(M, 64) * ceil_div(N, kWaveCols) * KS >= 4 * cus ? 4 : 2;
     w.sk = KS > 1 ? 2 : 4;
     return w;
 }
 
-hipError_t launch_gemm_wave(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
-                            const float* const* devscales, const float* const* bias, const I4Geom& g, const GemmPlan& p,
+hipError_t launch_gemm_wave(int bits, const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
+                            const float* const* scales, const float* const* bias, int mode, const GemmPlan& p,
                             const GemmWaveShape& w, const GemmEpilogue& ep, float* y, void* ws, hipStream_t s) {
-    const int gpw = g.spc % 16 == 0 ? 1 : (g.spc % 8 == 0 ? 2 : 4);
-    if (!gemm_wave_takes((int)g.spc) || (w.rb == 4 && gpw != 1) || nw < 1 || nw > 3 || (nw > 1 && (ep.gate || ep.res)))
+    const int gpw = bits == 8 || mode % 16 == 0 ? 1 : (mode % 8 == 0 ? 2 : 4);
+    if (!gemm_wave_takes(bits, mode) || (w.rb == 4 && gpw != 1) || nw < 1 || nw > 3 || (nw > 1 && (ep.gate || ep.res)))
         return hipErrorInvalidValue;
     GemmWaveArgs a{};
     a.x = x;
     a.M = (int)M, a.K = (int)K, a.N = (int)N;
-    for (int q = 0; q < nw; ++q) a.W[q] = (const uint4*)packed[q], a.S[q] = devscales[q], a.bias[q] = bias[q];
-    a.spc = (int)g.spc, a.Kpad = (int)g.Kpad, a.RQ = (int)g.RQ, a.NS = (int)g.NS;
-    a.ko = (int)(g.koct_off() / 256);
+    for (int q = 0; q < nw; ++q) a.W[q] = (const uint4*)packed[q], a.S[q] = scales[q], a.bias[q] = bias[q];
+    if (bits == 8) {
+        const I8Geom g(K, N);
+        a.Kpad = (int)g.Kpad, a.RQ = (int)g.RQ, a.NS = (int)g.NS;
+    } else {
+        const int64_t Kpad = round_up(K, kPadK);
+        a.spc = mode;
+        a.Kpad = (int)Kpad, a.RQ = (int)(Kpad / 4), a.NS = (int)(N / 8);
+        a.ko = (int)(round_up(N / 8 * (Kpad / 4) * 16, 256) / 256);  // I4Geom::koct_off
+    }
     a.KS = p.KS, a.sps = p.sps, a.sk = w.sk;
     a.ep = ep;
     a.y = y;
     a.part = p.KS > 1 ? (float*)ws : nullptr;
-    a.y16 = (((uintptr_t)(p.KS > 1 ? ws : y)) & 15) == 0;
+    a.y16 = N % 4 == 0 && (((uintptr_t)(p.KS > 1 ? ws : y)) & 15) == 0;
     const int64_t tm = ceil_div(M, w.rows()), tn = ceil_div(N, w.cols());
     a.ntn = (int)tn;
     const int xcds = device_xcds(s);
     a.xlog = xcd_log2(xcds);
-    a.xr = p.KS == 1 ? xcd_rect_rows(tm, tn, w.rows() * K * 4, w.cols() * K / 2, xcds) : 0;
+    a.xr = p.KS == 1 ? xcd_rect_rows(tm, tn, w.rows() * K * 4, w.cols() * K * bits / 8, xcds) : 0;
     const dim3 grid((unsigned)(tm * tn * p.KS), (unsigned)nw);
-    if (gpw == 1 && w.rb == 4)
-        k_gemm_wave<4, 1><<<grid, kWG, 0, s>>>(a);
-    else if (gpw == 1)
-        k_gemm_wave<2, 1><<<grid, kWG, 0, s>>>(a);
-    else if (gpw == 2)
-        k_gemm_wave<2, 2><<<grid, kWG, 0, s>>>(a);
-    else
-        k_gemm_wave<2, 4><<<grid, kWG, 0, s>>>(a);
+#define SGQ_GEMM_WAVE(BITS_, GPW_, PT_)                              \
+    if (w.rb == 4)                                                   \
+        k_gemm_wave<BITS_, 4, GPW_, PT_><<<grid, kWG, 0, s>>>(a);    \
+    else                                                             \
+        k_gemm_wave<BITS_, 2, GPW_, PT_><<<grid, kWG, 0, s>>>(a)
+    if (bits == 8 && mode) {
+        SGQ_GEMM_WAVE(8, 1, true);
+    } else if (bits == 8) {
+        SGQ_GEMM_WAVE(8, 1, false);
+    } else if (gpw == 1) {
+        SGQ_GEMM_WAVE(4, 1, false);
+    } else if (gpw == 2) {
+        k_gemm_wave<4, 2, 2, false><<<grid, kWG, 0, s>>>(a);
+    } else {
+        k_gemm_wave<4, 2, 4, false><<<grid, kWG, 0, s>>>(a);
+    }
+#undef SGQ_GEMM_WAVE
     return hipGetLastError();
 }
 

@@ -326,9 +326,11 @@ hipError_t launch_gemv_i8(const float* x, int64_t M, int64_t K, int64_t N, const
                           bool per_tensor, const float* bias, float* y, hipStream_t s);
 hipError_t launch_gemv_i4(const float* x, int64_t M, int64_t K, int64_t N, const void* packed,
                           const float* devscales, const I4Geom& g, const float* bias, float* y, hipStream_t s);
-// INT8 forward on k_skinny8 for a plan of skinny8_plan (C > 0).
+// INT8 forward on k_skinny8 for a plan of skinny8_plan (C > 0); gate (optional,
+// may be y): y = silu(gate) * (x W + bias).
 hipError_t launch_skinny_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* scales,
-                            bool per_tensor, const float* bias, const Skinny8Plan& p, float* y, hipStream_t s);
+                            bool per_tensor, const float* bias, const float* gate, const Skinny8Plan& p, float* y,
+                            hipStream_t s);
 // Skinny MFMA forward (plan p from skinny_plan, p.C > 0) of ng (1 or 2) tiled
 // INT4 weights of one shape on one input: ng == 1 writes y = x * W + bias,
 // ng == 2 the gated MLP h = silu(x * Wg + bg) * (x * Wu + bu).  With split K,
@@ -339,7 +341,7 @@ hipError_t launch_skinny_i8(const float* x, int64_t M, int64_t K, int64_t N, con
 // RMSNorm of x (gamma, eps) into the projections, as launch_gemv_i4_multi
 // does, and takes several weights only with it; the super-block form
 // (p.form == 1) adds res (same indexing as y) to the output, and takes several
-// weights of 17 or more rows of 16-byte aligned x.
+// weights of 17 or more rows.
 struct SkinnyExtra {
     int nw = 1;
     int64_t ldy = 0;  // 0: N
@@ -365,7 +367,7 @@ struct GemmPlan {
     int KS, sps;  // splits of K, 32-row stages per split
 };
 constexpr int kMaxSplits = 16;
-// What an INT4 GEMM does to each product v = x W + bias at element o before
+// What a GEMM does to each product v = x W + bias at element o before
 // it stores y[o]: v = silu(gate[o]) * v; v += res[o], each where its pointer is
 // set.  gate and res may be y itself (each element is read before it is
 // written, by the thread that writes it).
@@ -402,8 +404,12 @@ int64_t gemm_launch_ws_bytes(int bits, int64_t M, int64_t K, int64_t N, int mode
 // 4 the skinny MFMA kernel; ks the K splits (1: none).
 void linear_plan(int bits, int64_t M, int64_t K, int64_t N, int64_t group_size, int64_t cus, int* path, int* ks);
 int xcd_rect_rows(int64_t tm, int64_t tn, int64_t xb, int64_t wb, int64_t xcds);
+// gemm_i8_epilogue: whether the launch of this shape takes gate and res (k_gemm3
+// without a K split does not: the branches cost it 1%).
+bool gemm_i8_epilogue(const float* x, int64_t M, int64_t K, int64_t N, int64_t cus);
 hipError_t launch_gemm_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* scales,
-                          bool per_tensor, const float* bias, float* y, void* ws, hipStream_t s);
+                          bool per_tensor, const float* bias, const GemmEpilogue& ep, float* y, void* ws,
+                          hipStream_t s);
 // nw (1..3) weights of one shape on one input: weight w writes y + w * M * N.
 // ws: gemm_workspace_bytes(M, K, nw * N) bytes.
 hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
@@ -419,10 +425,13 @@ struct GemmWaveShape {
     int64_t rows() const { return (sk == 1 ? 2 : 1) * 16 * rb; }
     int64_t cols() const { return (sk == 4 ? 1 : 2) * 128; }
 };
-inline bool gemm_wave_takes(int spc) { return spc % 4 == 0; }
-GemmWaveShape gemm_wave_shape(int64_t M, int64_t N, int spc, int KS, int64_t cus);
-hipError_t launch_gemm_wave(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
-                            const float* const* devscales, const float* const* bias, const I4Geom& g, const GemmPlan& p,
+inline bool gemm_wave_takes(int bits, int spc) { return bits == 8 || spc % 4 == 0; }
+// one_scale: a wavefront's 128 columns share their scales.
+GemmWaveShape gemm_wave_shape(int64_t M, int64_t N, bool one_scale, int KS, int64_t cus);
+// mode: INT8 the per-tensor flag, INT4 strips per scale column; scales: INT4
+// the device scales.
+hipError_t launch_gemm_wave(int bits, const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
+                            const float* const* scales, const float* const* bias, int mode, const GemmPlan& p,
                             const GemmWaveShape& w, const GemmEpilogue& ep, float* y, void* ws, hipStream_t s);
 // y of nw weights: the sum of the KS partial results in part ([nw][KS][M][N]),
 // in split order, with bias and epilogue.
@@ -434,8 +443,9 @@ hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N
 // Gated MLP: h = silu(x*Wg + bg) * (x*Wu + bu).  The GEMV form (M <= kGemvMaxM)
 // runs both weights in one launch (as does the skinny kernel, launch_skinny_i4
 // with ng == 2); GEMM batches run two projections, the second with the first
-// as its epilogue's gate; the INT8 skinny kernel and the flat INT4 layout two
-// projections and launch_silu_mul (h = silu(h) * u, elementwise over n floats).
+// as its epilogue's gate (as does the INT8 skinny kernel); an INT8 GEMM without
+// a K split and the flat INT4 layout two projections and launch_silu_mul
+// (h = silu(h) * u, elementwise over n floats).
 hipError_t launch_swiglu_gemv_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed_g,
                                  const float* scales_g, const float* bias_g, const void* packed_u,
                                  const float* scales_u, const float* bias_u, bool per_tensor, float* h,

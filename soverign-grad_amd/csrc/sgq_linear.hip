@@ -153,7 +153,7 @@ inline GemvHot gemv_hot(const GemvArgs& a, int bits) {
 // accumulates (x * gamma * s) * q and sum(x^2) of the x rows it reads anyway
 // (all of K), and multiplies by inv_rms in the epilogue.  No separate norm
 // launch and no normed copy of x.
-template <int BITS, int MT, int NW, int U, bool KALIGN4, int NG, int SPW, bool NORM, bool STREAM>
+template <int BITS, int MT, int NW, int U, int NG, int SPW, bool NORM, bool STREAM>
 __global__ __launch_bounds__(NG * NW * 64) void k_gemv(const float* __restrict__ hx, const uint4* __restrict__ hW0,
                                                        const float* __restrict__ hS0, int K, int RQ, int NS, int hM,
                                                        int nblk, int pk, uint32_t spcm, const GemvArgs a) {
@@ -246,13 +246,13 @@ __global__ __launch_bounds__(NG * NW * 64) void k_gemv(const float* __restrict__
             for (int s = 0; s < SPW; ++s)
                 w[u][s] = STREAM ? buf_load16_stream(rW[s], voff, soff) : buf_load16(rW[s], voff, soff);
             if constexpr (BITS == 4) {
-                sv[u] = buf_load4f<true>(rS, voff, soff);  // devscales rows are padded to 16
+                sv[u] = buf_load4f(rS, voff, soff);  // devscales rows are padded to 16
             } else if (!mode) {
-                sv[u] = buf_load4f<KALIGN4>(rS, voff, soff);
+                sv[u] = buf_load4f(rS, voff, soff);
             }
 #pragma unroll
-            for (int m = 0; m < MT; ++m) xv[u][m] = buf_load4f<KALIGN4>(rX[m], voff, soff);
-            if constexpr (NORM) gv[u] = buf_load4f<KALIGN4>(rG, voff, soff);
+            for (int m = 0; m < MT; ++m) xv[u][m] = buf_load4f(rX[m], voff, soff);
+            if constexpr (NORM) gv[u] = buf_load4f(rG, voff, soff);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -478,7 +478,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int k = kt * kBK + kq * 4;
             const int vo = (row * K + kq * 4) * 4;
             if (KALIGN4) {
-                rg.a[i] = buf_load4f<true>(rX, k < K ? vo : kOobOff, soffA);
+                rg.a[i] = buf_load4f(rX, k < K ? vo : kOobOff, soffA);
             } else {
                 float t[4];
 #pragma unroll
@@ -514,7 +514,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int jc = bj < NS ? bj : NS - 1;
             // devscales rows stop at Kpad (codes there are zero); the
             // 1/16 turns the 16*q read of a high nibble back into q (exact)
-            const float4 s4 = buf_load4f<true>(rS, k < Kpad ? ((jc / mode) * Kpad + kl) * 4 : kOobOff,
+            const float4 s4 = buf_load4f(rS, k < Kpad ? ((jc / mode) * Kpad + kl) * 4 : kOobOff,
                                                kt * kBK * 4);
             const float sc[4] = {s4.x * 0.0625f, s4.y * 0.0625f, s4.z * 0.0625f, s4.w * 0.0625f};
             uint32_t lo[4], hi[4];
@@ -665,7 +665,7 @@ struct Gemm3Args {
     int xr, xlog;
 };
 
-template <bool KALIGN4, bool PT, class SH>
+template <bool PT, class SH>
 __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE))) void k_gemm3(const Gemm3Args ga) {
     const float* __restrict__ x = ga.x;
     const int M = ga.M, K = ga.K, N = ga.N;
@@ -742,20 +742,11 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const int vo = ((ar + kStep * h) * K + akg * 8 + 4 * q) * 4;
-                if (KALIGN4) {
-                    rg.a[h][q] = buf_load4f<true>(rX, kb + 4 * q < K ? vo : kOobOff, soff);
-                } else {
-                    float t[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        t[r] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                            rX, kb + 4 * q + r < K ? vo + 4 * r : kOobOff, soff, 0));
-                    rg.a[h][q] = make_float4(t[0], t[1], t[2], t[3]);
-                }
+                rg.a[h][q] = buf_load4f(rX, kb + 4 * q < K ? vo : kOobOff, soff);
             }
         if constexpr (!PT) {
 #pragma unroll
-            for (int q = 0; q < 2; ++q) rg.s[q] = buf_load4f<KALIGN4>(rS, (akg * 8 + 4 * q) * 4, soff);
+            for (int q = 0; q < 2; ++q) rg.s[q] = buf_load4f(rS, (akg * 8 + 4 * q) * 4, soff);
         }
         // RQ is a multiple of 4, so both row quads of the pair are in or out together.
         const bool in = kt * kB3RQ + 2 * akg < RQ;
@@ -967,8 +958,9 @@ __device__ __forceinline__ FastDiv fastdiv_of(uint32_t m, int l) {
 // k block.  NG == 2:
 // the gated MLP, h = silu(gate + bias) * (up + bias2).  NG == 1 runs a.wgpw
 // workgroups per weight over nw weights of one shape side by side (a LLaMA
-// block's q, k and v).  XA: x rows are 16-byte aligned and K % 4 == 0 (float4
-// loads); otherwise one float per load.
+// block's q, k and v).  x rows are loaded four floats at a time whatever K and
+// their alignment; the last quad of a row may hold floats of the next one,
+// which the zero scales past K remove.
 //
 // NORM: the input rows are RMS-normalised first (rms_norm, src/ops.cpp:
 // 1532-1556: x * inv_rms * gamma, inv_rms = 1 / sqrt(sum(x^2) / K + eps)), as
@@ -980,7 +972,7 @@ __device__ __forceinline__ FastDiv fastdiv_of(uint32_t m, int l) {
 // n + 8 k 8g + 4 .. 8g + 7 of the same row, and a row_ror:8 exchange gives
 // lane n the upper half of its operand.  The bf16 planes are the same bits as
 // without HALF; A rows 8..15 then hold copies whose outputs are never read.
-template <int NW, int U, int C, int NG, bool XA, bool NORM, bool HALF>
+template <int NW, int U, int C, int NG, bool NORM, bool HALF>
 __global__ __launch_bounds__(NW * 64) void k_skinny3(SGQ_SKINNY_HOT_PARAMS, const SkinnyArgs a) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, n = lane & 15;
@@ -1045,23 +1037,16 @@ __global__ __launch_bounds__(NW * 64) void k_skinny3(SGQ_SKINNY_HOT_PARAMS, cons
 #pragma unroll
             for (int h = 0; h < XV / 4; ++h) {
                 const int kk = k0 + 4 * h;
-                if constexpr (XA) {
-                    const float4 xq = buf_load4f<true>(rX, row_live && kk < K ? xrow + kk * 4 : kOobOff, 0);
-                    xv[u][4 * h] = xq.x, xv[u][4 * h + 1] = xq.y, xv[u][4 * h + 2] = xq.z, xv[u][4 * h + 3] = xq.w;
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        xv[u][4 * h + i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                            rX, row_live && kk + i < K ? xrow + (kk + i) * 4 : kOobOff, 0, 0));
-                }
+                const float4 xq = buf_load4f(rX, row_live && kk < K ? xrow + kk * 4 : kOobOff, 0);
+                xv[u][4 * h] = xq.x, xv[u][4 * h + 1] = xq.y, xv[u][4 * h + 2] = xq.z, xv[u][4 * h + 3] = xq.w;
 #pragma unroll
                 for (int q = 0; q < NG; ++q) {
-                    const float4 s4 = buf_load4f<true>(rS[q], kk * 4, 0);
+                    const float4 s4 = buf_load4f(rS[q], kk * 4, 0);
                     sv[u][q][4 * h] = s4.x, sv[u][q][4 * h + 1] = s4.y, sv[u][q][4 * h + 2] = s4.z,
                                  sv[u][q][4 * h + 3] = s4.w;
                 }
                 if constexpr (NORM) {
-                    const float4 g4 = buf_load4f<XA>(rG, kk * 4, 0);
+                    const float4 g4 = buf_load4f(rG, kk * 4, 0);
                     gv[u][4 * h] = g4.x, gv[u][4 * h + 1] = g4.y, gv[u][4 * h + 2] = g4.z, gv[u][4 * h + 3] = g4.w;
                 }
             }
@@ -1171,8 +1156,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny3(SGQ_SKINNY_HOT_PARAMS, cons
 
 // The super-block form (any row blocks, optional K split).  NG == 2: the gated MLP, gate and up blocks of the same columns in one
 // workgroup, h = silu(gate + bias) * (up + bias2) (split K: in
-// k_skinny_reduce).  XA: x rows are 16-byte aligned and K % 4 == 0 (float4
-// loads); otherwise one float per load.  MB: row blocks of 16 (M <= 16 MB).
+// k_skinny_reduce).  MB: row blocks of 16 (M <= 16 MB).
 //
 // The K range is walked in super-blocks of 128 rows, wavefront w taking
 // super-blocks w, w + NW, ...  A super-block is four k blocks of 32 rows of
@@ -1184,7 +1168,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny3(SGQ_SKINNY_HOT_PARAMS, cons
 // scales of the workgroup's K range sit in LDS (read once, coalesced); the
 // next super-block's codes and x are loaded while the current one is
 // computed.
-template <int NW, int C, int NG, bool XA, int MB, bool HALF>
+template <int C, int NG, int MB, bool HALF>
 struct SkinnyRegs {
     uint4 w[NG][C];                // dword i: the B operand of k block i
     float4 xq[MB][HALF ? 4 : 8];  // x quads of each batch row (HALF: half of them)
@@ -1198,7 +1182,7 @@ struct SkinnyRegs {
 //
 // MULTI (NG == 1): a.wgpw column groups per weight over nw weights of one
 // shape side by side, as k_skinny3.
-template <int NW, int C, int NG, bool XA, int MB, bool SPLIT, bool HALF, bool MULTI>
+template <int NW, int C, int NG, int MB, bool SPLIT, bool HALF, bool MULTI>
 __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, const SkinnyArgs a) {
     static_assert(!HALF || MB == 1, "the half-row form has one row block");
     static_assert(!MULTI || NG == 1, "weights side by side are plain projections");
@@ -1243,7 +1227,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
 #pragma unroll
         for (int it = 0; it < SCI; ++it) {
             const int r4 = threadIdx.x + it * NW * 64;
-            sreg[q][it] = buf_load4f<true>(rS, r4 < rows4 ? (row0 + 4 * r4) * 4 : kOobOff, 0);
+            sreg[q][it] = buf_load4f(rS, r4 < rows4 ? (row0 + 4 * r4) * 4 : kOobOff, 0);
         }
     }
 
@@ -1270,7 +1254,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
 
     // Loads of super-block sb; one past the range reads x as zeros (and codes
     // that are then multiplied by zero).
-    auto load = [&](SkinnyRegs<NW, C, NG, XA, MB, HALF>& r, int sb) {
+    auto load = [&](SkinnyRegs<C, NG, MB, HALF>& r, int sb) {
         const bool in = sb < sb_hi;
 #pragma unroll
         for (int q = 0; q < NG; ++q)
@@ -1285,19 +1269,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
 #pragma unroll
             for (int t = 0; t < XT; ++t) {
                 const int kk = sb * kSkinnySB + qrow(t);
-                if constexpr (XA) {
-                    r.xq[b][t] = buf_load4f<true>(rX, in && row_live[b] && kk < K ? xrow[b] + kk * 4 : kOobOff, 0);
-                } else {
-                    // One float per load from any 4-byte address; the row's
-                    // tail and the rows past M read as zeros by their offset.
-                    const int base = in && row_live[b] ? xrow[b] + kk * 4 : kOobOff;
-                    float f[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        f[i] = __uint_as_float(
-                            __builtin_amdgcn_raw_buffer_load_b32(rX, kk + i < K ? base + 4 * i : kOobOff, 0, 0));
-                    r.xq[b][t] = make_float4(f[0], f[1], f[2], f[3]);
-                }
+                r.xq[b][t] = buf_load4f(rX, in && row_live[b] && kk < K ? xrow[b] + kk * 4 : kOobOff, 0);
             }
     };
 
@@ -1309,7 +1281,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
 #pragma unroll
             for (int c = 0; c < C; ++c) acc[q][b][c] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    auto compute = [&](SkinnyRegs<NW, C, NG, XA, MB, HALF>& r, int sb) {
+    auto compute = [&](SkinnyRegs<C, NG, MB, HALF>& r, int sb) {
         // A super-block past the range has x = 0; its scale reads stay inside
         // the range's LDS rows.
         const int lr = (min(sb, sb_hi - 1) - sb_lo) * (kSkinnySB / 4);
@@ -1362,7 +1334,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
 
     // Two register sets: the loads of the next super-block are in flight
     // while the current one is computed.
-    SkinnyRegs<NW, C, NG, XA, MB, HALF> ra, rb;
+    SkinnyRegs<C, NG, MB, HALF> ra, rb;
     int sb = sb_lo + wave;
     load(ra, sb);
 #pragma unroll
@@ -1475,6 +1447,7 @@ struct Skinny8Args {
     int RQ, NS, Kpad;
     int ncg;      // column groups (workgroups per row tile)
     FastDiv cgd;  // division by ncg
+    const float* gate;  // y = silu(gate) * (x W + bias), or null; may be y
     float* y;
     int nblk;
     int xlog;  // log2 of the device's XCD count
@@ -1503,7 +1476,7 @@ inline Skinny8Hot skinny8_hot(const Skinny8Args& a) {
 // HALF (one row block, M <= 8): lane n < 8 loads and splits k 8g .. 8g + 3
 // of row n, lane n + 8 k 8g + 4 .. 8g + 7 of the same row, and a row_ror:8
 // exchange completes each A operand (the same bf16 planes), as in k_skinny3.
-template <int NW, int U, int C, int MB, bool PT, bool XA, bool HALF>
+template <int NW, int U, int C, int MB, bool PT, bool HALF>
 __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ hx, const uint4* __restrict__ hW,
                                                         const float* __restrict__ hS, int hM, int K, int RQ, int NS,
                                                         int nblk, int pk, uint32_t cgdm, int ncg,
@@ -1556,19 +1529,14 @@ __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ h
 #pragma unroll
                 for (int b = 0; b < MB; ++b) {
                     const int xo = (16 * b + xr) * K * 4;
-                    if constexpr (XA) {
-                        const float4 xq = buf_load4f<true>(rX, kk < K ? xo + kk * 4 : kOobOff, 0);
-                        xv[u][b][4 * h] = xq.x, xv[u][b][4 * h + 1] = xq.y, xv[u][b][4 * h + 2] = xq.z,
-                                     xv[u][b][4 * h + 3] = xq.w;
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            xv[u][b][4 * h + i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                                rX, kk + i < K ? xo + (kk + i) * 4 : kOobOff, 0, 0));
-                    }
+                    // The last quad of a row may hold floats of the next one: the
+                    // codes past K are zero.
+                    const float4 xq = buf_load4f(rX, kk < K ? xo + kk * 4 : kOobOff, 0);
+                    xv[u][b][4 * h] = xq.x, xv[u][b][4 * h + 1] = xq.y, xv[u][b][4 * h + 2] = xq.z,
+                                 xv[u][b][4 * h + 3] = xq.w;
                 }
                 if constexpr (!PT) {
-                    const float4 sq = buf_load4f<XA>(rS, kk * 4, 0);
+                    const float4 sq = buf_load4f(rS, kk * 4, 0);
                     sv[u][4 * h] = sq.x, sv[u][4 * h + 1] = sq.y, sv[u][4 * h + 2] = sq.z, sv[u][4 * h + 3] = sq.w;
                 }
             }
@@ -1642,7 +1610,10 @@ __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ h
             // h + m + l turns an infinite x into inf - inf: recompute a
             // non-finite total as the reference's k-order sum.
             if (!isfinite(s)) s = output_exact<8>(a.x + (int64_t)m * K, a.W, a.S, PT ? 1 : 0, a.Kpad, a.RQ, col, 0, K);
-            a.y[(int64_t)m * a.N + col] = a.bias ? s + a.bias[col] : s;
+            const int64_t o = (int64_t)m * a.N + col;
+            if (a.bias) s = s + a.bias[col];
+            if (a.gate) s = silu_f32(a.gate[o]) * s;
+            a.y[o] = s;
         }
     }
 }
@@ -1705,21 +1676,14 @@ hipError_t gemv_launch_st(const GemvArgs& a, int nw, hipStream_t s) {
     ag.nblk = (int)grid.x;
     if (a.Kpad != 4 * a.RQ || a.Plog > 255 || a.xlog > 255) return hipErrorInvalidValue;  // GemvHot's packing
     const GemvHot h = gemv_hot(ag, BITS);
-    const bool k4 = a.K % 4 == 0;
     if constexpr (BITS == 4 && SPW == 1) {  // the norm-fused form serves the INT4 LLaMA block
         if (a.gamma) {
-            if (k4)
-                k_gemv<BITS, MT, NW, U, true, NG, SPW, true, STREAM><<<grid, NG * NW * 64, 0, s>>>(SGQ_GEMV_HOT_ARGS(h, ag));
-            else
-                k_gemv<BITS, MT, NW, U, false, NG, SPW, true, STREAM><<<grid, NG * NW * 64, 0, s>>>(SGQ_GEMV_HOT_ARGS(h, ag));
+            k_gemv<BITS, MT, NW, U, NG, SPW, true, STREAM><<<grid, NG * NW * 64, 0, s>>>(SGQ_GEMV_HOT_ARGS(h, ag));
             return hipGetLastError();
         }
     }
     if (a.gamma) return hipErrorInvalidValue;
-    if (k4)
-        k_gemv<BITS, MT, NW, U, true, NG, SPW, false, STREAM><<<grid, NG * NW * 64, 0, s>>>(SGQ_GEMV_HOT_ARGS(h, ag));
-    else
-        k_gemv<BITS, MT, NW, U, false, NG, SPW, false, STREAM><<<grid, NG * NW * 64, 0, s>>>(SGQ_GEMV_HOT_ARGS(h, ag));
+    k_gemv<BITS, MT, NW, U, NG, SPW, false, STREAM><<<grid, NG * NW * 64, 0, s>>>(SGQ_GEMV_HOT_ARGS(h, ag));
     return hipGetLastError();
 }
 #undef SGQ_GEMV_HOT_ARGS
@@ -1884,7 +1848,7 @@ constexpr int kSkinnyWholeKWaves = 16;
 
 // One k_skinny3 launch (and, with split K, its reduce) for the plan's C and
 // MB; NG weights of equal shape with their devscales and biases.
-template <int C, int NG, int MB, bool XA>
+template <int C, int NG, int MB>
 hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const void* const* packed,
                          const float* const* devscales, const float* const* bias, const I4Geom& g, int form, int S,
                          float* y, float* part, const SkinnyExtra& ex, hipStream_t s) {
@@ -1933,9 +1897,9 @@ hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const 
             const SkinnyHot h = skinny_hot(a);
 #define SGQ_SKINNY3(NORM_)                                                                                 \
     if (M <= 8)                                                                                            \
-        k_skinny3<kSkinnyWholeKWaves, U, C, NG, XA, NORM_, true><<<a.nblk, kSkinnyWholeKWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a); \
+        k_skinny3<kSkinnyWholeKWaves, U, C, NG, NORM_, true><<<a.nblk, kSkinnyWholeKWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a); \
     else                                                                                                   \
-        k_skinny3<kSkinnyWholeKWaves, U, C, NG, XA, NORM_, false><<<a.nblk, kSkinnyWholeKWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a);
+        k_skinny3<kSkinnyWholeKWaves, U, C, NG, NORM_, false><<<a.nblk, kSkinnyWholeKWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a);
             if (ex.gamma) {
                 // The norm-fused form keeps two column blocks (register budget).
                 if constexpr (C == 2) {
@@ -1955,12 +1919,11 @@ hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const 
     a.nblk *= ex.nw;
     const SkinnyHot h = skinny_hot(a);
 #define SGQ_SKINNY_SB(SPLIT_, HALF_, MULTI_)                                                            \
-    k_skinny_sb<kSkinnyWaves, C, NG, XA, MB, SPLIT_, HALF_, MULTI_>                                     \
+    k_skinny_sb<kSkinnyWaves, C, NG, MB, SPLIT_, HALF_, MULTI_>                                     \
         <<<a.nblk, kSkinnyWaves * 64, 0, s>>>(SGQ_SKINNY_HOT_ARGS(h), a)
     if (ex.nw > 1) {
-        // Several weights: the LLaMA block's q, k and v of 17..32 sequences
-        // (their normed input is the library's own, 16-byte aligned).
-        if constexpr (NG == 1 && MB == 2 && XA) {
+        // Several weights: the LLaMA block's q, k and v of 17..32 sequences.
+        if constexpr (NG == 1 && MB == 2) {
             if (S > 1)
                 SGQ_SKINNY_SB(true, false, true);
             else
@@ -1998,34 +1961,24 @@ template <int NG>
 hipError_t skinny_dispatch(const SkinnyPlan& p, const float* x, int64_t M, int64_t K, int64_t N,
                            const void* const* packed, const float* const* devscales, const float* const* bias,
                            const I4Geom& g, float* y, float* part, const SkinnyExtra& ex, hipStream_t s) {
-    // The super-block form of the gated MLP, and two row blocks of
-    // unaligned x, keep two column blocks per workgroup, within the register
-    // budget (C does not change the order of any sum).
-    if (p.C != 2 && p.C != 4) return hipErrorInvalidValue;
-#define SGQ_SKINNY(C_, MB_, XA_) \
-    return skinny_launch<C_, NG, MB_, XA_>(x, M, K, N, packed, devscales, bias, g, p.form, p.S, y, part, ex, s)
-    const bool xa = x_aligned4(x, K);
-    // The norm-fused form runs two column blocks per workgroup (C does not
+    // The super-block form of the gated MLP and the norm-fused form keep two
+    // column blocks per workgroup, within the register budget (C does not
     // change the order of any sum).
-    if (p.C == 4 && p.MB == 1 && (NG == 1 || p.form == 0) && !ex.gamma) {
-        if (xa) SGQ_SKINNY(4, 1, true);
-        SGQ_SKINNY(4, 1, false);
-    }
+    if (p.C != 2 && p.C != 4) return hipErrorInvalidValue;
+#define SGQ_SKINNY(C_, MB_) \
+    return skinny_launch<C_, NG, MB_>(x, M, K, N, packed, devscales, bias, g, p.form, p.S, y, part, ex, s)
+    if (p.C == 4 && p.MB == 1 && (NG == 1 || p.form == 0) && !ex.gamma) SGQ_SKINNY(4, 1);
     if constexpr (NG == 1) {
-        if (p.C == 4 && xa && !ex.gamma) SGQ_SKINNY(4, 2, true);
+        if (p.C == 4 && p.MB == 2 && !ex.gamma) SGQ_SKINNY(4, 2);
     }
-    if (p.MB == 1) {
-        if (xa) SGQ_SKINNY(2, 1, true);
-        SGQ_SKINNY(2, 1, false);
-    }
-    if (xa) SGQ_SKINNY(2, 2, true);
-    SGQ_SKINNY(2, 2, false);
+    if (p.MB == 1) SGQ_SKINNY(2, 1);
+    SGQ_SKINNY(2, 2);
 #undef SGQ_SKINNY
 }
 
-template <int C, int MB, bool PT, bool XA>
+template <int C, int MB, bool PT>
 hipError_t skinny8_launch(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* scales,
-                          const float* bias, float* y, hipStream_t s) {
+                          const float* bias, const float* gate, float* y, hipStream_t s) {
     const I8Geom g(K, N);
     Skinny8Args a{};
     a.x = x;
@@ -2040,6 +1993,7 @@ hipError_t skinny8_launch(const float* x, int64_t M, int64_t K, int64_t N, const
     a.Kpad = (int)g.Kpad;
     a.ncg = (int)ceil_div(g.NS, 4 * C);
     a.cgd = FastDiv((uint32_t)a.ncg);
+    a.gate = gate;
     a.y = y;
     a.nblk = (int)(ceil_div(M, 16 * MB) * a.ncg);
     a.xlog = xcd_log2(device_xcds(s));
@@ -2047,25 +2001,21 @@ hipError_t skinny8_launch(const float* x, int64_t M, int64_t K, int64_t N, const
     if (g.Kpad != 4 * g.RQ) return hipErrorInvalidValue;  // Skinny8Hot carries RQ only
     const Skinny8Hot h = skinny8_hot(a);
     if (MB == 1 && M <= 8)
-        k_skinny8<kSkinnyWholeKWaves, U, C, MB, PT, XA, MB == 1><<<a.nblk, kSkinnyWholeKWaves * 64, 0, s>>>(h.x, h.W, h.S, h.M, h.K, h.RQ, h.NS, h.nblk, h.pk, h.cgdm, h.ncg, a);
+        k_skinny8<kSkinnyWholeKWaves, U, C, MB, PT, MB == 1><<<a.nblk, kSkinnyWholeKWaves * 64, 0, s>>>(h.x, h.W, h.S, h.M, h.K, h.RQ, h.NS, h.nblk, h.pk, h.cgdm, h.ncg, a);
     else
-        k_skinny8<kSkinnyWholeKWaves, U, C, MB, PT, XA, false><<<a.nblk, kSkinnyWholeKWaves * 64, 0, s>>>(h.x, h.W, h.S, h.M, h.K, h.RQ, h.NS, h.nblk, h.pk, h.cgdm, h.ncg, a);
+        k_skinny8<kSkinnyWholeKWaves, U, C, MB, PT, false><<<a.nblk, kSkinnyWholeKWaves * 64, 0, s>>>(h.x, h.W, h.S, h.M, h.K, h.RQ, h.NS, h.nblk, h.pk, h.cgdm, h.ncg, a);
     return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_skinny_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* scales,
-                            bool per_tensor, const float* bias, const Skinny8Plan& p, float* y, hipStream_t s) {
-    const bool xa = x_aligned4(x, K);
-#define SGQ_SKINNY8(C_, MB_)                                                                      \
-    if (p.C == C_ && p.MB == MB_) {                                                                \
-        if (per_tensor)                                                                           \
-            return xa ? skinny8_launch<C_, MB_, true, true>(x, M, K, N, packed, scales, bias, y, s)  \
-                      : skinny8_launch<C_, MB_, true, false>(x, M, K, N, packed, scales, bias, y, s); \
-        return xa ? skinny8_launch<C_, MB_, false, true>(x, M, K, N, packed, scales, bias, y, s)     \
-                  : skinny8_launch<C_, MB_, false, false>(x, M, K, N, packed, scales, bias, y, s);   \
-    }
+                            bool per_tensor, const float* bias, const float* gate, const Skinny8Plan& p, float* y,
+                            hipStream_t s) {
+#define SGQ_SKINNY8(C_, MB_)                                                                       \
+    if (p.C == C_ && p.MB == MB_)                                                                  \
+        return per_tensor ? skinny8_launch<C_, MB_, true>(x, M, K, N, packed, scales, bias, gate, y, s)  \
+                          : skinny8_launch<C_, MB_, false>(x, M, K, N, packed, scales, bias, gate, y, s);
     SGQ_SKINNY8(1, 1)
     SGQ_SKINNY8(2, 1)
     SGQ_SKINNY8(4, 1)
@@ -2329,8 +2279,8 @@ int gemm_rect_rows(int bits, int64_t M, int64_t K, int64_t N, int mode, int64_t 
     if (gemm_plan(M, K, N, t, cus).KS != 1) return 0;
     int64_t bm = t.bm, bn = t.bn;
     if (bits == 4) {
-        if (!gemm_wave_takes(mode)) return 0;  // the fp32 kernel keeps the plain order
-        const GemmWaveShape w = gemm_wave_shape(M, N, mode, 1, cus);
+        if (!gemm_wave_takes(4, mode)) return 0;  // the fp32 kernel keeps the plain order
+        const GemmWaveShape w = gemm_wave_shape(M, N, mode % 16 == 0, 1, cus);
         bm = w.rows(), bn = w.cols();
     }
     return xcd_rect_rows(ceil_div(M, bm), ceil_div(N, bn), bm * K * 4, bn * K * bits / 8, xcds);
@@ -2340,20 +2290,21 @@ namespace {
 
 // The three-term INT8 GEMM (k_gemm3) on the tile gemm_tile gives the batch.
 template <class SH>
-void gemm3_launch(const Gemm3Args& a, unsigned grid, bool k4, bool pt, hipStream_t s) {
-    if (k4 && pt)
-        k_gemm3<true, true, SH><<<grid, SH::NT, 0, s>>>(a);
-    else if (k4)
-        k_gemm3<true, false, SH><<<grid, SH::NT, 0, s>>>(a);
-    else if (pt)
-        k_gemm3<false, true, SH><<<grid, SH::NT, 0, s>>>(a);
+void gemm3_launch(const Gemm3Args& a, unsigned grid, bool pt, hipStream_t s) {
+    if (pt)
+        k_gemm3<true, SH><<<grid, SH::NT, 0, s>>>(a);
     else
-        k_gemm3<false, false, SH><<<grid, SH::NT, 0, s>>>(a);
+        k_gemm3<false, SH><<<grid, SH::NT, 0, s>>>(a);
 }
 }  // namespace
 
+bool gemm_i8_epilogue(const float* x, int64_t M, int64_t K, int64_t N, int64_t cus) {
+    return !x_aligned4(x, K) || gemm_plan(M, K, N, gemm_tile(8, M), cus).KS > 1;
+}
+
 hipError_t launch_gemm_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* scales,
-                          bool per_tensor, const float* bias, float* y, void* ws, hipStream_t s) {
+                          bool per_tensor, const float* bias, const GemmEpilogue& ep, float* y, void* ws,
+                          hipStream_t s) {
     const I8Geom g(K, N);
     const GemmTile t = gemm_tile(8, M);
     const GemmPlan p = gemm_plan(M, K, N, t, device_cus(s));
@@ -2372,15 +2323,28 @@ hipError_t launch_gemm_i8(const float* x, int64_t M, int64_t K, int64_t N, const
     a.xr = p.KS == 1 ? xcd_rect_rows(tm, tn, t.bm * K * 4, t.bn * K, xcds) : 0;
     a.xlog = xcd_log2(xcds);
     const unsigned grid = (unsigned)(tm * tn * p.KS);
-    const bool k4 = x_aligned4(x, K);
-    if (t.bm == 32)
-        gemm3_launch<G3Rows32>(a, grid, k4, per_tensor, s);
-    else if (t.bm == 64)
-        gemm3_launch<G3Rows64>(a, grid, k4, per_tensor, s);
-    else
-        gemm3_launch<G3Wide>(a, grid, k4, per_tensor, s);
-    const hipError_t e = hipGetLastError();
-    return e != hipSuccess || p.KS == 1 ? e : launch_splitk_reduce(a.part, p.KS, M, N, 1, &bias, {}, y, s);
+    hipError_t e = hipSuccess;
+    if (!x_aligned4(x, K)) {
+        // Rows of x at any 4-byte address: the wavefront tiles' loads do not
+        // care, this kernel's would be one float each.  Measured (us, one float
+        // per load -> wavefront tiles): 2048 x 4097 -> 4096 257 -> 183, 2048 x
+        // 1001 -> 11008 229 -> 137, 64 x 4097 -> 11008 per channel 60 -> 34.5, 130
+        // x 777 -> 1000 24 -> 12.  Aligned rows stay here (2048 x 4096 -> 4096 162
+        // against 187: both run at the power limit, and this kernel converts
+        // each code and splits each x for a whole 128 x 256 tile).
+        e = launch_gemm_wave(8, x, M, K, N, 1, &packed, &scales, &bias, per_tensor ? 1 : 0, p,
+                             gemm_wave_shape(M, N, true, p.KS, device_cus(s)), ep, y, ws, s);
+    } else {
+        if (p.KS == 1 && (ep.gate || ep.res)) return hipErrorInvalidValue;  // gemm_i8_epilogue
+        if (t.bm == 32)
+            gemm3_launch<G3Rows32>(a, grid, per_tensor, s);
+        else if (t.bm == 64)
+            gemm3_launch<G3Rows64>(a, grid, per_tensor, s);
+        else
+            gemm3_launch<G3Wide>(a, grid, per_tensor, s);
+        e = hipGetLastError();
+    }
+    return e != hipSuccess || p.KS == 1 ? e : launch_splitk_reduce(a.part, p.KS, M, N, 1, &bias, ep, y, s);
 }
 
 hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
@@ -2390,9 +2354,9 @@ hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, int n
     // Several weights side by side plan their splits as one of the total width.
     const GemmPlan p = gemm_plan(M, K, nw * N, gemm_i4_tile(M, (int)g.spc), cus);
     hipError_t e = hipSuccess;
-    if (gemm_wave_takes((int)g.spc)) {
-        e = launch_gemm_wave(x, M, K, N, nw, packed, devscales, bias, g, p,
-                             gemm_wave_shape(M, nw * N, (int)g.spc, p.KS, cus), ep, y, ws, s);
+    if (gemm_wave_takes(4, (int)g.spc)) {
+        e = launch_gemm_wave(4, x, M, K, N, nw, packed, devscales, bias, (int)g.spc, p,
+                             gemm_wave_shape(M, nw * N, g.spc % 16 == 0, p.KS, cus), ep, y, ws, s);
     } else {
         const unsigned grid = (unsigned)(ceil_div(M, kBM) * ceil_div(N, kBN) * p.KS);
         for (int w = 0; w < nw && e == hipSuccess; ++w) {
