@@ -149,7 +149,7 @@ SkinnyPlan decode_skinny_plan(int64_t B, int64_t K, int64_t N, int nw, int64_t G
 // Past the GEMV batches the block's projections run the super-block form of
 // the skinny kernel where the forward's plan gives it for the total width (q,
 // k and v side by side; gate and up in one launch): 17..32 rows.  Measured for
-// 32 sequences of 2000 tokens, D = 2048, H = 5632: one block 219 us with it and
+// 32 sequences of 2000 tokens, D = 2048, H = 5632: one block 220 us with it and
 // the GEMMs' epilogues below, 275 with seven GEMMs (and their split-K sums)
 // and separate adds and silu.
 SkinnyPlan decode_rows_plan(int64_t B, int64_t K, int64_t N, int nw, int64_t G, int cus) {

@@ -57,6 +57,46 @@ __global__ __launch_bounds__(kBlock) void k_rms_norm(const float* __restrict__ x
     for (int64_t d = threadIdx.x; d < D; d += kBlock) orow[d] = (xr[d] * inv) * g[d];
 }
 
+// The same for rows of up to 1024 V floats, a multiple of four: each thread
+// keeps its V quads of x (and loads g under the sum) instead of reading the row
+// twice, one float at a time.  Latency-bound: 32 rows of 2048 5.8 -> 5.0 us
+// traced, one block step of 32 sequences (two norms) 220 -> 212 us, one row of a
+// model's last norm 6.5 -> 2.3.
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+template <int V>
+__global__ __launch_bounds__(kBlock) void k_rms_norm_row(const float* x, int D, const float* __restrict__ g, float eps,
+                                                         float* out) {
+    __shared__ float red[kBlock / 64];
+    const f32x4_u* xr = (const f32x4_u*)(x + (int64_t)blockIdx.x * D);
+    f32x4_u* orow = (f32x4_u*)(out + (int64_t)blockIdx.x * D);
+    f32x4_u v[V], w[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int q = threadIdx.x + i * kBlock;
+        v[i] = 4 * q < D ? xr[q] : f32x4_u{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int q = threadIdx.x + i * kBlock;
+        w[i] = 4 * q < D ? ((const f32x4_u*)g)[q] : f32x4_u{0.f, 0.f, 0.f, 0.f};
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss = fmaf(v[i][e], v[i][e], ss);
+    ss = block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float)D + eps);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int q = threadIdx.x + i * kBlock;
+        f32x4_u o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (v[i][e] * inv) * w[i][e];
+        if (4 * q < D) orow[q] = o;
+    }
+}
+
 // out[i, :] = w[(int)idx[i], :], or zeros for an id outside [0, V)
 // (embedding, src/ops.cpp:2624-2650: ids are fp32 values truncated to int).
 __global__ __launch_bounds__(kBlock) void k_embedding(const float* __restrict__ idx, const float* __restrict__ w,
@@ -364,7 +404,12 @@ __global__ __launch_bounds__(kBlock) void k_poison_rows(const int32_t* __restric
 hipError_t launch_rms_norm(const float* x, int64_t rows, int64_t D, const float* g, float eps, float* out,
                            hipStream_t s) {
     if (rows <= 0 || D <= 0) return hipSuccess;
-    k_rms_norm<<<(unsigned)rows, kBlock, 0, s>>>(x, D, g, eps, out);
+    if (D % 4 == 0 && D <= 2 * 4 * kBlock)
+        k_rms_norm_row<2><<<(unsigned)rows, kBlock, 0, s>>>(x, (int)D, g, eps, out);
+    else if (D % 4 == 0 && D <= 8 * 4 * kBlock)
+        k_rms_norm_row<8><<<(unsigned)rows, kBlock, 0, s>>>(x, (int)D, g, eps, out);
+    else
+        k_rms_norm<<<(unsigned)rows, kBlock, 0, s>>>(x, D, g, eps, out);
     return hipGetLastError();
 }
 
