@@ -27,7 +27,7 @@
 //
 // What bounds it: the power limit.  At 2048 x 4096 -> 11008 (g128) the MFMAs
 // run at 1.16 PFLOP/s (three times the 387 TFLOP/s of the product) with the
-// clock at 1.9 GHz; the large bf16 library product of the same box runs at
+// clock at 1.9 GHz; a large bf16 library product on the same card runs at
 // 1.2 PFLOP/s with the clock at 1.5-1.8 GHz.  Smaller groups are VALU-bound:
 // the split costs 208 VALU instructions per group, row block set and stage.
 // Measured on MI355X, previous kernels -> this (us): g128 2048 x 4096 -> 11008

@@ -14,12 +14,13 @@
 // of a strip are combined by a butterfly that halves the values each lane
 // carries at every step, the four wavefronts through LDS.
 //
-// Prefill path (M > 16): output tiles of 128 rows, K staged through LDS 32
-// rows at a time.  k_gemm3 runs the fp32 products on the bf16 matrix cores as
-// three exact bf16 products each (x * s split into three bf16 terms, codes
-// exact in bf16, fp32 accumulation); k_gemm (INT4 groups that are not a
-// multiple of 128) dequantizes codes on the way into LDS (code * scale, the
-// reference's own product) and feeds v_mfma_f32_16x16x4_f32.
+// Prefill path (M > 16): output tiles of up to 128 rows, K staged through LDS
+// 32 rows at a time.  k_gemm3 (INT8) runs the fp32 products on the bf16 matrix
+// cores as three exact bf16 products each (x * s split into three bf16 terms,
+// codes exact in bf16, fp32 accumulation), as k_gemm_wave does for INT4
+// (sgq_gemm.hip); k_gemm (INT4 scale columns of other than a multiple of four
+// strips) dequantizes codes on the way into LDS (code * scale, the reference's
+// own product) and feeds v_mfma_f32_16x16x4_f32.
 #include <atomic>
 #include <type_traits>
 
@@ -621,8 +622,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 // as the reference's x . (q * s) in k order, so infinities and NaNs land
 // where the reference puts them.
 //
-// Tiles (G3Shape): INT8 128x256 with eight wavefronts in 2x4, INT4 128x128
-// with four in 2x2; each wavefront owns 64x64 as 4x4 MFMA blocks.  One 32-k
+// Tiles (G3Shape): 128x256 with eight wavefronts in 2x4, each owning 64x64 as
+// 4x4 MFMA blocks (fewer rows for small batches).  One 32-k
 // stage per LDS buffer, double-buffered, global loads two stages ahead (as
 // k_gemm).  LDS entries are 16 bytes, eight consecutive k of one row (A
 // planes) or one column (B): one MFMA operand.  Per-tensor INT8 puts x itself
@@ -635,8 +636,7 @@ constexpr int kB3RQ = kB3BK / 4;    // row quads per stage
 // Tile shape: WM x WN wavefronts, each RB x CB blocks of 16x16 outputs, so
 // the tile is BM = 16 * RB * WM rows by BN = 16 * CB * WN columns.  A wider
 // tile splits each x value once for more columns (less split work per
-// MFMA); INT4 tiles are 128 columns, the width of one scale column at group
-// 128.
+// MFMA).
 template <int WM_, int RB_, int WN_, int CB_>
 struct G3Shape {
     static constexpr int WM = WM_, RB = RB_, WN = WN_, CB = CB_;
