@@ -267,8 +267,9 @@ int sgq_linear_int4_noalloc(const float* x, int64_t M, int64_t K, int64_t N, con
  * runs on the GEMV or on the INT4 skinny MFMA kernel (above), with the tiled
  * layout, run both weights in one launch (x read once per strip pair, no
  * intermediate in HBM; a split K adds its reduce kernel); otherwise two
- * projections (the INT8 skinny kernel, the GEMM or flat INT4) and an
- * elementwise kernel, so that the sums are those of two forward calls.
+ * projections (the INT8 skinny kernel, the GEMM or flat INT4), the product
+ * taken in the second one's epilogue or by an elementwise kernel, so that the
+ * sums are those of two forward calls.
  * Biases may be NULL.  workspace:
  * sgq_swiglu_workspace_bytes(bits, M, K, N, group_size) bytes (group_size is
  * ignored for bits 8), else SGQ_ERR_WORKSPACE. */
@@ -340,7 +341,9 @@ int64_t sgq_llama_decode_workspace_bytes(int64_t B, int64_t D, int64_t H, int64_
  * launch; the RMSNorms folded in; the residual adds in the epilogues), except
  * that 5..16 rows run the norm-fused q/k/v and gate/up launches on the skinny
  * bf16 MFMA kernel where its plan takes the projection's total width (e.g.
- * the NanoLLaMA shape); larger B on the MFMA GEMM.  fp32 results throughout;
+ * the NanoLLaMA shape); larger B on the skinny kernel's super-block form where
+ * its plan takes the shape (17..32 rows), else the MFMA GEMM, the residual adds
+ * in the epilogues.  fp32 results throughout;
  * outputs match the reference's full-sequence forward within 1e-5 relative. */
 int sgq_llama_block_decode_int4(const sgq_llama_block_int4* block, const float* x, float* out, int64_t B,
                                 float* k_cache, float* v_cache, int64_t max_tokens, const int32_t* pos,

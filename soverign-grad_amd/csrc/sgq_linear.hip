@@ -615,7 +615,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 //   - a bf16 x bf16 product is exact in fp32, and v_mfma_f32_16x16x32_bf16
 //     sums into an fp32 accumulator, so acc += h.q, m.q and l.q (three MFMAs
 //     per 16x16x32 block) computes sum(xs * q) with fp32 accumulation.
-//     (Measured on the box: a 32-term dot product of split fp32 values and
+//     (Measured: a 32-term dot product of split fp32 values and
 //     codes came out within 5e-9 of fp64, against 1.6e-8 for an fp32 FMA chain.)
 // An output whose total is not finite (an infinite or NaN input, or an
 // overflow, where h + m + l would be inf - inf) is recomputed by its thread
