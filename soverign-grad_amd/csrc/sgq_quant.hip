@@ -115,16 +115,20 @@ enum PackFrom { kFromX, kFromXInv, kFromCodes };
 // g32 186 -> 32, g24 (scales found first) 208 -> 137; INT8 4096 x 4096 per
 // tensor 141 -> 67, 4096 x 4097 per channel 141 -> 66.
 constexpr int kPackRows = 32, kPackCols = 128;
+// Tiles of one launch: a launch holds fewer than 2^32 threads, which the tiles
+// of a very long, narrow weight exceed (K > 2^29 at up to 128 columns).
+constexpr int64_t kPackTiles = (int64_t)1 << 22;
 
 // INT8 strip-major: chunk (strip, row quad) is 4 columns x 4 rows, dword d
 // column d, byte r row r.
 template <PackFrom FROM>
-__global__ __launch_bounds__(kBlock) void k_pack_i8_tiled(const float* __restrict__ src, int64_t K, int64_t N, int64_t RQ,
+__global__ __launch_bounds__(kBlock) void k_pack_i8_tiled(const float* __restrict__ src, uint32_t t0, int64_t K, int64_t N, int64_t RQ,
                                                           int64_t NS, int ncol, const float* __restrict__ inv,
                                                           int per_tensor, uint4* __restrict__ packed,
                                                           float* __restrict__ qdata, int* __restrict__ bad) {
     __shared__ __attribute__((aligned(16))) unsigned char col[kPackCols][kPackRows + 4];
-    const int64_t kb = blockIdx.x / ncol, cb = blockIdx.x - kb * ncol;
+    const uint32_t tile = t0 + blockIdx.x;
+    const int64_t kb = tile / ncol, cb = tile - kb * ncol;
     const int64_t k0 = kb * kPackRows, n0 = cb * kPackCols;
     const int cq = threadIdx.x & 31, r0 = threadIdx.x >> 5;
     const int64_t n = n0 + 4 * cq;
@@ -194,7 +198,7 @@ __global__ __launch_bounds__(kBlock) void k_pack_i8_tiled(const float* __restric
 // kFromX needs whole groups in the tile's rows (G divides 128 and N): the
 // group's maximum is taken over its G / 8 lanes.
 template <PackFrom FROM>
-__global__ __launch_bounds__(kBlock) void k_pack_i4_tiled(const float* __restrict__ src, int64_t K, int64_t N, int64_t G,
+__global__ __launch_bounds__(kBlock) void k_pack_i4_tiled(const float* __restrict__ src, uint32_t t0, int64_t K, int64_t N, int64_t G,
                                                           int64_t Kpad, int64_t RQ, int64_t NS, int ncol,
                                                           const float* __restrict__ inv, uint32_t* __restrict__ strips,
                                                           uint32_t* __restrict__ koct, int ngap,
@@ -203,7 +207,8 @@ __global__ __launch_bounds__(kBlock) void k_pack_i4_tiled(const float* __restric
     constexpr int kOct = kPackCols / 8;
     __shared__ uint32_t word[kOct][kPackRows + 1];
     __shared__ float tsc[FROM == kFromX ? kOct : 1][kPackRows + 1];
-    const int64_t kb = blockIdx.x / ncol, cb = blockIdx.x - kb * ncol;
+    const uint32_t tile = t0 + blockIdx.x;
+    const int64_t kb = tile / ncol, cb = tile - kb * ncol;
     const int64_t k0 = kb * kPackRows, j0 = cb * kOct;
     const int oc = threadIdx.x & (kOct - 1), r0 = threadIdx.x / kOct;
     const int64_t j = j0 + oc;
@@ -285,7 +290,7 @@ __global__ __launch_bounds__(kBlock) void k_pack_i4_tiled(const float* __restric
     }
     // The dwords between the strips and the copy, so that the whole buffer is a
     // function of the codes.
-    if (blockIdx.x == 0 && (int)threadIdx.x < ngap) koct[(int64_t)threadIdx.x - ngap] = 0u;
+    if (tile == 0 && (int)threadIdx.x < ngap) koct[(int64_t)threadIdx.x - ngap] = 0u;
 }
 
 // INT4 flat pack: one thread per byte (elements 2b, 2b+1 of the flattened tensor).
@@ -450,12 +455,15 @@ hipError_t launch_pack_i8_tiled(const float* src, bool from_codes, int64_t K, in
     if (g.chunks() <= 0) return hipSuccess;
     const int64_t ncol = ceil_div(N, kPackCols), blocks = ceil_div(g.Kpad, kPackRows) * ncol;
     if (blocks >= (int64_t)1 << 31) return hipErrorInvalidValue;
-    if (from_codes)
-        k_pack_i8_tiled<kFromCodes><<<(unsigned)blocks, kBlock, 0, s>>>(src, K, N, g.RQ, g.NS, (int)ncol, inv, per_tensor,
-                                                                        (uint4*)packed, qdata, bad);
-    else
-        k_pack_i8_tiled<kFromXInv><<<(unsigned)blocks, kBlock, 0, s>>>(src, K, N, g.RQ, g.NS, (int)ncol, inv, per_tensor,
-                                                                       (uint4*)packed, qdata, bad);
+    for (int64_t t0 = 0; t0 < blocks; t0 += kPackTiles) {
+        const unsigned n = (unsigned)(blocks - t0 < kPackTiles ? blocks - t0 : kPackTiles);
+        if (from_codes)
+            k_pack_i8_tiled<kFromCodes><<<n, kBlock, 0, s>>>(src, (uint32_t)t0, K, N, g.RQ, g.NS, (int)ncol, inv,
+                                                             per_tensor, (uint4*)packed, qdata, bad);
+        else
+            k_pack_i8_tiled<kFromXInv><<<n, kBlock, 0, s>>>(src, (uint32_t)t0, K, N, g.RQ, g.NS, (int)ncol, inv,
+                                                            per_tensor, (uint4*)packed, qdata, bad);
+    }
     return hipGetLastError();
 }
 
@@ -469,19 +477,20 @@ hipError_t launch_pack_i4_tiled(const float* src, bool from_codes, int64_t K, in
     if (blocks >= (int64_t)1 << 31) return hipErrorInvalidValue;
     const int ngap = (int)((g.koct_off() - g.chunks() * 16) / 4);
     uint32_t* koct = (uint32_t*)((char*)packed + g.koct_off());
-#define SGQ_PACK_I4(FROM_)                                                                                          \
-    k_pack_i4_tiled<FROM_><<<(unsigned)blocks, kBlock, 0, s>>>(src, K, N, g.G, g.Kpad, g.RQ, g.NS, (int)ncol, inv, \
-                                                               (uint32_t*)packed, koct, ngap, scales, devscales,   \
-                                                               qdata, bad)
-    if (from_codes)
-        SGQ_PACK_I4(kFromCodes);
-    else if (inv)
-        SGQ_PACK_I4(kFromXInv);
-    else if (pack_i4_finds_scales(g))
-        SGQ_PACK_I4(kFromX);
-    else
-        return hipErrorInvalidValue;
+    if (!from_codes && !inv && !pack_i4_finds_scales(g)) return hipErrorInvalidValue;
+    for (int64_t t0 = 0; t0 < blocks; t0 += kPackTiles) {
+        const unsigned n = (unsigned)(blocks - t0 < kPackTiles ? blocks - t0 : kPackTiles);
+#define SGQ_PACK_I4(FROM_)                                                                                        \
+    k_pack_i4_tiled<FROM_><<<n, kBlock, 0, s>>>(src, (uint32_t)t0, K, N, g.G, g.Kpad, g.RQ, g.NS, (int)ncol, inv, \
+                                                (uint32_t*)packed, koct, ngap, scales, devscales, qdata, bad)
+        if (from_codes)
+            SGQ_PACK_I4(kFromCodes);
+        else if (inv)
+            SGQ_PACK_I4(kFromXInv);
+        else
+            SGQ_PACK_I4(kFromX);
 #undef SGQ_PACK_I4
+    }
     return hipGetLastError();
 }
 

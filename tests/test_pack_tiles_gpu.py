@@ -48,3 +48,27 @@ def test_int8_tiles(sgq, dev, oracle, synth, K, N, scheme):
         assert helpers.same_bits(qw.qdata.cpu().numpy(), q) and helpers.same_bits(qw.scales.cpu().numpy(), s)
         for got in (qw, sgq.pack_int8(qw.qdata, qw.scales, scheme)):
             assert np.array_equal(got.packed.cpu().numpy()[: helpers.model_pack_i8(q).size], helpers.model_pack_i8(q))
+
+
+# Narrow weights whose tiles, 256 threads each, pass 2^32 threads: the last tile's
+# rows and the first of the second launch come out like the first rows.
+@pytest.mark.parametrize("bits,N", [(8, 1), (4, 8)])
+def test_more_tiles_than_one_launch(sgq, dev, bits, N):
+    K = (1 << 29) + 40
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 64 GiB of free GPU memory")
+    x = torch.empty((K, N), device=dev)
+    rows = torch.arange(37, device=dev)
+    small = ((rows[:, None] * 3 + torch.arange(N, device=dev)) % 15 - 7).float()
+    at = [0, 1 << 27, (1 << 29) - 64, K - 37]  # 2^27 rows are the tiles of a launch
+    x.zero_()
+    for a in at:
+        x[a : a + 37] = small
+    qw = sgq.quantize_int8(x, 0, keep_qdata=False) if bits == 8 else sgq.quantize_int4(x, 8, keep_qdata=False)
+    del x
+    w = (sgq.dequantize_int8 if bits == 8 else sgq.dequantize_int4)(qw)
+    want = w[:37].clone()
+    assert (want - small).abs().max().item() <= 7.0 / (127 if bits == 8 else 7) / 2 + 1e-5
+    for a in at:
+        assert torch.equal(w[a : a + 37], want)
+    assert not w[1 << 28 : (1 << 28) + 64].any()
