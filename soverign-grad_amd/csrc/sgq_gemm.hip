@@ -45,6 +45,7 @@ namespace {
 constexpr int kWaveCols = 128;  // columns of a wavefront's tile
 constexpr int kWG = 256;        // threads per workgroup: four wavefronts
 constexpr int kStageK = 32;     // k per stage: one 16x16x32 MFMA step
+constexpr int64_t kMaxTiles = (int64_t)1 << 23;  // of a launch, which holds fewer than 2^32 threads
 
 struct GemmWaveArgs {
     const float* x;
@@ -410,6 +411,14 @@ hipError_t launch_gemm_wave(int bits, const float* x, int64_t M, int64_t K, int6
     const int gpw = bits == 8 || mode % 16 == 0 ? 1 : (mode % 8 == 0 ? 2 : 4);
     if (!gemm_wave_takes(bits, mode) || (w.rb == 4 && gpw != 1) || nw < 1 || nw > 3 || (nw > 1 && (ep.gate || ep.res)))
         return hipErrorInvalidValue;
+    const int64_t tm = ceil_div(M, w.rows()), tn = ceil_div(N, w.cols());
+    if (p.KS == 1 && nw == 1 && tm > 1 && tm * tn >= kMaxTiles) {  // very many rows: two halves
+        const int64_t h = tm / 2 * w.rows(), o = h * N;
+        const GemmEpilogue rest{ep.gate ? ep.gate + o : nullptr, ep.res ? ep.res + o : nullptr};
+        const hipError_t e = launch_gemm_wave(bits, x, h, K, N, 1, packed, scales, bias, mode, p, w, ep, y, ws, s);
+        if (e != hipSuccess) return e;
+        return launch_gemm_wave(bits, x + h * K, M - h, K, N, 1, packed, scales, bias, mode, p, w, rest, y + o, ws, s);
+    }
     GemmWaveArgs a{};
     a.x = x;
     a.M = (int)M, a.K = (int)K, a.N = (int)N;
@@ -428,7 +437,6 @@ hipError_t launch_gemm_wave(int bits, const float* x, int64_t M, int64_t K, int6
     a.y = y;
     a.part = p.KS > 1 ? (float*)ws : nullptr;
     a.y16 = N % 4 == 0 && (((uintptr_t)(p.KS > 1 ? ws : y)) & 15) == 0;
-    const int64_t tm = ceil_div(M, w.rows()), tn = ceil_div(N, w.cols());
     a.ntn = (int)tn;
     const int xcds = device_xcds(s);
     a.xlog = xcd_log2(xcds);

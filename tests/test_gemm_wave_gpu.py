@@ -80,3 +80,24 @@ def test_gated_epilogue(sgq, dev, M, K, N, bits, G):
     h = sgq.quantized_swiglu(x, q[0], q[1], b[0], b[1])
     ref = gate / (1 + torch.exp(-gate)) * up
     assert float(((h.double() - ref).abs() / ref.abs().clamp_min(1e-30)).max()) < 16 * 2.0**-24
+
+
+def test_rows_past_one_launch(sgq, dev):
+    """More 64-row tiles than a launch takes: the second half's rows and outputs follow the first's."""
+    M, K = (1 << 29) + 70, 5
+    if torch.cuda.mem_get_info()[0] < 32 << 30:
+        pytest.skip("needs 32 GiB of free GPU memory")
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(5)
+    x = torch.empty((M, K), device=dev)
+    x.copy_(torch.arange(K, device=dev).float().expand(M, K))
+    rows = torch.randn(200, K, generator=gen, device=dev)
+    at = [0, (1 << 28) - 100, 1 << 28, M - 200]
+    for a in at:
+        x[a : a + 200] = rows
+    qw = sgq.quantize_int8(torch.randn(K, 1, generator=gen, device=dev) * 0.02, 1)
+    y, w = sgq.quantized_matmul_int8(x, qw), sgq.dequantize_int8(qw)
+    for a in at[:1] + at[2:]:
+        _check(y[a : a + 200], x[a : a + 200], w, None, K)
+    _check(y[at[1] : at[1] + 100], x[at[1] : at[1] + 100], w, None, K)
+    assert torch.equal(y[1000:2000], y[-2000:-1000])
