@@ -295,7 +295,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
 // ---------------------------------------------------------------------------
 // The remaining flat weights: groups or widths below eight, codes at an odd
-// address or past 32-bit indices.  One thread per output; per-element scale index, the reference's own
+// address or past 32-bit indices or grids.  One thread per output; per-element scale index, the reference's own
 // product code*scale, FMA accumulation in k order.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_linear_i4_flat(const float* __restrict__ x, int64_t M, int64_t K,
@@ -333,9 +333,11 @@ hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N
                                  const float* scales, int64_t G, const float* bias, float* y, hipStream_t s) {
     // Elements are indexed in 31 bits, one row and a workgroup's columns past
     // the last; an octet has at most two scales from groups of eight on; codes
-    // are read by aligned dwords.
+    // are read by aligned dwords.  Rows fit an int, and a grid of 64 columns to
+    // 1024 threads stays below 2^32 threads.
     const bool fast = G >= 8 && N >= 8 && G < ((int64_t)1 << 31) && (K + 1) * N + G + 1024 < ((int64_t)1 << 31) &&
-                      K <= ((int64_t)1 << 21) && (((uintptr_t)packed) & 3) == 0;
+                      K <= ((int64_t)1 << 21) && N < ((int64_t)1 << 27) && M < ((int64_t)1 << 31) &&
+                      (((uintptr_t)packed) & 3) == 0;
     if (!fast) {
         int64_t blocks = ceil_div(M * N, 256);
         if (blocks > 65536) blocks = 65536;

@@ -58,3 +58,13 @@ def test_non_finite(sgq, dev, M, K, N):
     w = (code.reshape(-1) * scale.repeat_interleave(32)[: K * N]).reshape(K, N)
     ref = torch.stack([(x[m].double()[:, None] * w).sum(0) for m in range(M)])
     assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.equal(torch.isinf(y), torch.isinf(ref))
+
+
+def test_wide_row(sgq, dev):
+    """Columns past the row kernels' grid: one product each, so the result is exact."""
+    N = (1 << 27) + 1
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(6)
+    qw = sgq.quantize_int4(torch.randn(1, N, generator=gen, device=dev) * 0.02, 32, keep_qdata=False)
+    x = torch.full((1, 1), 1.5, device=dev)
+    assert torch.equal(sgq.quantized_matmul_int4(x, qw), x * sgq.dequantize_int4(qw).reshape(1, N))
