@@ -38,7 +38,7 @@ GROUPED = 2  # QuantizationScheme::GroupedAsymmetric
 LAYOUT_INT4_TILED = 0
 LAYOUT_INT4_FLAT = 1
 
-_raw_stream = torch._C._cuda_getCurrentRawStream
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # a CPU-only torch has none
 
 # Every entry point of include/sgq.h with its ctypes signature.
 _i64, _int, _vp = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p
