@@ -5,7 +5,10 @@
 //
 // k_gemm_wave runs the fp32 products on the bf16 matrix cores as three exact
 // bf16 products each, as k_gemm3 does for INT8 (sgq_linear.hip): x * s split
-// into three bf16 terms, codes exact in bf16, fp32 accumulation.
+// into three bf16 terms, codes exact in bf16, fp32 accumulation.  INT4's x * s
+// carry a factor of 2^16, so that the terms hold all of a product as small as
+// fp32's smallest normal number (kScaleUp; 0.5% of a g32 product's time); INT8's
+// do from 2^-110 on.
 //
 // Each wavefront computes a tile of its own, 16 RB rows by 128 columns, with
 // no LDS and no barrier in the K loop.  The lanes load what their MFMA
@@ -19,7 +22,7 @@
 //
 // Why this shape: with the planes staged in LDS a 128 x 128 tile moved 96 KB
 // through LDS per 32-k stage, as many cycles as its MFMAs take; here a stage
-// is 96 MFMAs, 332 VALU instructions and 18 loads (RB = 4, one group), and
+// is 96 MFMAs, 340 VALU instructions and 18 loads (RB = 4, one group), and
 // the registers leave two wavefronts per SIMD.  In a stage the loads of the
 // next are issued as soon as the registers they replace are consumed, and the
 // split of the next row block (or the next stage's first) is interleaved with
@@ -157,6 +160,13 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
                 s[1] = buf_load4f(rS[q], 32 * g + 16, kt * 128);
             }
         };
+        // kScaleUp goes into the scales, or into x where a wavefront has more
+        // scale groups than row blocks (fewer products per stage).
+        constexpr bool kUpX = BITS == 4 && GPW > RB, kUpS = BITS == 4 && !kUpX;
+        auto scaleUp = [&](float4 (&v)[2]) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[h].x *= kScaleUp, v[h].y *= kScaleUp, v[h].z *= kScaleUp, v[h].w *= kScaleUp;
+        };
         // 128-bit buffer loads need dword alignment only, so rows of any K
         // (and any x) load the same way; full stages stay inside their row.
         auto loadX = [&](int i, int kt) {
@@ -196,6 +206,8 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
             for (int i = 0; i < RB; ++i) loadX(i, kt0);
 #pragma unroll
             for (int c = 0; c < CB; ++c) convB(c);
+            if constexpr (kUpS) scaleUp(sv[0]);
+            if constexpr (kUpX) scaleUp(xq[0]);
             split(ap, 0, sv[0]);
             if (GPW == 1) loadX(0, kt0 + 1);
             for (int kt = kt0; kt < kf; ++kt) {
@@ -210,6 +222,9 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
                         const int i2 = (i + 1) % RB, q2 = i == RB - 1 ? (q + 1) % GPW : q;
                         const bool wrap = i2 == 0 && q2 == 0;
                         uint4 an[3];
+                        // At the first use since they were loaded.
+                        if (kUpS && i2 == 0) scaleUp(GPW == 1 ? sn : sv[q2]);
+                        if (kUpX && q2 == 0) scaleUp(xq[i2]);
                         split(an, i2, GPW == 1 && wrap ? sn : sv[q2]);
                         if (i == RB - 1) {
 #pragma unroll
@@ -252,7 +267,10 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
                                            one(rS[0], 4 * k0, 4 * h + 2), one(rS[0], 4 * k0, 4 * h + 3));
             } else {
 #pragma unroll
-                for (int q = 0; q < GPW; ++q) loadS(sv[q], q, kt);
+                for (int q = 0; q < GPW; ++q) {
+                    loadS(sv[q], q, kt);
+                    if constexpr (kUpS) scaleUp(sv[q]);
+                }
             }
 #pragma unroll
             for (int i = 0; i < RB; ++i) {
@@ -261,6 +279,7 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
                 for (int h = 0; h < 2; ++h)
                     xq[i][h] = make_float4(one(rX, base, 4 * h), one(rX, base, 4 * h + 1), one(rX, base, 4 * h + 2),
                                            one(rX, base, 4 * h + 3));
+                if constexpr (kUpX) scaleUp(xq[i]);
             }
 #pragma unroll
             for (int c = 0; c < CB; ++c) convB(c);
@@ -312,8 +331,9 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
             const int m = (tm * (sk == 1 ? 2 : 1) + um) * BM + i * 16 + row;
             const int n = (tn * (sk == 4 ? 1 : 2) + un) * kWaveCols + col;
             if (m >= M || n >= N) continue;
-            // INT4 codes entered as 16q; per tensor, x itself in place of x * s.
-            const float f = BITS == 4 ? 0.0625f : s_all;
+            // INT4 codes entered as 16q, the scales as kScaleUp s; per tensor, x
+            // itself in place of x * s.
+            const float f = BITS == 4 ? kScaleDown : s_all;
             v.x *= f, v.y *= f, v.z *= f, v.w *= f;
             // h + m + l turns an infinite x * s into inf - inf: recompute a
             // non-finite total as the reference's k-order sum.

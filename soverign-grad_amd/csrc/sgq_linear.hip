@@ -1342,7 +1342,8 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
 #pragma unroll
         for (int it = 0; it < SCI; ++it) {
             const int r4 = threadIdx.x + it * NW * 64;
-            if (r4 < rows4) ssc[q][r4] = sreg[q][it];
+            const float4 s4 = sreg[q][it];
+            if (r4 < rows4) ssc[q][r4] = make_float4(s4.x * kScaleUp, s4.y * kScaleUp, s4.z * kScaleUp, s4.w * kScaleUp);
         }
     lds_barrier();  // the scales are in LDS (the codes and x loads stay in flight)
     for (; sb < sb_hi; sb += 2 * NW) {
@@ -1383,7 +1384,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
                 if (t < 256 * C && m < a.M && col < a.N) {
 #pragma unroll
                     for (int w2 = 0; w2 < NW; ++w2) s += red[w2][c][mr & 3][16 * (mr >> 2) + sl];
-                    s *= 0.0625f;  // the codes entered as 16q
+                    s *= kScaleDown;  // the codes entered as 16q, the scales times kScaleUp
                     // h + m + l turns an infinite x * s into inf - inf: recompute
                     // a non-finite total as the reference's k-order sum.
                     if (!isfinite(s))

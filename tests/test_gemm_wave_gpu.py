@@ -15,12 +15,12 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _check(y, x, w, b, K, splits=16 + 4):
+def _check(y, x, w, b, K, splits=16 + 4, floor=0.0):
     x, w = x.double(), w.double()
     ref, mag = x @ w, x.abs() @ w.abs()
     if b is not None:
         ref, mag = ref + b.double(), mag + b.double().abs()
-    bound = (3 * -(-K // 32) + splits + 4) * 2.0**-23 * mag
+    bound = (3 * -(-K // 32) + splits + 4) * 2.0**-23 * mag + floor
     bad = ((y.double() - ref).abs() > bound).sum()
     assert int(bad) == 0, (int(bad), float(((y.double() - ref).abs() / bound).max()))
 
@@ -62,6 +62,18 @@ def test_non_finite_inputs(sgq, dev, G):
     assert torch.equal(torch.isinf(y), torch.isinf(ref))
     fin = torch.isfinite(ref)
     assert torch.equal(torch.sign(y[~fin & ~torch.isnan(ref)]), torch.sign(ref[~fin & ~torch.isnan(ref)]))
+
+
+@pytest.mark.parametrize("G", [32, 64, 128])
+@pytest.mark.parametrize("M,K,N", [(256, 1000, 256), (24, 4096, 4096)])
+def test_small_products(sgq, dev, M, K, N, G):
+    """Products near fp32's smallest normal number (|x s| about 2^-126) keep
+    their bits, on the wavefront tiles and the skinny kernel's super-block
+    form; one below it may lose a subnormal's last place (2^-149, times a code
+    of up to 8)."""
+    x, qw, b = _inputs(sgq, dev, M, K, N, G, 8)
+    x = x * 2.0**-118
+    _check(sgq.quantized_matmul_int4(x, qw), x, sgq.dequantize_int4(qw), None, K, floor=K * 8 * 2.0**-149)
 
 
 @pytest.mark.parametrize("bits,G", [(4, 128), (4, 32), (4, 24), (8, 0), (8, 1)])
