@@ -124,13 +124,13 @@ __device__ __forceinline__ bf16x8 nibbles_bf16x16(uint32_t t) {
     return __builtin_bit_cast(bf16x8, b);
 }
 
-// The INT4 kernels that split x * s put s * kScaleUp in its place and take
-// kScaleUp (and the 16 of the codes) back out of the sums.  h + m + l keeps all
-// 24 bits of v only while the lowest of them is no smaller than bf16's smallest
-// subnormal, 2^-133, that is for |v| >= 2^-110; times 2^16 that holds for every
-// normal fp32 product (and a smaller one loses no more than fp32's own
-// subnormals would).  A product or sum that this carries past fp32's range
-// comes out non-finite, and is then recomputed in k order.
+// h + m + l keeps all 24 bits of v only while the lowest of them is no smaller
+// than bf16's smallest subnormal, 2^-133, that is for |v| >= 2^-110.  Kernels that
+// took over from fp32 products put s * kScaleUp (or x * kScaleUp) into x * s and
+// take kScaleUp (and the 16 of the codes) back out of the sums: times 2^16 that
+// holds for every normal fp32 product, and a smaller one loses no more than
+// fp32's own subnormals would.  A product or sum that this carries past fp32's
+// range comes out non-finite, and is then recomputed in k order.
 constexpr float kScaleUp = 65536.0f;
 constexpr float kScaleDown = 0.0625f / 65536.0f;
 

@@ -5,10 +5,10 @@
 //
 // k_gemm_wave runs the fp32 products on the bf16 matrix cores as three exact
 // bf16 products each, as k_gemm3 does for INT8 (sgq_linear.hip): x * s split
-// into three bf16 terms, codes exact in bf16, fp32 accumulation.  INT4's x * s
-// carry a factor of 2^16, so that the terms hold all of a product as small as
-// fp32's smallest normal number (kScaleUp; 0.5% of a g32 product's time); INT8's
-// do from 2^-110 on.
+// into three bf16 terms, codes exact in bf16, fp32 accumulation.  The terms hold
+// all of a product from 2^-110 on (per tensor, of x), as in k_gemm3; groups
+// below 128 ran on fp32 products before, and carry a factor of 2^16 that keeps
+// all of fp32's normal range (kScaleUp; 0.5% of the time).
 //
 // Each wavefront computes a tile of its own, 16 RB rows by 128 columns, with
 // no LDS and no barrier in the K loop.  The lanes load what their MFMA
@@ -22,7 +22,7 @@
 //
 // Why this shape: with the planes staged in LDS a 128 x 128 tile moved 96 KB
 // through LDS per 32-k stage, as many cycles as its MFMAs take; here a stage
-// is 96 MFMAs, 340 VALU instructions and 18 loads (RB = 4, one group), and
+// is 96 MFMAs, 332 VALU instructions and 18 loads (RB = 4, one group), and
 // the registers leave two wavefronts per SIMD.  In a stage the loads of the
 // next are issued as soon as the registers they replace are consumed, and the
 // split of the next row block (or the next stage's first) is interleaved with
@@ -160,9 +160,9 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
                 s[1] = buf_load4f(rS[q], 32 * g + 16, kt * 128);
             }
         };
-        // kScaleUp goes into the scales, or into x where a wavefront has more
-        // scale groups than row blocks (fewer products per stage).
-        constexpr bool kUpX = BITS == 4 && GPW > RB, kUpS = BITS == 4 && !kUpX;
+        // Several scale groups: kScaleUp goes into the scales, or into x where
+        // there are more groups than row blocks (fewer products per stage).
+        constexpr bool kUpX = GPW > RB, kUpS = GPW > 1 && !kUpX;
         auto scaleUp = [&](float4 (&v)[2]) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) v[h].x *= kScaleUp, v[h].y *= kScaleUp, v[h].z *= kScaleUp, v[h].w *= kScaleUp;
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
                         const bool wrap = i2 == 0 && q2 == 0;
                         uint4 an[3];
                         // At the first use since they were loaded.
-                        if (kUpS && i2 == 0) scaleUp(GPW == 1 ? sn : sv[q2]);
+                        if (kUpS && i2 == 0) scaleUp(sv[q2]);
                         if (kUpX && q2 == 0) scaleUp(xq[i2]);
                         split(an, i2, GPW == 1 && wrap ? sn : sv[q2]);
                         if (i == RB - 1) {
@@ -331,9 +331,8 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
             const int m = (tm * (sk == 1 ? 2 : 1) + um) * BM + i * 16 + row;
             const int n = (tn * (sk == 4 ? 1 : 2) + un) * kWaveCols + col;
             if (m >= M || n >= N) continue;
-            // INT4 codes entered as 16q, the scales as kScaleUp s; per tensor, x
-            // itself in place of x * s.
-            const float f = BITS == 4 ? kScaleDown : s_all;
+            // INT4 codes entered as 16q; per tensor, x itself in place of x * s.
+            const float f = BITS == 8 ? s_all : (GPW > 1 ? kScaleDown : 0.0625f);
             v.x *= f, v.y *= f, v.z *= f, v.w *= f;
             // h + m + l turns an infinite x * s into inf - inf: recompute a
             // non-finite total as the reference's k-order sum.

@@ -64,8 +64,8 @@ def test_non_finite_inputs(sgq, dev, G):
     assert torch.equal(torch.sign(y[~fin & ~torch.isnan(ref)]), torch.sign(ref[~fin & ~torch.isnan(ref)]))
 
 
-@pytest.mark.parametrize("G", [32, 64, 128])
-@pytest.mark.parametrize("M,K,N", [(256, 1000, 256), (24, 4096, 4096)])
+@pytest.mark.parametrize("M,K,N,G", [(256, 1000, 256, 32), (256, 1000, 256, 64), (256, 1000, 288, 96),
+                                     (24, 4096, 4096, 32), (24, 4096, 4096, 64), (32, 2048, 5632, 128)])
 def test_small_products(sgq, dev, M, K, N, G):
     """Products near fp32's smallest normal number (|x s| about 2^-126) keep
     their bits, on the wavefront tiles and the skinny kernel's super-block
