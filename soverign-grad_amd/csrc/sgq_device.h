@@ -171,24 +171,64 @@ __device__ __forceinline__ void split3_4(const float* v, uint2& h, uint2& m, uin
     l = make_uint2(pl[0], pl[1]);
 }
 
-// One output of the forward as the reference forms it: sum over k in
-// [k0, k1) of x[k] * (q[k][n] * s), in k order (the non-finite fallback).
-template <int BITS>
-__device__ float output_exact(const float* xrow, const uint4* W, const float* S, int mode, int Kpad, int RQ, int n,
-                              int k0, int k1) {
+// C neighbouring outputs of a row as the reference forms them (the non-finite
+// fallback): sums over k in [k0, k1) of x[k] * (q[k][n + c] * s), in k order.
+// C > 1: n .. n + C - 1 lie in one strip.  The loads of
+// U k are issued together, and a thread stops once all its sums are NaN, which
+// no further term changes: the NaN rows of a batch's inactive sequences end with
+// their first k.  Measured (us, one k at a time to the end -> this): 256 x 2048 ->
+// 5632 g32 with one row of NaN 323 -> 52, with one infinity 323 -> 104; a block
+// step with inactive sequences, two of 8 at g128 350 -> 41, four of 24 at g32 481
+// -> 72.
+constexpr int kExactK = 8;
+template <int BITS, int C, int U>
+__device__ __forceinline__ void outputs_exact(const float* xrow, const uint4* W, const float* S, int mode, int Kpad, int RQ,
+                                              int n, int k0, int k1, float (&acc)[C]) {
+    const uint32_t* wd = reinterpret_cast<const uint32_t*>(W + (int64_t)(BITS == 8 ? n >> 2 : n >> 3) * RQ);
+    if constexpr (BITS == 4) S += (int64_t)((n >> 3) / mode) * Kpad;
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] = 0.0f;
+#pragma unroll 1
+    for (int kb = k0; kb < k1; kb += U) {
+        float xv[U], sv[U];
+        uint32_t d[U][BITS == 8 ? C : 1];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            const int k = min(kb + i, k1 - 1);
+            xv[i] = xrow[k];
+            sv[i] = BITS == 8 && mode ? S[0] : S[k];
+            if constexpr (BITS == 4) {
+                d[i][0] = wd[k];
+            } else {
+#pragma unroll
+                for (int c = 0; c < C; ++c)
+                    d[i][c] = reinterpret_cast<const unsigned char*>(wd)[(k >> 2) * 16 + ((n & 3) + c) * 4 + (k & 3)];
+            }
+        }
+        bool all_nan = true;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                const float q = BITS == 8 ? (float)(signed char)d[i][BITS == 8 ? c : 0]
+                                          : (float)(((int)(d[i][0] << (28 - 4 * ((n & 7) + c)))) >> 28);
+                if (kb + i < k1) acc[c] = fmaf(xv[i], q * sv[i], acc[c]);
+            }
+            all_nan = all_nan && isnan(acc[c]);
+        }
+        if (all_nan) break;
+    }
+}
+// One INT8 output, one k at a time to the end: k_gemm3 inlines it for each of a
+// thread's outputs, where anything longer costs its small batches (24 x 4096 ->
+// 11008 24.2 -> 25.1 us).
+__device__ __forceinline__ float output_exact_i8(const float* xrow, const uint4* W, const float* S, bool per_tensor, int RQ, int n, int k0,
+                                 int k1) {
     float acc = 0.0f;
     for (int k = k0; k < k1; ++k) {
-        float q, s;
-        if constexpr (BITS == 8) {
-            q = (float)reinterpret_cast<const signed char*>(W)[((int64_t)(n >> 2) * RQ + (k >> 2)) * 16 + (n & 3) * 4 +
-                                                                (k & 3)];
-            s = mode ? S[0] : S[k];
-        } else {
-            const uint32_t d = reinterpret_cast<const uint32_t*>(W + (int64_t)(n >> 3) * RQ)[k];
-            q = (float)(((int)(d << (28 - 4 * (n & 7)))) >> 28);
-            s = S[(int64_t)((n >> 3) / mode) * Kpad + k];
-        }
-        acc = fmaf(xrow[k], q * s, acc);
+        const float q = (float)reinterpret_cast<const signed char*>(W)[((int64_t)(n >> 2) * RQ + (k >> 2)) * 16 +
+                                                                       (n & 3) * 4 + (k & 3)];
+        acc = fmaf(xrow[k], q * (per_tensor ? S[0] : S[k]), acc);
     }
     return acc;
 }

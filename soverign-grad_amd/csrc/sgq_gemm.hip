@@ -338,14 +338,12 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
             // non-finite total as the reference's k-order sum.
             const int nc = BITS == 4 ? 4 : min(4, N - n);  // INT4: N is a multiple of 8
             if (!(isfinite(v.x) && isfinite(v.y) && isfinite(v.z) && isfinite(v.w))) {
-#pragma unroll 1
-                for (int e = 0; e < nc; ++e) {
-                    const float w = f4get(v, e);
-                    if (isfinite(w)) continue;
-                    const float r = output_exact<BITS>(a.x + (int64_t)m * K, W, S, BITS == 8 ? (PT ? 1 : 0) : a.spc, a.Kpad,
-                                                       a.RQ, n + e, klo, khi);
-                    v.x = e == 0 ? r : v.x, v.y = e == 1 ? r : v.y, v.z = e == 2 ? r : v.z, v.w = e == 3 ? r : v.w;
-                }
+                float r[4];
+                // (U for INT8: more loads together spill in the loop above.)
+                outputs_exact<BITS, 4, BITS == 8 ? 2 : kExactK>(a.x + (int64_t)m * K, W, S, BITS == 8 ? (PT ? 1 : 0) : a.spc,
+                                                                a.Kpad, a.RQ, n, klo, khi, r);
+                v.x = isfinite(v.x) ? v.x : r[0], v.y = isfinite(v.y) ? v.y : r[1];
+                v.z = isfinite(v.z) ? v.z : r[2], v.w = isfinite(v.w) ? v.w : r[3];
             }
             const int64_t o = (int64_t)m * N + n;
             float* out = KS > 1 ? a.part + (int64_t)(wi * KS + split) * M * N : a.y + (int64_t)wi * M * N;

@@ -67,10 +67,22 @@ __device__ float i4_column_exact(const uint4* W, const float* SC, int j, int e, 
     const uint32_t* wd = reinterpret_cast<const uint32_t*>(W + (int64_t)j * RQ);
     const float* sc = SC + (int64_t)(j / spc) * Kpad;
     float acc = 0.0f;
-    for (int k = k0; k < k1; ++k) {
-        const int q = ((int)(wd[k] << (28 - 4 * e))) >> 28;
-        const float s = NORM ? gamma[k] * sc[k] : sc[k];
-        acc = fmaf((float)q, xrow[k] * s, acc);
+    // Eight k at a time, until the sum is NaN, as outputs_exact.
+#pragma unroll 1
+    for (int kb = k0; kb < k1; kb += kExactK) {
+        float xv[kExactK], sv[kExactK];
+        uint32_t d[kExactK];
+#pragma unroll
+        for (int i = 0; i < kExactK; ++i) {
+            const int k = min(kb + i, k1 - 1);
+            xv[i] = xrow[k];
+            sv[i] = NORM ? gamma[k] * sc[k] : sc[k];
+            d[i] = wd[k];
+        }
+#pragma unroll
+        for (int i = 0; i < kExactK; ++i)
+            if (kb + i < k1) acc = fmaf((float)(((int)(d[i] << (28 - 4 * e))) >> 28), xv[i] * sv[i], acc);
+        if (isnan(acc)) break;
     }
     return acc;
 }
@@ -852,7 +864,7 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(SH::WPE)
                 const int m = m0 + wm * 16 * RB + i * 16 + lkg * 4 + r;
                 if (m < M) {
                     float v = PT ? acc[i][j][r] * s_all : acc[i][j][r];
-                    if (!isfinite(v)) v = output_exact<8>(x + (int64_t)m * K, W, S, PT ? 1 : 0, Kpad, RQ, n, klo, khi);
+                    if (!isfinite(v)) v = output_exact_i8(x + (int64_t)m * K, W, S, PT, RQ, n, klo, khi);
                     out[(int64_t)m * N + n] = (bias && KS == 1) ? v + bv : v;
                 }
             }
@@ -1610,7 +1622,11 @@ __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ h
             if constexpr (PT) s = s * s_all;
             // h + m + l turns an infinite x into inf - inf: recompute a
             // non-finite total as the reference's k-order sum.
-            if (!isfinite(s)) s = output_exact<8>(a.x + (int64_t)m * K, a.W, a.S, PT ? 1 : 0, a.Kpad, a.RQ, col, 0, K);
+            if (!isfinite(s)) {
+                float r[1];
+                outputs_exact<8, 1, kExactK>(a.x + (int64_t)m * K, a.W, a.S, PT ? 1 : 0, a.Kpad, a.RQ, col, 0, K, r);
+                s = r[0];
+            }
             const int64_t o = (int64_t)m * a.N + col;
             if (a.bias) s = s + a.bias[col];
             if (a.gate) s = silu_f32(a.gate[o]) * s;
