@@ -45,6 +45,9 @@
 namespace sgq {
 namespace {
 
+// Four floats at any 4-byte address, as 128-bit stores take them.
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+
 constexpr int kWaveCols = 128;  // columns of a wavefront's tile
 constexpr int kWG = 256;        // threads per workgroup: four wavefronts
 constexpr int kStageK = 32;     // k per stage: one 16x16x32 MFMA step
@@ -63,7 +66,6 @@ struct GemmWaveArgs {
     GemmEpilogue ep;
     float* y;
     float* part;            // KS > 1: partial results of each weight, [KS][M][N]
-    int y16;                // y and part are 16-byte aligned
     int ntn;                // workgroup tiles along N
     int xr, xlog;           // as k_gemm3: tile rows of an XCD's rectangle, log2 of the XCDs
 };
@@ -253,32 +255,28 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
             }
         }
         if (kf < kt1) {
-            // The last, partial stage: x by single floats, zero past K.
+            // The last, partial stage.  The scales and codes past K are zero or
+            // unused; x past it is the next row's, so it is zeroed here.
             const int kt = kt1 - 1;
             const int k0 = kt * kStageK + 8 * g;
             loadB(kt);
-            auto one = [&](const __amdgpu_buffer_rsrc_t& r, int base, int e) {
-                return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, k0 + e < K ? base + 4 * e : kOobOff, 0, 0));
-            };
-            if constexpr (BITS == 8 && !PT) {  // K scales, unpadded
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    sv[0][h] = make_float4(one(rS[0], 4 * k0, 4 * h), one(rS[0], 4 * k0, 4 * h + 1),
-                                           one(rS[0], 4 * k0, 4 * h + 2), one(rS[0], 4 * k0, 4 * h + 3));
-            } else {
+            for (int q = 0; q < GPW; ++q) loadS(sv[q], q, kt);
 #pragma unroll
-                for (int q = 0; q < GPW; ++q) {
-                    loadS(sv[q], q, kt);
-                    if constexpr (kUpS) scaleUp(sv[q]);
-                }
+            for (int i = 0; i < RB; ++i) loadX(i, kt);
+            if constexpr (kUpS) {
+#pragma unroll
+                for (int q = 0; q < GPW; ++q) scaleUp(sv[q]);
             }
 #pragma unroll
             for (int i = 0; i < RB; ++i) {
-                const int base = xo[i] + kt * 128;
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    xq[i][h] = make_float4(one(rX, base, 4 * h), one(rX, base, 4 * h + 1), one(rX, base, 4 * h + 2),
-                                           one(rX, base, 4 * h + 3));
+                for (int h = 0; h < 2; ++h) {
+                    float4& v = xq[i][h];
+                    const int left = K - k0 - 4 * h;
+                    v.x = left > 0 ? v.x : 0.0f, v.y = left > 1 ? v.y : 0.0f;
+                    v.z = left > 2 ? v.z : 0.0f, v.w = left > 3 ? v.w : 0.0f;
+                }
                 if constexpr (kUpX) scaleUp(xq[i]);
             }
 #pragma unroll
@@ -347,15 +345,17 @@ __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(2))) void k
             }
             const int64_t o = (int64_t)m * N + n;
             float* out = KS > 1 ? a.part + (int64_t)(wi * KS + split) * M * N : a.y + (int64_t)wi * M * N;
-            if (a.y16 && nc == 4) {
+            if (nc == 4) {
                 if (KS == 1) {
                     if (bias) v.x += bias[n], v.y += bias[n + 1], v.z += bias[n + 2], v.w += bias[n + 3];
                     v.x = gemm_epilogue(a.ep, v.x, o), v.y = gemm_epilogue(a.ep, v.y, o + 1);
                     v.z = gemm_epilogue(a.ep, v.z, o + 2), v.w = gemm_epilogue(a.ep, v.w, o + 3);
                 }
-                *(float4*)(out + o) = v;
+                *(f32x4_u*)(out + o) = f32x4_u{v.x, v.y, v.z, v.w};
             } else {
-                for (int e = 0; e < nc; ++e) {
+#pragma unroll
+                for (int e = 0; e < 3; ++e) {
+                    if (e >= nc) continue;
                     float w = f4get(v, e);
                     if (KS == 1) w = gemm_epilogue(a.ep, bias ? w + bias[n + e] : w, o + e);
                     out[o + e] = w;
@@ -415,8 +415,23 @@ __global__ __launch_bounds__(kWG) void k_splitk_reduce(const float* __restrict__
 // ranges against two without a split: 384 x 4096 -> 11008 116 against 134,
 // 2048 x 4096 -> 11008 457 against 477; with one 40 x 4096 -> 4096 26.4
 // against 23.5, 96 x 11008 -> 4096 45 against 43.
-GemmWaveShape gemm_wave_shape(int64_t M, int64_t N, bool one_scale, int KS, int64_t cus) {
+//
+// A short K has too few stages for four ranges: with many tiles each wavefront
+// takes one of its own (half with two ranges in between), and two row blocks,
+// whose epilogue is shorter.  Measured at K = 64 (us, four ranges / two / one, the
+// kernels before this one): g32 2048 rows -> 2048 (1024 tiles) 19.9 / 14.4 / 16.3,
+// 18.5; -> 4096 (2048 tiles) 33.8 / 24.6 / 20.3, 24.2; -> 11008 81.7 / 57.2 / 48.2,
+// 61.8; at K = 512 g128 4096 -> 16384 272 / 231 / 217, 271; 512 tiles at K = 96
+// 11.1 / 13.2 / 17.0, 19.2.
+GemmWaveShape gemm_wave_shape(int64_t M, int64_t K, int64_t N, bool one_scale, int KS, int64_t cus) {
+    constexpr int64_t kShortK = 512;
     GemmWaveShape w;
+    if (KS == 1 && K <= kShortK) {
+        const int64_t tiles = ceil_div(M, 32) * ceil_div(N, kWaveCols);
+        w.rb = 2;
+        w.sk = tiles >= 8 * cus ? 1 : (tiles >= 4 * cus ? 2 : 4);
+        return w;
+    }
     w.rb = one_scale && ceil_div(M, 64) * ceil_div(N, kWaveCols) * KS >= 4 * cus ? 4 : 2;
     w.sk = KS > 1 ? 2 : 4;
     return w;
@@ -453,7 +468,6 @@ hipError_t launch_gemm_wave(int bits, const float* x, int64_t M, int64_t K, int6
     a.ep = ep;
     a.y = y;
     a.part = p.KS > 1 ? (float*)ws : nullptr;
-    a.y16 = N % 4 == 0 && (((uintptr_t)(p.KS > 1 ? ws : y)) & 15) == 0;
     a.ntn = (int)tn;
     const int xcds = device_xcds(s);
     a.xlog = xcd_log2(xcds);

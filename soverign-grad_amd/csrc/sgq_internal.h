@@ -427,7 +427,7 @@ struct GemmWaveShape {
 };
 inline bool gemm_wave_takes(int bits, int spc) { return bits == 8 || spc % 4 == 0; }
 // one_scale: a wavefront's 128 columns share their scales.
-GemmWaveShape gemm_wave_shape(int64_t M, int64_t N, bool one_scale, int KS, int64_t cus);
+GemmWaveShape gemm_wave_shape(int64_t M, int64_t K, int64_t N, bool one_scale, int KS, int64_t cus);
 // mode: INT8 the per-tensor flag, INT4 strips per scale column; scales: INT4
 // the device scales.
 hipError_t launch_gemm_wave(int bits, const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,

@@ -2297,7 +2297,7 @@ int gemm_rect_rows(int bits, int64_t M, int64_t K, int64_t N, int mode, int64_t 
     int64_t bm = t.bm, bn = t.bn;
     if (bits == 4) {
         if (!gemm_wave_takes(4, mode)) return 0;  // the fp32 kernel keeps the plain order
-        const GemmWaveShape w = gemm_wave_shape(M, N, mode % 16 == 0, 1, cus);
+        const GemmWaveShape w = gemm_wave_shape(M, K, N, mode % 16 == 0, 1, cus);
         bm = w.rows(), bn = w.cols();
     }
     return xcd_rect_rows(ceil_div(M, bm), ceil_div(N, bn), bm * K * 4, bn * K * bits / 8, xcds);
@@ -2350,7 +2350,7 @@ hipError_t launch_gemm_i8(const float* x, int64_t M, int64_t K, int64_t N, const
         // against 187: both run at the power limit, and this kernel converts
         // each code and splits each x for a whole 128 x 256 tile).
         e = launch_gemm_wave(8, x, M, K, N, 1, &packed, &scales, &bias, per_tensor ? 1 : 0, p,
-                             gemm_wave_shape(M, N, true, p.KS, device_cus(s)), ep, y, ws, s);
+                             gemm_wave_shape(M, K, N, true, p.KS, device_cus(s)), ep, y, ws, s);
     } else {
         if (p.KS == 1 && (ep.gate || ep.res)) return hipErrorInvalidValue;  // gemm_i8_epilogue
         if (t.bm == 32)
@@ -2373,7 +2373,7 @@ hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, int n
     hipError_t e = hipSuccess;
     if (gemm_wave_takes(4, (int)g.spc)) {
         e = launch_gemm_wave(4, x, M, K, N, nw, packed, devscales, bias, (int)g.spc, p,
-                             gemm_wave_shape(M, nw * N, g.spc % 16 == 0, p.KS, cus), ep, y, ws, s);
+                             gemm_wave_shape(M, K, nw * N, g.spc % 16 == 0, p.KS, cus), ep, y, ws, s);
     } else {
         const unsigned grid = (unsigned)(ceil_div(M, kBM) * ceil_div(N, kBN) * p.KS);
         for (int w = 0; w < nw && e == hipSuccess; ++w) {
