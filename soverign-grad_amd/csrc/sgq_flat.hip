@@ -79,8 +79,8 @@ struct FlatArgs {
     int xlog;  // log2 of the device's XCD count
 };
 
-// Batches of up to 32 rows.  A workgroup of 16 wavefronts owns 8 LC columns over
-// all of K for MT batch rows (blockIdx.y picks the rows): LC lanes take eight
+// Batches of a few rows, or of narrow weights.  A workgroup of 16 wavefronts owns
+// 8 LC columns over all of K for MT batch rows (blockIdx.y picks the rows): LC lanes take eight
 // consecutive columns each, the other 64 / LC lanes of a wavefront and the
 // wavefronts take rows k in turn, so a wavefront reads runs of 4 LC bytes and
 // a workgroup's loads walk the tensor in order.  x goes through LDS as [k][m]
@@ -294,9 +294,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 }
 
 // ---------------------------------------------------------------------------
-// The remaining flat weights: groups or widths below eight, codes at an odd
-// address or past 32-bit indices or grids.  One thread per output; per-element scale index, the reference's own
-// product code*scale, FMA accumulation in k order.
+// A short K (flat_form), and the remaining flat weights: groups or widths below
+// eight, codes at an odd address or past 32-bit indices or grids.  One thread per
+// output; per-element scale index, the reference's own product code*scale, FMA
+// accumulation in k order.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_linear_i4_flat(const float* __restrict__ x, int64_t M, int64_t K,
                                                              int64_t N, const unsigned char* __restrict__ P,
@@ -316,12 +317,50 @@ __global__ __launch_bounds__(256) void k_linear_i4_flat(const float* __restrict_
     }
 }
 
+// 128 columns per workgroup of the row form where that gives every CU one, else 64.
+bool flat_wide(int64_t groups, int64_t N, int64_t cus) { return ceil_div(N, 128) * groups >= cus; }
+
+// The form with the least expected time, us on an MI355X, fitted to nine hundred
+// shapes of 1 to 65536 rows, K 1 to 4096 and N 9 to 32001 with each form timed: of
+// those the choice is at most 9% slower than a thread per output, and all but ten
+// lie within 15% of the best form (those ten take 10 to 30 us).
+//  - a thread per output walks K at 0.17 us a step while the chip is not full,
+//    then at 1.4 products per ps and 0.65 outputs per ps.  Short K: 100000 x 8 ->
+//    12 12.4 us against 397 for the row form and 13 for tiles, 39 x 6 -> 9671 5.1
+//    against 20, one row x 3 -> 7095 2.8 against 5.0.
+//  - the row form: a workgroup per CU at a time, each a fixed cost (x into LDS, the
+//    reductions) and a time per k, by rows and columns per workgroup.
+//  - tiles cost 3.6 us for 32 k and every 128 rows, however few of them: 2048 ->
+//    32001 takes the rows 34 us per eight and tiles 241 up to 128 rows.
+enum class FlatForm { kThreads, kRows, kTiles };
+FlatForm flat_form(int64_t M, int64_t K, int64_t N, int64_t cus) {
+    const double k = (double)K, mn = (double)M * (double)N;
+    FlatForm best = FlatForm::kThreads;
+    double t = 3.0 + 0.17 * k + mn * (k / 1.4e6 + 1 / 6.5e5);
+    const int mlog = M == 1 ? 0 : (M == 2 ? 1 : (M <= 4 ? 2 : 3));
+    const int64_t groups = ceil_div(M, (int64_t)1 << mlog);
+    if (groups <= 65535) {  // grid.y
+        static const double fixed[2][4] = {{3.0, 3.5, 4.5, 7.5}, {4.5, 6.5, 8.5, 9.0}};
+        static const double per_k[2][4] = {{.003, .0033, .0045, .0065}, {.0055, .007, .0085, .0135}};
+        const bool wide = flat_wide(groups, N, cus);
+        const int64_t rounds = ceil_div(groups * ceil_div(N, wide ? 128 : 64), cus);
+        const double rows = 3.0 + (wide && rounds == 1 && mlog == 3 ? 6.0 : 0.0) +
+                            (double)rounds * (fixed[wide][mlog] + per_k[wide][mlog] * k);
+        if (rows < t) t = rows, best = FlatForm::kRows;
+    }
+    if (M > 32) {
+        const int64_t tiles = ceil_div(M, kFT) * ceil_div(N, kFT);
+        const double gemm =
+            12.0 + mn / 5.5e5 + (double)ceil_div(K, kFK) * (tiles <= cus ? 3.6 : 2.9 * (double)ceil_div(tiles, cus));
+        if (gemm < t) best = FlatForm::kTiles;
+    }
+    return best;
+}
 
 template <int MT>
 void flat_rows_launch(const FlatArgs& a, int64_t cus, hipStream_t s) {
     const unsigned groups = (unsigned)ceil_div(a.M, MT);
-    // 128 columns per workgroup where that gives every CU one, else 64.
-    if (ceil_div(a.N, 128) * groups >= cus)
+    if (flat_wide(groups, a.N, cus))
         k_flat_rows<MT, 16><<<dim3((unsigned)ceil_div(a.N, 128), groups), kFlatWaves * 64, 0, s>>>(a);
     else
         k_flat_rows<MT, 8><<<dim3((unsigned)ceil_div(a.N, 64), groups), kFlatWaves * 64, 0, s>>>(a);
@@ -338,7 +377,9 @@ hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N
     const bool fast = G >= 8 && N >= 8 && G < ((int64_t)1 << 31) && (K + 1) * N + G + 1024 < ((int64_t)1 << 31) &&
                       K <= ((int64_t)1 << 21) && N < ((int64_t)1 << 27) && M < ((int64_t)1 << 31) &&
                       (((uintptr_t)packed) & 3) == 0;
-    if (!fast) {
+    const int64_t cus = device_cus(s);
+    const FlatForm form = fast ? flat_form(M, K, N, cus) : FlatForm::kThreads;
+    if (form == FlatForm::kThreads) {
         int64_t blocks = ceil_div(M * N, 256);
         if (blocks > 65536) blocks = 65536;
         if (blocks < 1) blocks = 1;
@@ -357,30 +398,16 @@ hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N
     a.bias = bias;
     a.y = y;
     a.xlog = xcd_log2(device_xcds(s));
-    const int64_t cus = device_cus(s);
-    // The row form costs time for every eight rows, the GEMM for every 128
-    // however few its tiles: 2048 -> 32001 takes the rows 34 us per eight and
-    // the GEMM 241 up to 128 rows, 2048 -> 5003 the rows 103 at 128 rows and
-    // 137 at 200 against 108 and 144 for the GEMM, so the line lies near M * N
-    // = 7 * 2^18 for either.
-    if (M > 32 && M * N >= ((int64_t)7 << 18)) {
+    if (form == FlatForm::kTiles)
         k_flat_gemm<<<(unsigned)(ceil_div(M, kFT) * ceil_div(N, kFT)), 256, 0, s>>>(a);
-    } else {
-        for (int64_t m = 0; m < M; m += 8 * 65535) {  // grid.y
-            FlatArgs p = a;
-            p.x = x + m * K;
-            p.y = y + m * N;
-            p.M = (int)(M - m < 8 * 65535 ? M - m : 8 * 65535);
-            if (p.M == 1)
-                flat_rows_launch<1>(p, cus, s);
-            else if (p.M == 2)
-                flat_rows_launch<2>(p, cus, s);
-            else if (p.M <= 4)
-                flat_rows_launch<4>(p, cus, s);
-            else
-                flat_rows_launch<8>(p, cus, s);
-        }
-    }
+    else if (M == 1)
+        flat_rows_launch<1>(a, cus, s);
+    else if (M == 2)
+        flat_rows_launch<2>(a, cus, s);
+    else if (M <= 4)
+        flat_rows_launch<4>(a, cus, s);
+    else
+        flat_rows_launch<8>(a, cus, s);
     return hipGetLastError();
 }
 

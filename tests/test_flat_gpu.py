@@ -39,6 +39,46 @@ def test_gemm(sgq, dev, M, K, N, G):
     _check(sgq, dev, M, K, N, G)
 
 
+@pytest.mark.parametrize("M,K,N,G", [(1, 1, 9, 32), (40, 3, 4001, 24), (5000, 15, 9, 12), (300, 40, 33, 32),
+                                     (9000, 64, 17, 32), (9000, 20, 8193, 32), (33, 2, 70001, 8)])
+def test_short_k(sgq, dev, M, K, N, G):
+    """Few products per output: a thread per output, tiles where there are many rows."""
+    _check(sgq, dev, M, K, N, G)
+
+
+@pytest.mark.parametrize("M,K,N,G", [(M, K, N, 32) for M, K in ((1, 4095), (2, 4097), (4, 8193), (5, 2047), (8, 2049), (9, 4097))
+                                     for N in (33, 32801 if M < 9 else 16411)])
+def test_k_chunks(sgq, dev, M, K, N, G):
+    """x restaged in LDS: K around one and two chunks of 4096 rows (2048 from five
+    batch rows on), workgroups of 64 and of 128 columns."""
+    _check(sgq, dev, M, K, N, G)
+
+
+def _queued_us(fn, reps=20):
+    fn()
+    best = float("inf")
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        torch.cuda.synchronize()
+        a.record()
+        for _ in range(reps):
+            fn()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1000 / reps)
+    return best
+
+
+@pytest.mark.parametrize("M,K,N,few,most", [(20306, 15, 9, 64, 4), (39, 6, 9671, 1, 2)])
+def test_short_k_costs_few_launches(sgq, dev, M, K, N, few, most):
+    """Some hundred thousand products of a short K take about a launch's time,
+    as a few rows do (measured 1.0 to 1.2 times; the row form 9 and 2.7)."""
+    qw = sgq.quantize_int4(torch.randn(K, N, device=dev), 24, keep_qdata=False)
+    x = torch.randn(M, K, device=dev)
+    base = _queued_us(lambda: sgq.quantized_matmul_int4(x[:few], qw))
+    assert _queued_us(lambda: sgq.quantized_matmul_int4(x, qw)) < most * base
+
+
 @pytest.mark.parametrize("M,K,N,G", [(3, 50, 5, 32), (4, 40, 33, 7), (2, 16, 40, 5)])
 def test_narrow_and_small_groups(sgq, dev, M, K, N, G):
     _check(sgq, dev, M, K, N, G)
