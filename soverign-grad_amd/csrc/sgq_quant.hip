@@ -190,6 +190,44 @@ __global__ __launch_bounds__(kBlock) void k_pack_i8_tiled(const float* __restric
     }
 }
 
+// A thread per chunk, consecutive threads on consecutive strips of the same rows:
+// for weights that leave most of a 32 x 128 tile empty (launch_pack_i8_tiled).
+template <PackFrom FROM>
+__global__ __launch_bounds__(kBlock) void k_pack_i8_chunks(const float* __restrict__ src, int64_t K, int64_t N, int64_t RQ,
+                                                           int64_t NS, int64_t nchunks, const float* __restrict__ inv,
+                                                           int per_tensor, uint4* __restrict__ packed,
+                                                           float* __restrict__ qdata, int* __restrict__ bad) {
+    for (int64_t c = blockIdx.x * (int64_t)kBlock + threadIdx.x; c < nchunks; c += (int64_t)gridDim.x * kBlock) {
+        const int64_t rq = c / NS, j = c - rq * NS;
+        const int64_t k0 = rq * 4, n0 = j * 4;
+        uint32_t dw[4];
+        int badflag = 0;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const int64_t n = n0 + d;
+            uint32_t word = 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t k = k0 + r;
+                float v = 0.0f;
+                if (k < K && n < N) {
+                    v = src[k * N + n];
+                    if constexpr (FROM == kFromCodes) {
+                        if (!valid_code(v, -128.0f, 127.0f)) badflag = 1, v = 0.0f;
+                    } else {
+                        v = ref_code(v, per_tensor ? inv[0] : inv[k], -127.0f, 127.0f);
+                        if (qdata) qdata[k * N + n] = v;
+                    }
+                }
+                word |= ((uint32_t)(int)v & 0xFFu) << (8 * r);
+            }
+            dw[d] = word;
+        }
+        if (packed) packed[j * RQ + rq] = make_uint4(dw[0], dw[1], dw[2], dw[3]);
+        if (badflag) atomicOr(bad, 1);
+    }
+}
+
 // INT4 strip-major: the strips, the k-octet copy and (kFromX) the scales in
 // both layouts from one read of x.  A thread takes eight columns of two rows,
 // one strip dword each; a strip's 32 rows are consecutive dwords, and the
@@ -449,10 +487,31 @@ hipError_t launch_absmax_partial(const float* x, int64_t total, float* partial, 
     return hipGetLastError();
 }
 
+// Weights that leave most of every tile empty: one row, a column or two, and
+// long ones of up to 4 (16) columns, whose tiles outnumber the chip.  Measured (us
+// a quantize with fp32 codes, tiles -> chunks): 1 x 2^20 22.7 -> 17.7, 2^20 x 1 67 ->
+// 11.8, 2^20 x 3 80 -> 34, 131072 x 8 18.8 -> 13.7, x 16 19.7 -> 16.1; the tiles keep
+// 2 x 2^20 (25.1 against 28.0), 4096 x 3 (10.5, 11.4), 131072 x 24 (23.0, 23.7), 2^20
+// x 8 (90, 107).
+static bool pack_i8_by_chunks(int64_t K, int64_t N) {
+    constexpr int64_t kLong = 1 << 16, kVeryLong = 1 << 19;
+    return K == 1 || N <= 2 || (K >= kLong && (N <= 4 || (N <= 16 && K < kVeryLong)));
+}
+
 hipError_t launch_pack_i8_tiled(const float* src, bool from_codes, int64_t K, int64_t N, const float* inv,
                                 bool per_tensor, void* packed, float* qdata, int* bad, hipStream_t s) {
     const I8Geom g(K, N);
     if (g.chunks() <= 0) return hipSuccess;
+    if (pack_i8_by_chunks(K, N)) {
+        const unsigned blocks = grid_for(g.chunks());
+        if (from_codes)
+            k_pack_i8_chunks<kFromCodes><<<blocks, kBlock, 0, s>>>(src, K, N, g.RQ, g.NS, g.chunks(), inv, per_tensor,
+                                                                   (uint4*)packed, qdata, bad);
+        else
+            k_pack_i8_chunks<kFromXInv><<<blocks, kBlock, 0, s>>>(src, K, N, g.RQ, g.NS, g.chunks(), inv, per_tensor,
+                                                                  (uint4*)packed, qdata, bad);
+        return hipGetLastError();
+    }
     const int64_t ncol = ceil_div(N, kPackCols), blocks = ceil_div(g.Kpad, kPackRows) * ncol;
     if (blocks >= (int64_t)1 << 31) return hipErrorInvalidValue;
     for (int64_t t0 = 0; t0 < blocks; t0 += kPackTiles) {

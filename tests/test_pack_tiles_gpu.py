@@ -50,9 +50,45 @@ def test_int8_tiles(sgq, dev, oracle, synth, K, N, scheme):
             assert np.array_equal(got.packed.cpu().numpy()[: helpers.model_pack_i8(q).size], helpers.model_pack_i8(q))
 
 
+@pytest.mark.parametrize("K,N", [(1, 65541), (65541, 2), (65541, 3), (65541, 16), (65541, 17), (524291, 4), (524291, 5)])
+@pytest.mark.parametrize("scheme", [0, 1])
+def test_int8_narrow(sgq, dev, oracle, synth, K, N, scheme):
+    """Both sides of the line between the tiles and a thread per chunk."""
+    W = _x(synth, K, N, 80 + N)
+    q, s = oracle.quantize_int8(W, scheme)
+    qw = sgq.quantize_int8(torch.from_numpy(W).to(dev), scheme)
+    assert helpers.same_bits(qw.qdata.cpu().numpy(), q) and helpers.same_bits(qw.scales.cpu().numpy(), s)
+    for got in (qw, sgq.pack_int8(qw.qdata, qw.scales, scheme), sgq.quantize_int8(torch.from_numpy(W).to(dev), scheme, keep_qdata=False)):
+        assert np.array_equal(got.packed.cpu().numpy()[: helpers.model_pack_i8(q).size], helpers.model_pack_i8(q))
+    bad = qw.qdata.clone()
+    bad[-1, -1] = 0.5
+    with pytest.raises(sgq.SGQError):
+        sgq.pack_int8(bad, qw.scales, scheme)
+
+
+def test_int8_narrow_is_no_slower_than_square(sgq, dev):
+    """A column of 2^20 weights quantizes like a square of them (measured about the
+    same; in tiles of 128 columns 3.2 times)."""
+    def us(K, N):
+        w = torch.randn(K, N, device=dev)
+        best = float("inf")
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            a.record()
+            for _ in range(20):
+                sgq.quantize_int8(w, 0, keep_qdata=False)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 1000 / 20)
+        return best
+
+    assert us(1 << 20, 1) < 2 * us(1 << 10, 1 << 10)
+
+
 # Narrow weights whose tiles, 256 threads each, pass 2^32 threads: the last tile's
 # rows and the first of the second launch come out like the first rows.
-@pytest.mark.parametrize("bits,N", [(8, 1), (4, 8)])
+@pytest.mark.parametrize("bits,N", [(8, 1), (8, 5), (4, 8)])
 def test_more_tiles_than_one_launch(sgq, dev, bits, N):
     K = (1 << 29) + 40
     if torch.cuda.mem_get_info()[0] < 64 << 30:
