@@ -404,9 +404,14 @@ __global__ __launch_bounds__(kBlock) void k_poison_rows(const int32_t* __restric
 hipError_t launch_rms_norm(const float* x, int64_t rows, int64_t D, const float* g, float eps, float* out,
                            hipStream_t s) {
     if (rows <= 0 || D <= 0) return hipSuccess;
-    if (D % 4 == 0 && D <= 2 * 4 * kBlock)
+    // Short rows leave most threads without a quad and its predicated loads cost
+    // more than the loop's (us, loop and registers: 65536 rows of 4 25.5 and 37.2, of
+    // 64 27.6 and 39.4, of 128 39.2 and 41.5, of 192 47.4 and 42.5, of 512 71.6 and
+    // 47.7; 8000 of 128 6.7 and 7.5, of 192 7.6 and 7.7).
+    constexpr int64_t kRegistersFrom = 192;
+    if (D % 4 == 0 && D >= kRegistersFrom && D <= 2 * 4 * kBlock)
         k_rms_norm_row<2><<<(unsigned)rows, kBlock, 0, s>>>(x, (int)D, g, eps, out);
-    else if (D % 4 == 0 && D <= 8 * 4 * kBlock)
+    else if (D % 4 == 0 && D >= kRegistersFrom && D <= 8 * 4 * kBlock)
         k_rms_norm_row<8><<<(unsigned)rows, kBlock, 0, s>>>(x, (int)D, g, eps, out);
     else
         k_rms_norm<<<(unsigned)rows, kBlock, 0, s>>>(x, D, g, eps, out);

@@ -1,5 +1,5 @@
-"""rms_norm over row lengths at the edges of its forms (quads kept in registers up
-to 2048 and 8192 floats, the scalar loop for the rest), in place and from an
+"""rms_norm over row lengths at the edges of its forms (quads kept in registers from
+192 up to 2048 and 8192 floats, the scalar loop for the rest), in place and from an
 address that is no multiple of 16, against 64 bits.  The sum of squares is D
 positive terms in any order (relative error at most D * 2^-24, typically far
 less: D / 256 per thread), then a division, a square root and two products."""
@@ -9,7 +9,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("D", [1, 3, 4, 1020, 2044, 2048, 2052, 4099, 8188, 8192, 8196])
+@pytest.mark.parametrize("D", [1, 3, 4, 188, 192, 196, 1020, 2044, 2048, 2052, 4099, 8188, 8192, 8196])
 @pytest.mark.parametrize("rows", [1, 33])
 def test_rows(sgq, dev, rows, D):
     import soverign_grad_amd.decode as decode
