@@ -38,7 +38,8 @@ GROUPED = 2  # QuantizationScheme::GroupedAsymmetric
 LAYOUT_INT4_TILED = 0
 LAYOUT_INT4_FLAT = 1
 
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # a CPU-only torch has none
+# A CPU-only torch has none, and no other need have it: it is not public.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 # Every entry point of include/sgq.h with its ctypes signature.
 _i64, _int, _vp = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p
@@ -128,6 +129,8 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def _stream(device: torch.device) -> int:
     # The raw handle, without building a torch.cuda.Stream around it (1.0 us of an eager call).
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
     return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
 
 
