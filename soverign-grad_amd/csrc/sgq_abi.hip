@@ -86,7 +86,10 @@ int check_linear_ws(const char* fn, int bits, int64_t M, int64_t K, int64_t N, c
 
 // Gated MLP workspace: nothing for the one-launch GEMV; otherwise
 // [up projection: M*N floats, 256-byte aligned][split-K partials of either GEMM].
-// The flat INT4 layout always takes the two-projection form.  Tiled INT4
+// The up projection is written there by the flat INT4 layout, an INT8 GEMM without
+// a K split and K == 0; where it multiplies in its epilogue the room stays unused,
+// so that the size is the one callers have had.  The flat INT4 layout always takes
+// the two-projection form.  Tiled INT4
 // batches the skinny kernel takes (one launch for both weights) need its
 // split-K partials of both weights; the size covers every device (a device
 // with fewer CUs may run the GEMV or GEMM form instead).
@@ -99,8 +102,7 @@ int64_t swiglu_ws_bytes(int bits, bool flat, int64_t M, int64_t K, int64_t N, in
         }
     int64_t other = 0;
     // The one-launch GEMV form takes the batches the plain forward runs on the
-    // GEMV; INT8 batches of the skinny kernel run it once per weight, up into
-    // the workspace (no split K).
+    // GEMV; INT8 batches of the skinny kernel run it once per weight (no split K).
     const bool skinny8 = bits == 8 && K > 0 && skinny8_plan(M, K, N, kMaxCus).C > 0;
     if (flat || skinny8 || !linear_uses_gemv(M, K, N) || K == 0) {
         const int64_t split =
@@ -156,6 +158,8 @@ SkinnyPlan decode_rows_plan(int64_t B, int64_t K, int64_t N, int nw, int64_t G, 
     const I4Geom g(K, N, G);
     SkinnyPlan p = skinny_plan(B, K, I4Geom(K, nw * N, G), cus);
     if (p.C == 0 || p.form != 1 || p.MB != 2 || g.spc % (2 * p.C) != 0) return SkinnyPlan{};
+    // Weights side by side run over all of K (q, k and v of D <= 8192 never split it).
+    if (nw > 1 && p.S > 1) return SkinnyPlan{};
     return p;
 }
 
@@ -216,7 +220,10 @@ bool forward_fits(int bits, int64_t M, int64_t K, int64_t N, int64_t group_size)
     if (round_up(K, kPadK) > kGemvMaxKpad) return false;
     if (linear_uses_gemv(M, K, N)) return true;
     if (K > kGemmMaxK) return false;
-    if (bits == 4) {  // the fp32-MFMA kernel (groups not a multiple of 128) maps all devscales at once
+    // The fp32-MFMA kernel maps all devscales at once.  (Groups of a multiple of
+    // 32 that divide N run on the wavefront tiles, which do not, but shapes that
+    // were refused stay refused.)
+    if (bits == 4) {
         const I4Geom g(K, N, group_size);
         if (g.tiled && g.spc % 16 != 0 && g.devscale_count() * 4 >= ((int64_t)1 << 32)) return false;
     }

@@ -336,12 +336,11 @@ hipError_t launch_skinny_i8(const float* x, int64_t M, int64_t K, int64_t N, con
 // ng == 2 the gated MLP h = silu(x * Wg + bg) * (x * Wu + bu).  With split K,
 // ws holds skinny_ws_bytes(p, M, N, ng) bytes (16-byte aligned).
 // Both forms can also run nw (1..3, ng == 1) weights of one shape side by
-// side, weight w writing columns w * N .. w * N + N - 1 of rows of ldy floats
-// (ws: nw times the bytes).  The whole-K form (p.form == 0, p.S == 1) folds an
-// RMSNorm of x (gamma, eps) into the projections, as launch_gemv_i4_multi
-// does, and takes several weights only with it; the super-block form
-// (p.form == 1) adds res (same indexing as y) to the output, and takes several
-// weights of 17 or more rows.
+// side, weight w writing columns w * N .. w * N + N - 1 of rows of ldy floats, over
+// all of K (p.S == 1).  The whole-K form (p.form == 0) folds an RMSNorm of x (gamma,
+// eps) into the projections, as launch_gemv_i4_multi does, and takes several
+// weights only with it; the super-block form (p.form == 1) adds res (same indexing
+// as y) to the output, and takes several weights of 17 or more rows.
 struct SkinnyExtra {
     int nw = 1;
     int64_t ldy = 0;  // 0: N

@@ -1198,12 +1198,12 @@ struct SkinnyRegs {
 // second; a row_ror:8 exchange completes each A operand (the same bf16
 // planes).
 //
-// MULTI (NG == 1): a.wgpw column groups per weight over nw weights of one
-// shape side by side, as k_skinny3.
+// MULTI (NG == 1, all of K): a.wgpw column groups per weight over nw weights of
+// one shape side by side, as k_skinny3.
 template <int NW, int C, int NG, int MB, bool SPLIT, bool HALF, bool MULTI>
 __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, const SkinnyArgs a) {
     static_assert(!HALF || MB == 1, "the half-row form has one row block");
-    static_assert(!MULTI || NG == 1, "weights side by side are plain projections");
+    static_assert(!MULTI || (NG == 1 && !SPLIT), "weights side by side are plain projections of all of K");
     constexpr int XT = HALF ? 4 : 8;  // x quads per lane, row block and super-block
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, n = lane & 15;
@@ -1426,7 +1426,7 @@ __global__ __launch_bounds__(NW * 64) void k_skinny_sb(SGQ_SKINNY_HOT_PARAMS, co
                     const int64_t MN = (int64_t)a.M * a.N, at = (int64_t)m * a.N + col;
 #pragma unroll
                     for (int q = 0; q < NG; ++q)
-                        a.part[((int64_t)(NG == 1 ? wt : q) << a.slog | split) * MN + at] = o[q][b][i];
+                        a.part[((int64_t)q << a.slog | split) * MN + at] = o[q][b][i];
                 } else {
                     const int64_t at = (int64_t)m * a.ldy + (int64_t)wt * a.N + col;
                     float r0 = o[0][b][i];
@@ -1642,26 +1642,23 @@ __global__ __launch_bounds__(NW * 64) void k_skinny8(const float* __restrict__ h
 }
 
 // The skinny kernel's K ranges added in range order, plus the bias; NG == 2:
-// h = silu(gate + bias) * (up + bias2).  part is [NG][S][M*N].  NG == 1 sums
-// blockIdx.y of nw weights side by side (rows of ldy floats) and adds res
-// where it is set (same indexing as y, which it may be).
+// h = silu(gate + bias) * (up + bias2).  part is [NG][S][M*N].  res, where it is
+// set, is added (it may be y).
 // The leading scalar arguments are preloaded into SGPRs.
 struct SkinnyReduceArgs {
-    const float* bias[3];
+    const float* bias[2];
     const float* res;
-    int ldy;
 };
 template <int NG>
 __global__ __launch_bounds__(kThreads) void k_skinny_reduce(const float* __restrict__ part, float* y, int MN, int S, int N,
                                                             const SkinnyReduceArgs a) {
-    const int wt = NG == 1 ? (int)blockIdx.y : 0;
     const int o = blockIdx.x * kThreads + threadIdx.x;  // M <= 32 rows: 32-bit indices
     if (o >= MN) return;
     float r[NG];
-    int m = 0, n = o;
+    int n = 0;
 #pragma unroll
     for (int q = 0; q < NG; ++q) {
-        const float* pq = part + (int64_t)(NG == 1 ? wt : q) * S * MN + o;
+        const float* pq = part + (int64_t)q * S * MN + o;
         float t[kSkinnyMaxSplits];
 #pragma unroll
         for (int sp = 0; sp < kSkinnyMaxSplits; ++sp)  // all loads first
@@ -1670,16 +1667,14 @@ __global__ __launch_bounds__(kThreads) void k_skinny_reduce(const float* __restr
 #pragma unroll
         for (int sp = 0; sp < kSkinnyMaxSplits; ++sp)
             if (sp < S) v += t[sp];
-        const float* bq = a.bias[NG == 1 ? wt : q];
-        if (q == 0 && (bq || a.bias[1] || a.ldy != N)) m = (unsigned)o / (unsigned)N, n = o - m * N;
-        if (bq) v = v + bq[n];
+        if (q == 0 && (a.bias[0] || a.bias[1])) n = (unsigned)o % (unsigned)N;
+        if (a.bias[q]) v = v + a.bias[q][n];
         r[q] = v;
     }
-    const int64_t at = (int64_t)m * a.ldy + (int64_t)wt * N + n;
     float v = r[0];
     if constexpr (NG == 2) v = silu_f32(r[0]) * r[1];
-    if (a.res) v = v + a.res[at];
-    y[at] = v;
+    if (a.res) v = v + a.res[o];
+    y[o] = v;
 }
 
 // h[i] = silu(h[i]) * u[i]: the gated MLP's elementwise tail after two
@@ -1876,6 +1871,7 @@ hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const 
                          const float* const* devscales, const float* const* bias, const I4Geom& g, int form, int S,
                          float* y, float* part, const SkinnyExtra& ex, hipStream_t s) {
     if (form == 0 && (S != 1 || ex.res)) return hipErrorInvalidValue;
+    if (S > 1 && ex.ldy != N) return hipErrorInvalidValue;  // k_skinny_reduce writes whole rows
     // The folded RMSNorm: whole-K form only, where side-by-side weights come
     // with it (the plain kernels take their one weight from the preloaded
     // arguments); the super-block form runs them side by side without it.
@@ -1947,10 +1943,8 @@ hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const 
     if (ex.nw > 1) {
         // Several weights: the LLaMA block's q, k and v of 17..32 sequences.
         if constexpr (NG == 1 && MB == 2) {
-            if (S > 1)
-                SGQ_SKINNY_SB(true, false, true);
-            else
-                SGQ_SKINNY_SB(false, false, true);
+            if (S > 1) return hipErrorInvalidValue;
+            SGQ_SKINNY_SB(false, false, true);
         } else {
             return hipErrorInvalidValue;
         }
@@ -1969,11 +1963,9 @@ hipError_t skinny_launch(const float* x, int64_t M, int64_t K, int64_t N, const 
         if (e != hipSuccess) return e;
         if (M * N >= (int64_t)1 << 31) return hipErrorInvalidValue;
         SkinnyReduceArgs ra{};
-        for (int q = 0; q < nq; ++q) ra.bias[q] = bias[q];
+        for (int q = 0; q < NG; ++q) ra.bias[q] = bias[q];
         ra.res = ex.res;
-        ra.ldy = (int)ex.ldy;
-        k_skinny_reduce<NG><<<dim3((unsigned)ceil_div(M * N, kThreads), (unsigned)ex.nw), kThreads, 0, s>>>(
-            part, y, (int)(M * N), S, (int)N, ra);
+        k_skinny_reduce<NG><<<(unsigned)ceil_div(M * N, kThreads), kThreads, 0, s>>>(part, y, (int)(M * N), S, (int)N, ra);
     }
     return hipGetLastError();
 }
