@@ -728,7 +728,7 @@ def other_config(pkg, key, dev, oracle, steps):
 
 XOVER_M = (4, 5, 8, 16, 17, 24, 32, 48, 64, 128)
 # sgq_linear_plan's path codes (include/sgq.h)
-PATH_NAMES = ("gemv", "gemm_bf16x3", "gemm_fp32", "flat", "skinny_bf16x3")
+PATH_NAMES = ("gemv", "gemm_bf16x3", "gemm_small_groups", "flat", "skinny_bf16x3")
 
 
 def c3_crossover(pkg, dev, oracle, steps):

@@ -114,8 +114,9 @@ int64_t sgq_linear_workspace_bytes(int bits, int64_t M, int64_t K, int64_t N);
  * MI355X has 256, a partition fewer).  *path: 0 the GEMV, 1 the three-term
  * bf16 MFMA GEMM, 2 the GEMM of INT4 groups that are not a multiple of 128
  * (three-term bf16 where a scale column spans a multiple of four strips, as
- * for groups of 32, 64 and 96 that divide N; else fp32 MFMA), 3 the generic kernel of the flat INT4 layout, 4 the skinny bf16
- * MFMA kernels (INT4: 5..32 rows over a weight wide enough to fill the
+ * for groups of 32, 64 and 96 that divide N; else fp32 MFMA), 3 the kernels of
+ * the flat INT4 layout (a row form, tiles on the fp32 MFMA or a thread per
+ * output, by shape), 4 the skinny bf16 MFMA kernels (INT4: 5..32 rows over a weight wide enough to fill the
  * device with workgroups of 32 or 64 columns, and 5..32 rows over narrower
  * weights with (M rounded up to 8) * K * N >= 2^28, K split; INT8: 5..128
  * rows with (M rounded up to 8) * K * N >= 2^26, above 16 rows only while

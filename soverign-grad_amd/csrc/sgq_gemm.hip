@@ -33,12 +33,12 @@
 // clock at 1.9 GHz; a large bf16 library product on the same card runs at
 // 1.2 PFLOP/s with the clock at 1.5-1.8 GHz.  Smaller groups are VALU-bound:
 // the split costs 208 VALU instructions per group, row block set and stage.
-// Measured on MI355X, previous kernels -> this (us): g128 2048 x 4096 -> 11008
-// 575 -> 457, 2048 x 11008 -> 4096 535 -> 431, 512 x 2048 -> 5632 71.5 -> 58.7;
-// g64 512 x 2048 -> 5632 158.7 -> 65.8; g32 512 x 2048 -> 5632 158.3 -> 80.2,
-// 2048 x 4096 -> 11008 1691 -> 752, 40 x 11008 -> 4096 108.6 -> 39.7.  The
-// error against 64 bits is no larger (g128 2048 x 4096 -> 11008 5.9e-7 ->
-// 3.0e-7 with four K ranges, g32 512 x 2048 -> 5632 5.4e-7 -> 2.2e-7).
+// Measured on MI355X, both builds in turn, the kernels before this one -> this (us,
+// with bias): g128 2048 x 4096 -> 11008 607 -> 473, 2048 x 11008 -> 4096 578 -> 439,
+// 512 x 2048 -> 5632 74.9 -> 51.5; g64 512 x 2048 -> 5632 162 -> 58.1 to 60.5; g32 512
+// x 2048 -> 5632 162 -> 72.1 to 74.8, 2048 x 4096 -> 11008 1684 -> 812, 40 x 11008 ->
+// 4096 109 -> 37.5.  The error against 64 bits is no larger (g128 2048 x 4096 ->
+// 11008 5.9e-7 -> 3.0e-7 with four K ranges, g32 512 x 2048 -> 5632 5.4e-7 -> 2.2e-7).
 #include "sgq_device.h"
 #include "sgq_internal.h"
 

@@ -106,16 +106,17 @@ struct I4Geom {
     int64_t devscale_count() const { return tiled ? nsc * Kpad : 0; }
 };
 
-constexpr int kGemvMaxM = 16;  // M <= this runs the GEMV, larger M the MFMA GEMM (but see below)
+constexpr int kGemvMaxM = 16;  // up to this many rows never run the MFMA GEMM (but see below)
 // The plain forward also runs the GEMV for batches of up to this many rows
 // (row groups of 8, one workgroup each) when the work is small: the GEMV's
 // time grows with M * K * N at the VALU rate from a fixed ~3 us, the GEMM's
 // from ~10-15 us of pipeline fill, split-K partials and reduce.  Measured on
-// MI355X with each path forced (INT4 g128): at 16 rows the GEMV wins on every
-// shape tried (4096->11008 31 vs 35 us, 2048->2048 5.6 vs 11.8 us); from 17
-// rows the GEMM's 32- and 64-row tiles win once M * K * N passes about 2^28
-// (4096x4096 at 17..32 rows 19-23 vs 23 us, 4096->11008 at 17 rows 35 vs
-// 54 us) and lose below it (2048x2048 at 64 rows 17 vs 14 us).
+// MI355X with each path forced (INT4 g128, GEMV vs GEMM, us): at 16 rows the GEMV
+// wins where the work is small (2048->2048 5.9 vs 12.0, 5632->2048 11.1 vs 15.0,
+// 4096x4096 14.1 vs 15.0; 4096->11008, 29.0 vs 20.1, is the skinny kernel's, 15.0);
+// from 17 rows the GEMM wins once M * K * N passes about 2^28 (4096x4096 at 17..32
+// rows 23.5-24.0 vs 15.4-17.4, 4096->11008 at 17 rows 50.2 vs 20.8) and loses below
+// it (2048x2048 at 64 rows 14.1 vs 15.4).
 constexpr int64_t kGemvRowsMax = 128;
 constexpr int64_t kGemvSmallWork = (int64_t)1 << 28;  // M * K * N
 inline bool linear_uses_gemv(int64_t M, int64_t K, int64_t N) {
@@ -161,9 +162,11 @@ struct SkinnyPlan {
 };
 // Narrow weights split K only from this much work, M rounded up to the
 // GEMV's row group of 8 (its time steps up with each group).  Measured (us,
-// GEMV or GEMM -> split): 11008 -> 4096 at 8 / 10 / 16 rows 19.6 / 31.7 /
-// 32.0 -> 18.3 / 18.5 / 20.2; 4096 -> 4096 at 12 / 16 / 24 rows 14.0 / 14.6 /
-// 21.8 -> 10.4 / 10.9 / 14.1; 5632 -> 2048 at 24 rows 20.3 -> 15.6.  Kept:
+// GEMV -> split): 11008 -> 4096 at 8 / 10 / 16 rows 19.6 / 31.7 / 32.0 -> 18.3 /
+// 18.5 / 20.2; 4096 -> 4096 at 12 / 16 rows 14.0 / 14.6 -> 10.4 / 10.9; against the
+// GEMM (of wavefront tiles) 4096 -> 4096 at 24 rows 16.3 -> 13.2, 5632 -> 2048 15.5
+// -> 15.2; at 17..32 rows of 4096 -> 11008 and 11008 -> 4096 that GEMM is the faster
+// one, 20.8-22.7 and 20.5-21.9 against 24.2-27.0 and 22.0-24.5.  Kept:
 // 4096 -> 4096 at 8 rows (9.2 vs 10.3), 5632 -> 2048 at 16 (11.7 vs 12.4),
 // 2048 -> 2048 (5.8 vs 9.0 at 16 rows), four rows (11008 -> 4096 13.7 vs
 // 17.7).
@@ -355,11 +358,11 @@ hipError_t launch_skinny_i4(const float* x, int64_t M, int64_t K, int64_t N, int
 // nw (1..3) tiled INT4 weights of one shape [K, N] side by side on one input:
 // weight w writes y[m * ldy + w * N + n] (+ res at the same index when res is
 // set).  gamma (optional): the input is rms_norm(x, gamma, eps), applied
-// inside the kernel.  Strip layout only; M <= kGemvMaxM.
+// inside the kernel.  Strip layout only; batches that linear_uses_gemv takes.
 hipError_t launch_gemv_i4_multi(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
                                 const float* const* devscales, const float* const* bias, const I4Geom& g, float* y,
                                 int64_t ldy, const float* res, const float* gamma, float eps, hipStream_t s);
-// MFMA GEMM (M > kGemvMaxM).  Grids with fewer 128x128 tiles than CUs split K
+// MFMA GEMM (batches past linear_uses_gemv).  Grids with fewer 128x128 tiles than CUs split K
 // over workgroups; their partial tiles go to ws (gemm_workspace_bytes(M, K, N)
 // bytes, 0 when K is not split) and a second kernel adds them in fixed order.
 struct GemmPlan {
@@ -399,8 +402,9 @@ int64_t gemm_workspace_bytes(int64_t M, int64_t K, int64_t N);
 // unused) takes on `cus` compute units: what launch_gemm_i8/i4 writes.
 int64_t gemm_launch_ws_bytes(int bits, int64_t M, int64_t K, int64_t N, int mode, int64_t cus);
 // The plan a forward of this shape runs on `cus` compute units: path 0 the
-// GEMV, 1 the three-term bf16 GEMM, 2 the fp32 GEMM, 3 the flat INT4 kernel,
-// 4 the skinny MFMA kernel; ks the K splits (1: none).
+// GEMV, 1 the three-term bf16 GEMM, 2 the GEMM of INT4 groups that are not a
+// multiple of 128 (wavefront tiles or the fp32 MFMA), 3 the flat INT4 kernels, 4 the
+// skinny MFMA kernels; ks the K splits over workgroups (1: none).
 void linear_plan(int bits, int64_t M, int64_t K, int64_t N, int64_t group_size, int64_t cus, int* path, int* ks);
 int xcd_rect_rows(int64_t tm, int64_t tn, int64_t xb, int64_t wb, int64_t xcds);
 // gemm_i8_epilogue: whether the launch of this shape takes gate and res (k_gemm3
@@ -439,7 +443,7 @@ hipError_t launch_splitk_reduce(const float* part, int KS, int64_t M, int64_t N,
 hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N, const void* packed,
                                  const float* scales, int64_t G, const float* bias, float* y, hipStream_t s);
 
-// Gated MLP: h = silu(x*Wg + bg) * (x*Wu + bu).  The GEMV form (M <= kGemvMaxM)
+// Gated MLP: h = silu(x*Wg + bg) * (x*Wu + bu).  The GEMV form (linear_uses_gemv)
 // runs both weights in one launch (as does the skinny kernel, launch_skinny_i4
 // with ng == 2); GEMM batches run two projections, the second with the first
 // as its epilogue's gate (as does the INT8 skinny kernel); an INT8 GEMM without

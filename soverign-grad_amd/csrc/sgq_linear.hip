@@ -2193,9 +2193,9 @@ GemmPlan gemm_plan(int64_t M, int64_t K, int64_t N, const GemmTile& t, int64_t c
     if (cus < 1) cus = 1;
     if (cus > kMaxCus) cus = kMaxCus;
     // Splits fill the resident slots, rounded down: a grid just past them
-    // runs its last few workgroups as a second pass (4096->11008 at 128 rows,
-    // 86 tiles of 128 x 128: 6 splits, 516 workgroups on 512 slots, 94 us; 5
-    // splits 61 us).
+    // runs its last few workgroups as a second pass (4096->11008 at 128 rows on
+    // the LDS-staged 128 x 128 tiles INT4 used to have, 86 of them: 6 splits, 516
+    // workgroups on 512 slots, 94 us; 5 splits 61 us).
     const int64_t slots = t.per_cu * cus;
     if (tiles < slots && KT >= 4) {
         int64_t ks = slots / tiles;
@@ -2211,12 +2211,19 @@ GemmPlan gemm_plan(int64_t M, int64_t K, int64_t N, const GemmTile& t, int64_t c
 
 // Tile of the three-term GEMM for a code width and batch (the fp32 kernel
 // uses the 128 x 128 tile), with the workgroups a split-K grid gives each CU:
-// two of the 128 x 128 tiles, one of the 128 x 256 (its LDS and registers fill
-// the CU), four of the 32-row tile (28 KB of LDS) and two of the 64-row tile.
-// Three of the latter fit (40 KB of LDS) but cost more in partial tiles
-// (KS * M * N * 4 bytes, written and read back) than they gain: 2048->6144 at
-// 64 rows 16 splits 31.6 us, 10 splits 24.3 us; 4096->11008 at 48 rows 9
-// splits 50.4 us, 5 splits 42.1 us.
+// one of INT8's 128 x 256 tile (its LDS and registers fill the CU), four of the
+// 32-row tile (28 KB of LDS) and two of the 64-row tile.  Three of the latter
+// fit (40 KB of LDS) but cost more in partial tiles (KS * M * N * 4 bytes,
+// written and read back) than they gain: 2048->6144 at 64 rows 16 splits 31.6
+// us, 10 splits 24.3 us; 4096->11008 at 48 rows 9 splits 50.4 us, 5 splits 42.1
+// us.
+//
+// INT4's wavefront tiles (gemm_wave_shape) have their splits over workgroups
+// planned by these tiles and the 128 x 128 one, those of the LDS-staged kernel
+// they replaced, not by their own.  Where the ranges within a workgroup alone
+// would give as many wavefronts the split costs its partial tiles and the
+// reduce launch: 512 x 2048 -> 5632 g32 runs 704 workgroups either way, two
+// splits of two ranges or one of four.
 GemmTile gemm_tile(int bits, int64_t M) {
     if (M <= 32) return GemmTile{32, kBN, 4};
     if (M <= 64) return GemmTile{64, kBN, 2};
@@ -2234,8 +2241,8 @@ int64_t gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     return ks > 1 ? ks * M * N * 4 : 0;
 }
 
-// The tile an INT4 GEMM plans its K splits by: 128 x 128 for groups that are
-// not a multiple of 128, whatever the batch.
+// The tile an INT4 GEMM plans its K splits over workgroups by: 128 x 128 for
+// groups that are not a multiple of 128, whatever the batch.
 static GemmTile gemm_i4_tile(int64_t M, int mode) { return mode % 16 == 0 ? gemm_tile(4, M) : GemmTile{kBM, kBN, 2}; }
 
 int64_t gemm_launch_ws_bytes(int bits, int64_t M, int64_t K, int64_t N, int mode, int64_t cus) {

@@ -110,10 +110,11 @@ enum PackFrom { kFromX, kFromXInv, kFromCodes };
 // the fp32 codes move in rows (512 contiguous bytes), the packed codes go
 // through LDS so that a strip's rows leave as one 128-byte run (a thread per
 // 16-byte chunk wrote chunks RQ * 16 bytes apart).  HBM bounds them.  Measured
-// on MI355X, a quantize with fp32 codes, before -> now (us): INT4 4096 x 11008
-// g128 373 -> 83 (385 MB, 4.6 TB/s, what a large copy reaches), 4096 x 4096
-// g32 186 -> 32, g24 (scales found first) 208 -> 137; INT8 4096 x 4096 per
-// tensor 141 -> 67, 4096 x 4097 per channel 141 -> 66.
+// on MI355X in graphs, a quantize with fp32 codes, a thread per chunk and its
+// passes -> this (us): INT4 4096 x 11008 g128 368 -> 82.5 (385 MB, 4.7 TB/s, what a
+// large copy reaches), 4096 x 4096 g32 164 -> 28.1, g24 (scales found first) 184 ->
+// 61, flat 4096 x 4100 g64 73.8 -> 43.8 (its scales by eight lanes a group); INT8
+// 4096 x 4096 per tensor 125 -> 47.4, 4096 x 4097 per channel 124 -> 38.9.
 constexpr int kPackRows = 32, kPackCols = 128;
 // Tiles of one launch: a launch holds fewer than 2^32 threads, which the tiles
 // of a very long, narrow weight exceed (K > 2^29 at up to 128 columns).

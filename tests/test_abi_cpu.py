@@ -352,7 +352,7 @@ def test_plan_examples(lib):
     assert _plan(lib, 8, 2048, 4096, 4096, 0, 256) == (1, 1)
     assert _plan(lib, 8, 256, 4096, 1024, 0, 256)[1] > _plan(lib, 8, 256, 4096, 1024, 0, 32)[1]
     assert _plan(lib, 4, 1, 4096, 4096, 128, 256) == (0, 1)  # decode: the GEMV
-    assert _plan(lib, 4, 300, 2048, 640, 32, 256)[0] == 2  # group 32: the fp32 MFMA kernel
+    assert _plan(lib, 4, 300, 2048, 640, 32, 256)[0] == 2  # group 32: the GEMM of groups that are not a multiple of 128
     assert _plan(lib, 4, 300, 2048, 644, 32, 256)[0] == 3  # N % 8 != 0: flat layout
     # A CU count above the full chip is planned as the full chip.
     assert _plan(lib, 8, 256, 4096, 1024, 0, 1024) == _plan(lib, 8, 256, 4096, 1024, 0, 256)

@@ -17,7 +17,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import rel_err
+from helpers import i4_geom, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -62,7 +62,12 @@ def _path(sgq, bits, M, K, N, g):
 def test_draws_cross_the_dispatch(sgq):
     paths = {_path(sgq, b, M, K, N, g) for b, M, K, N, g, _, _ in CASES}
     kinds = {p for p, _ in paths}
-    assert {0, 1, 2, 3, 4} <= kinds, paths  # GEMV, three-term GEMM, fp32-MFMA GEMM, flat INT4, skinny MFMA
+    assert {0, 1, 2, 3, 4} <= kinds, paths  # GEMV, GEMM (INT8 or groups of 128 n), GEMM of other groups, flat INT4, skinny MFMA
+    # Paths 1 and 2 by the kernel that runs: INT8's staged tiles, INT4's wavefront
+    # tiles (scale columns of a multiple of four strips) and the fp32 MFMA kernel.
+    gemms = {"int8" if b == 8 else ("wave" if i4_geom(K, N, g)["spc"] % 4 == 0 else "fp32")
+             for b, M, K, N, g, _, _ in CASES if _path(sgq, b, M, K, N, g)[0] in (1, 2)}
+    assert gemms == {"int8", "wave", "fp32"}, gemms
 
 
 @pytest.mark.parametrize("bits,M,K,N,g,bias,i", CASES, ids=[f"d{c[6]}_{c[0]}b_{c[1]}x{c[2]}x{c[3]}" for c in CASES])
