@@ -332,6 +332,14 @@ def dequantize_codes(qx: QuantizedTensor) -> torch.Tensor:
     return out
 
 
+def _new_output(x: torch.Tensor, M: int, N: int) -> torch.Tensor:
+    # new_empty costs less than torch.empty with its keywords, but a subclass of
+    # Tensor makes one of its own kind; results are plain tensors.
+    if type(x) is torch.Tensor:
+        return x.new_empty((M, N))
+    return torch.empty((M, N), dtype=torch.float32, device=x.device)
+
+
 def _linear_args(x: torch.Tensor, qw: QuantizedTensor, bias: Optional[torch.Tensor]):
     if x.dim() != 2:
         raise ValueError("matmul currently requires 2D tensors!")  # src/ops.cpp:380-382
@@ -353,7 +361,7 @@ def quantized_matmul_int8(x: torch.Tensor, qw: QuantizedTensor, bias: Optional[t
     x, K, N, b = _linear_args(x, qw, bias)
     M = x.shape[0]
     dev = x.device
-    y = out if out is not None else x.new_empty((M, N))
+    y = out if out is not None else _new_output(x, M, N)
     ws, nws = _linear_ws.get(lib.sgq_linear_workspace_bytes(8, M, K, N), dev)
     _check(lib.sgq_linear_int8(_ptr(x), M, K, N, _ptr(qw.packed), _ptr(qw.scales), _int8_branch(qw), _ptr(b),
                                _ptr(y), ws, nws, _stream(dev)))
@@ -366,7 +374,7 @@ def quantized_matmul_int4(x: torch.Tensor, qw: QuantizedTensor, bias: Optional[t
     x, K, N, b = _linear_args(x, qw, bias)
     M = x.shape[0]
     dev = x.device
-    y = out if out is not None else x.new_empty((M, N))
+    y = out if out is not None else _new_output(x, M, N)
     ws, nws = _linear_ws.get(lib.sgq_linear_workspace_bytes(4, M, K, N), dev)
     _check(lib.sgq_linear_int4(_ptr(x), M, K, N, _ptr(qw.packed), _ptr(qw.scales), _ptr(qw.devscales),
                                qw.group_size, _ptr(b), _ptr(y), ws, nws, _stream(dev)))
