@@ -251,11 +251,13 @@ inline Skinny8Plan skinny8_plan(int64_t M, int64_t K, int64_t N, int64_t cus) {
     // / 19.1, at 17 rows over K = 2048 23.4 / 18.4 / 11.9; 2048 -> 5632 at 16 rows
     // 13.5 / 8.8 / 10.7; 8192 -> 28672 at 8 rows per tensor 88.9 / 73.2 / 58.2;
     // 4096^2 at 16 rows 12.9 / 14.9 / 18.9; 1024 -> 4096 at 100 rows per tensor
-    // 18.2 / 13.1 / 11.5.
+    // 18.2 / 13.1 / 11.5.  Each column block also has its sum over the wavefronts and
+    // its epilogue, as long as some 800 rows of K: per tensor 324 -> 5632 at 128 rows
+    // 12.0 / 11.6 / 14.1, 512 -> 5632 19.6 / 16.2 / 18.9.
     int64_t best = 0;
     for (int c : {1, 2, 4}) {
         const int64_t wgs = ceil_div(M, 16 * p.MB) * ceil_div(N, 16 * c);
-        const int64_t cost = ceil_div(wgs, cus < 1 ? 1 : cus) * (52 + 15 * c);
+        const int64_t cost = ceil_div(wgs, cus < 1 ? 1 : cus) * ((52 + 15 * c) * K + 15 * 800 * c);
         if (best == 0 || cost < best) best = cost, p.C = c;
     }
     return p;
