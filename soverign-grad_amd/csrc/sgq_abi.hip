@@ -86,8 +86,8 @@ int check_linear_ws(const char* fn, int bits, int64_t M, int64_t K, int64_t N, c
 
 // Gated MLP workspace: nothing for the one-launch GEMV; otherwise
 // [up projection: M*N floats, 256-byte aligned][split-K partials of either GEMM].
-// The up projection is written there by the flat INT4 layout, an INT8 GEMM without
-// a K split and K == 0; where it multiplies in its epilogue the room stays unused,
+// The up projection is written there by the flat INT4 layout, an INT8 or fp32 MFMA
+// GEMM without a K split and K == 0; where it multiplies in its epilogue the room stays unused,
 // so that the size is the one callers have had.  The flat INT4 layout always takes
 // the two-projection form.  Tiled INT4
 // batches the skinny kernel takes (one launch for both weights) need its
@@ -767,7 +767,12 @@ int sgq_swiglu_int4(const float* x, int64_t M, int64_t K, int64_t N, const void*
     if (lw != SGQ_OK) return lw;
     void* split = (char*)workspace + align_up(M * N * 4);
     SGQ_HIP(launch_gemm_i4(x, M, K, N, 1, &packed_gate, &devscales_gate, &bias_gate, g, {}, h, split, s), "gemm_i4");
-    SGQ_HIP(launch_gemm_i4(x, M, K, N, 1, &packed_up, &devscales_up, &bias_up, g, {h}, h, split, s), "gemm_i4");
+    if (gemm_i4_epilogue(M, K, N, g, cus)) {
+        SGQ_HIP(launch_gemm_i4(x, M, K, N, 1, &packed_up, &devscales_up, &bias_up, g, {h}, h, split, s), "gemm_i4");
+    } else {
+        SGQ_HIP(launch_gemm_i4(x, M, K, N, 1, &packed_up, &devscales_up, &bias_up, g, {}, u, split, s), "gemm_i4");
+        SGQ_HIP(launch_silu_mul(h, u, M * N, s), "silu_mul");
+    }
     return ok();
 }
 

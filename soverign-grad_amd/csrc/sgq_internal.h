@@ -412,6 +412,13 @@ int xcd_rect_rows(int64_t tm, int64_t tn, int64_t xb, int64_t wb, int64_t xcds);
 // gemm_i8_epilogue: whether the launch of this shape takes gate and res (k_gemm3
 // without a K split does not: the branches cost it 1%).
 bool gemm_i8_epilogue(const float* x, int64_t M, int64_t K, int64_t N, int64_t cus);
+// Whether the gate belongs in the epilogue of an INT4 launch of this shape: not in
+// the fp32 kernel's without a K split, where a thread takes 64 divisions and
+// exponentials one after another while most of the device is done (gated MLP of
+// 182 x 20 -> 1080 g24 37.9 us, 28.6 with a launch of its own; 2000 x 64 -> 4800
+// 98, 90).  It does take gate and res, for the block's step, which has no room for
+// a second product.
+bool gemm_i4_epilogue(int64_t M, int64_t K, int64_t N, const I4Geom& g, int64_t cus);
 hipError_t launch_gemm_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed, const float* scales,
                           bool per_tensor, const float* bias, const GemmEpilogue& ep, float* y, void* ws,
                           hipStream_t s);
@@ -448,8 +455,8 @@ hipError_t launch_linear_i4_flat(const float* x, int64_t M, int64_t K, int64_t N
 // Gated MLP: h = silu(x*Wg + bg) * (x*Wu + bu).  The GEMV form (linear_uses_gemv)
 // runs both weights in one launch (as does the skinny kernel, launch_skinny_i4
 // with ng == 2); GEMM batches run two projections, the second with the first
-// as its epilogue's gate (as does the INT8 skinny kernel); an INT8 GEMM without
-// a K split and the flat INT4 layout two projections and launch_silu_mul
+// as its epilogue's gate (as does the INT8 skinny kernel); an INT8 or fp32 MFMA
+// GEMM without a K split and the flat INT4 layout two projections and launch_silu_mul
 // (h = silu(h) * u, elementwise over n floats).
 hipError_t launch_swiglu_gemv_i8(const float* x, int64_t M, int64_t K, int64_t N, const void* packed_g,
                                  const float* scales_g, const float* bias_g, const void* packed_u,

@@ -2369,6 +2369,10 @@ hipError_t launch_gemm_i8(const float* x, int64_t M, int64_t K, int64_t N, const
     return e != hipSuccess || p.KS == 1 ? e : launch_splitk_reduce(a.part, p.KS, M, N, 1, &bias, ep, y, s);
 }
 
+bool gemm_i4_epilogue(int64_t M, int64_t K, int64_t N, const I4Geom& g, int64_t cus) {
+    return gemm_wave_takes(4, (int)g.spc) || gemm_plan(M, K, N, gemm_i4_tile(M, (int)g.spc), cus).KS > 1;
+}
+
 hipError_t launch_gemm_i4(const float* x, int64_t M, int64_t K, int64_t N, int nw, const void* const* packed,
                           const float* const* devscales, const float* const* bias, const I4Geom& g,
                           const GemmEpilogue& ep, float* y, void* ws, hipStream_t s) {

@@ -147,7 +147,7 @@ def test_small_products(sgq, dev, M, K, N, G):
 
 
 @pytest.mark.parametrize("bits,G", [(4, 128), (4, 32), (4, 24), (8, 0), (8, 1)])
-@pytest.mark.parametrize("M,K,N", [(130, 256, 384), (300, 2048, 768), (1100, 96, 4224), (2051, 35, 4224)])
+@pytest.mark.parametrize("M,K,N", [(130, 256, 384), (300, 2048, 768), (1100, 96, 4224), (2051, 35, 4224), (182, 20, 1080)])
 def test_gated_epilogue(sgq, dev, M, K, N, bits, G):
     """The gated MLP of GEMM batches: the up projection's epilogue multiplies
     by silu of the gate projection, the same values as the two forwards and an
