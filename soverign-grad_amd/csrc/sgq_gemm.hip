@@ -416,20 +416,28 @@ __global__ __launch_bounds__(kWG) void k_splitk_reduce(const float* __restrict__
 // 2048 x 4096 -> 11008 457 against 477; with one 40 x 4096 -> 4096 26.4
 // against 23.5, 96 x 11008 -> 4096 45 against 43.
 //
-// A short K has too few stages for four ranges: with many tiles each wavefront
-// takes one of its own (half with two ranges in between), and two row blocks,
-// whose epilogue is shorter.  Measured at K = 64 (us, four ranges / two / one, the
-// kernels before this one): g32 2048 rows -> 2048 (1024 tiles) 19.9 / 14.4 / 16.3,
-// 18.5; -> 4096 (2048 tiles) 33.8 / 24.6 / 20.3, 24.2; -> 11008 81.7 / 57.2 / 48.2,
-// 61.8; at K = 512 g128 4096 -> 16384 272 / 231 / 217, 271; 512 tiles at K = 96
-// 11.1 / 13.2 / 17.0, 19.2.
+// A short K has too few stages for four ranges: a grid runs in rounds of two
+// workgroups per CU, each costing its tiles' pass through LDS and its stages, and
+// the arrangement with the least is taken, with two row blocks (their epilogue is
+// shorter).  Fitted (us a round, four ranges / two / one): 6.2 / 8.5 / 12.6 and .44 /
+// .97 / 1.98 a stage of 32 k.  Measured at K = 64 (us, the same, then the kernels
+// before this one): g32 2048 rows -> 2048 19.9 / 14.4 / 16.3, 18.5; -> 4096 33.8 /
+// 24.6 / 20.3, 24.2; -> 11008 81.7 / 57.2 / 48.2, 61.8; at K = 512 g128 4096 -> 16384
+// 272 / 231 / 217, 271; at K = 96 512 rows -> 4096 11.1 / 13.2 / 17.0, 19.2.
 GemmWaveShape gemm_wave_shape(int64_t M, int64_t K, int64_t N, bool one_scale, int KS, int64_t cus) {
     constexpr int64_t kShortK = 512;
     GemmWaveShape w;
     if (KS == 1 && K <= kShortK) {
-        const int64_t tiles = ceil_div(M, 32) * ceil_div(N, kWaveCols);
-        w.rb = 2;
-        w.sk = tiles >= 8 * cus ? 1 : (tiles >= 4 * cus ? 2 : 4);
+        static const struct {
+            int sk, round, stage;
+        } forms[3] = {{4, 620, 44}, {2, 850, 97}, {1, 1260, 198}};
+        int64_t best = 0;
+        for (const auto& f : forms) {
+            const GemmWaveShape t{2, f.sk};
+            const int64_t rounds = ceil_div(ceil_div(M, t.rows()) * ceil_div(N, t.cols()), 2 * (cus < 1 ? 1 : cus));
+            const int64_t cost = rounds * (f.round + f.stage * ceil_div(K, kStageK));
+            if (best == 0 || cost < best) best = cost, w = t;
+        }
         return w;
     }
     w.rb = one_scale && ceil_div(M, 64) * ceil_div(N, kWaveCols) * KS >= 4 * cus ? 4 : 2;

@@ -46,7 +46,7 @@ def test_tile_edges(sgq, dev, M, K, G, N):
 @pytest.mark.parametrize("M,K,N,G", [(2048, 160, 4096, 128), (2049, 97, 4224, 128), (40, 4096, 4096, 32),
                                      (1025, 512, 5632, 64), (33, 8200, 1152, 128),
                                      (1100, 97, 4224, 32), (1100, 512, 4096, 128), (1100, 513, 4096, 128),
-                                     (2049, 33, 4160, 64), (2081, 512, 4128, 96)])
+                                     (2049, 33, 4160, 64), (2081, 512, 4128, 96), (1020, 64, 4096, 32), (1020, 70, 4096, 128)])
 def test_large_grids(sgq, dev, M, K, N, G):
     """Four row blocks per wavefront, grids without a K split, small batches over
     long K, a short K in one and two ranges per workgroup."""
